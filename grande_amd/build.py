@@ -29,7 +29,7 @@ SOURCES = ["gemm.hip", "attention.hip", "norm.hip", "laya.hip", "model.cpp", "gg
 # Per-file device flags.  The GEMM and attention kernels keep their MFMA
 # accumulators in ordinary VGPRs: with the AGPR form the register allocator
 # shuffles them between loop iterations (v_accvgpr moves in the main loop).
-EXTRA = {name: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for name in ("gemm.hip", "attention.hip", "laya.hip")}
+EXTRA = {name: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for name in ("gemm.hip", "attention.hip", "norm.hip", "laya.hip")}
 HEADERS = sorted(CSRC.glob("*.h")) + [INCLUDE / "omg_hip.h"]
 
 

@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <memory>
 #include <string>
 #include <vector>
@@ -19,8 +20,62 @@ struct omg_builder {
 struct omg_engine {
     std::unique_ptr<omg::Engine> e;
 };
+// Scratch of stream-ordered calls on one object, kept from call to call: an
+// allocation and its release cost the host about 14 us a call, more than a
+// small readout's kernels take.  It serves the first stream it is asked for
+// (calls there run in order, so they share it); any other stream, the
+// per-thread stream (one handle, many streams), calls being captured and
+// requests above LIMIT allocate in stream order.
+class StreamScratch {
+   public:
+    ~StreamScratch() {
+        if (p_) (void)hipFree(p_);
+    }
+    // f(scratch) with at least `bytes`; queues its work on s.
+    template <class F>
+    void with(hipStream_t s, size_t bytes, F&& f) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (s != hipStreamPerThread) OMG_HIP(hipStreamIsCapturing(s, &cap));
+        if (s != hipStreamPerThread && cap == hipStreamCaptureStatusNone && bytes <= LIMIT) {
+            int dev = 0;  // the null stream is one per device
+            OMG_HIP(hipGetDevice(&dev));
+            std::lock_guard<std::mutex> lock(mu_);
+            if (!p_ || (s == owner_ && dev == dev_)) {
+                if (bytes > bytes_) {
+                    if (p_) OMG_HIP(hipFreeAsync(p_, s));
+                    p_ = nullptr;
+                    bytes_ = 0;
+                    OMG_HIP(hipMallocAsync(&p_, bytes, s));
+                    bytes_ = bytes;
+                    owner_ = s;
+                    dev_ = dev;
+                }
+                f(p_);
+                return;
+            }
+        }
+        void* p = nullptr;
+        OMG_HIP(hipMallocAsync(&p, bytes, s));
+        try {
+            f(p);
+        } catch (...) {
+            (void)hipFreeAsync(p, s);
+            throw;
+        }
+        OMG_HIP(hipFreeAsync(p, s));
+    }
+
+   private:
+    static constexpr size_t LIMIT = size_t(64) << 20;
+    std::mutex mu_;
+    void* p_ = nullptr;
+    size_t bytes_ = 0;
+    hipStream_t owner_ = nullptr;
+    int dev_ = 0;
+};
 struct omg_weight {
     omg::DevTensor t;
+    mutable StreamScratch scratch;
 };
 struct omg_weights {
     std::map<std::string, omg::QTensor> tensors;
@@ -479,23 +534,10 @@ int omg_dev_label_readout(const omg_weight* embed, const float* rows, int64_t nr
         if (!embed || !rows || !labels || !out) omg::fail(omg::E_INVALID, "null argument");
         if (nrows <= 0 || nlabels <= 0) omg::fail(omg::E_INVALID, "label readout: no rows or no labels");
         const hipStream_t s = static_cast<hipStream_t>(stream);
-        const int64_t vocab = embed->t.w.rows, nb = omg::logits_blocks(vocab);
-        // scratch: the full logits rows, then the per-workgroup partials
-        // (float2, on an 8-byte boundary)
-        const int64_t nlog = (nrows * vocab + 1) / 2 * 2;
-        const size_t bytes = size_t(nlog) * 4 + size_t(nb * nrows) * 8;
-        void* scratch = nullptr;
-        OMG_HIP(hipMallocAsync(&scratch, bytes, s));
-        float* logits = static_cast<float*>(scratch);
-        float2* part = reinterpret_cast<float2*>(logits + nlog);
-        try {
-            omg::launch_logits(s, embed->t.w, rows, nrows, nullptr, vocab, softcap, logits, part);
-            omg::launch_label_lse(s, logits, nrows, vocab, part, nb, labels, nlabels, out);
-        } catch (...) {
-            (void)hipFreeAsync(scratch, s);
-            throw;
-        }
-        OMG_HIP(hipFreeAsync(scratch, s));
+        const omg::DevWeight& E = embed->t.w;
+        embed->scratch.with(s, size_t(omg::label_readout_bytes(nrows, E.rows, nlabels, E.cols)), [&](void* p) {
+            omg::launch_label_readout(s, E, rows, nrows, labels, nlabels, softcap, out, p);
+        });
     });
 }
 

@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstdio>
 #include <fstream>
+#include <type_traits>
 
 // Most split-K partials of one product (a_ holds this many).
 #ifndef OMG_KSPLIT
@@ -75,26 +76,35 @@ DevTensor upload_weight(const QTensor& t, bool tiled) {
     const int64_t rb = (d.w.rows + 31) / 32, st = (d.w.cols + 63) / 64;
     const int PK = tile_packet_bytes(d.w.dtype);
     const int64_t row_bytes = t.dtype == Q4 ? d.w.cols / 2 : (t.dtype == Q8 ? d.w.cols : 2 * d.w.cols);
-    const int CB = PK / 32, piece = CB / 8;  // bytes of one row per stage, per (k-step, half)
+    const int CB = PK / 32;  // bytes of one row per stage: 8 pieces, one per (k-step, half)
     std::vector<uint8_t> tiles(size_t(rb * st * PK), 0);
     std::vector<uint8_t> tsc(t.dtype == F16 ? 0 : size_t(rb * st * TILE_SCALE_BYTES), 0);
-    for (int64_t r = 0; r < d.w.rows; ++r) {
-        const int64_t b = r / 32, rr = r % 32;
-        for (int64_t s = 0; s < st; ++s) {
-            uint8_t* pk = tiles.data() + (b * st + s) * PK;
-            for (int ks = 0; ks < 4; ++ks)
-                for (int h = 0; h < 2; ++h) {
-                    const int64_t at = s * CB + ks * (CB / 4) + h * piece;
-                    if (at + piece <= row_bytes)
-                        std::memcpy(pk + (32 * h + rr) * (PK / 64) + ks * (PK / 256), src + r * row_bytes + at,
-                                    size_t(piece));
+    // Whole packets one after another, pieces of a fixed size.
+    auto pack = [&](auto size) {
+        constexpr int PIECE = decltype(size)::value;
+        for (int64_t b = 0; b < rb; ++b)
+            for (int64_t s = 0; s < st; ++s) {
+                uint8_t* pk = tiles.data() + (b * st + s) * PK;
+                const int live = int(std::min<int64_t>(32, d.w.rows - 32 * b));
+                const int n = int(std::min<int64_t>(8, (row_bytes - s * CB) / PIECE));  // 4 in a half stage
+                for (int rr = 0; rr < live; ++rr) {
+                    const uint8_t* row = src + (32 * b + rr) * row_bytes + s * CB;
+                    for (int q = 0; q < n; ++q)  // piece q: k-step q / 2, half q % 2
+                        std::memcpy(pk + (32 * (q % 2) + rr) * (PK / 64) + (q / 2) * (PK / 256), row + q * PIECE, PIECE);
                 }
-            if (t.dtype != F16)
-                for (int64_t blk = 2 * s; blk < 2 * s + 2 && blk < kb; ++blk)
-                    std::memcpy(tsc.data() + (b * st + s) * TILE_SCALE_BYTES + rr * 4 + (blk - 2 * s) * 2,
-                                t.scales.data() + (r * kb + blk) * 2, 2);
-        }
-    }
+                if (t.dtype == F16) continue;
+                const int64_t blocks = std::min<int64_t>(2, kb - 2 * s);
+                for (int rr = 0; rr < live; ++rr)
+                    std::memcpy(tsc.data() + (b * st + s) * TILE_SCALE_BYTES + rr * 4,
+                                t.scales.data() + ((32 * b + rr) * kb + 2 * s) * 2, size_t(blocks) * 2);
+            }
+    };
+    if (t.dtype == Q4)
+        pack(std::integral_constant<int, 4>{});
+    else if (t.dtype == Q8)
+        pack(std::integral_constant<int, 8>{});
+    else
+        pack(std::integral_constant<int, 16>{});
     d.tiles = upload_bytes(tiles.data(), tiles.size());
     if (!tsc.empty()) d.tscales = upload_bytes(tsc.data(), tsc.size());
     d.w.tiles = d.tiles.as<uint8_t>();
@@ -135,9 +145,9 @@ void Builder::push(const std::string& name, const QTensor& t) {
         return;
     }
     if (t.shape[1] % 32 != 0) fail(E_INVALID, name + ": inner dimension is not a multiple of 32");
-    // The embedding tables are only gathered by rows (and the token table
-    // read by the readout's own kernel), never fed to a GEMM.
-    linears_[name] = upload_weight(t, name != "embed" && name != "per_layer_table");
+    // The per-layer token table is only gathered by rows, never a product's
+    // operand (the token embedding is the readout's).
+    linears_[name] = upload_weight(t, name != "per_layer_table");
     norms_.erase(name);
 }
 
@@ -285,7 +295,8 @@ std::unique_ptr<Engine> Builder::finish(int64_t capacity, int64_t max_rows) {
     const int64_t width = std::max(c.vocab, d);
     E.logits_ = DevBuf(size_t(max_rows * width) * 4);
     E.label_lse_ = DevBuf(size_t(max_rows * (c.vocab + 1)) * 4);
-    E.lse_part_ = DevBuf(size_t(logits_blocks(c.vocab) * max_rows) * 8);
+    // the readout's partials, full rows and split rows
+    E.readout_ = DevBuf(size_t(label_readout_bytes(max_rows, c.vocab, c.vocab, d)));
     E.kv_stage_ = DevBuf(size_t(E.cap_pad_ * 2 * c.kv_heads * hd) * 2);
     if (c.per_layer_dim > 0) {
         const int64_t P = c.per_layer_dim;
@@ -1153,27 +1164,25 @@ void Engine::readout(const PassPlan& p) {
         launch_final_rows(stream_, out_rows_ ? x_w_.as<float>() : x_.as<float>(), out_rows_ ? nullptr : d_wanted_,
                           p.nrows, c.d, final_norm_.as<float>(), c.eps, rows_.as<float>());
     });
+    LogitsOut o;
     if (p.want == WANT_LOGITS) {
+        o.out = logits_.as<float>();
         step("logits", 0, [&] {
-            launch_logits(stream_, embed_.w, rows_.as<float>(), p.nrows, nullptr, c.vocab, c.softcap,
-                          logits_.as<float>());
+            launch_logits(stream_, embed_.w, rows_.as<float>(), p.nrows, nullptr, c.vocab, c.softcap, o, readout_.p);
         });
     } else if (p.want == WANT_LABELS) {
+        o.out = logits_.as<float>();
         step("logits", 0, [&] {
-            launch_logits(stream_, embed_.w, rows_.as<float>(), p.nrows, d_labels_, p.nlabels,
-                          c.softcap, logits_.as<float>());
+            launch_logits(stream_, embed_.w, rows_.as<float>(), p.nrows, d_labels_, p.nlabels, c.softcap, o,
+                          readout_.p);
         });
     } else if (p.want == WANT_LABELS_LSE) {
         // Readout::distribution (readout.rs:124-146) needs the label logits
         // and the log-sum-exp of the whole row: every logit is computed,
         // only k + 1 floats per row leave the device.
-        step("logits", 0, [&] {
-            launch_logits(stream_, embed_.w, rows_.as<float>(), p.nrows, nullptr, c.vocab, c.softcap,
-                          logits_.as<float>(), lse_part_.as<float2>());
-        });
-        step("label_lse", 0, [&] {
-            launch_label_lse(stream_, logits_.as<float>(), p.nrows, c.vocab, lse_part_.as<float2>(),
-                             logits_blocks(c.vocab), d_labels_, p.nlabels, label_lse_.as<float>());
+        step("label_readout", 0, [&] {
+            launch_label_readout(stream_, embed_.w, rows_.as<float>(), p.nrows, d_labels_, p.nlabels, c.softcap,
+                                 label_lse_.as<float>(), readout_.p);
         });
     }
 }

@@ -228,7 +228,7 @@ class Engine {
     const uint32_t* d_labels_ = nullptr;
     // Label logits + full-row log-sum-exp per wanted row (WANT_LABELS_LSE),
     // and the logits kernel's per-workgroup (max, sum of exp) pairs.
-    DevBuf label_lse_, lse_part_;
+    DevBuf label_lse_, readout_;
     DevBuf x16_, pli_, plg_, pl16_;  // per-layer inputs: f16(x), [t][layers x P] f32, gate f32, gated f16
     // attention chunk lengths in key tiles: [0] sliding layers, [1] global
     int attn_chunk_[2] = {0, 0};

@@ -104,6 +104,17 @@ __device__ inline half8 dq4_word(uint32_t w, half2v dd) {
     return half8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 
+// The eight codes of a Q4 device word as exact f16 integers q - 8 (no scale).
+__device__ inline half8 q4_word_codes(uint32_t w) {
+    const half2v o0 = {half_t(1032.0f), half_t(1032.0f)}, o1 = {half_t(72.0f), half_t(72.0f)};
+    const uint32_t u = w >> 8;
+    const half2v h0 = as_half2(and_or(w, 0x000F000Fu, 0x64006400u)) - o0;
+    const half2v h1 = as_half2(and_or(w, 0x00F000F0u, 0x54005400u)) - o1;
+    const half2v h2 = as_half2(and_or(u, 0x000F000Fu, 0x64006400u)) - o0;
+    const half2v h3 = as_half2(and_or(u, 0x00F000F0u, 0x54005400u)) - o1;
+    return half8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
+}
+
 // The same four elements as f32: element 8w+p of a Q4 device word.
 __device__ inline float q4_elem_f32(uint32_t w, int p, float d) {
     const int sh = (p & 1) ? 16 + 4 * (p >> 1) : 4 * (p >> 1);
@@ -124,6 +135,15 @@ __device__ inline half8 dq8_words(uint32_t w0, uint32_t w1, half2v dd) {
     const half2v h1 = (q8_pair(a, 0x04030402u) - off) * dd;
     const half2v h2 = (q8_pair(b, 0x04010400u) - off) * dd;
     const half2v h3 = (q8_pair(b, 0x04030402u) - off) * dd;
+    return half8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
+}
+
+// Eight Q8 codes as exact f16 integers (no scale).
+__device__ inline half8 q8_words_codes(uint32_t w0, uint32_t w1) {
+    const half2v off = {half_t(1152.0f), half_t(1152.0f)};
+    const uint32_t a = w0 ^ 0x80808080u, b = w1 ^ 0x80808080u;
+    const half2v h0 = q8_pair(a, 0x04010400u) - off, h1 = q8_pair(a, 0x04030402u) - off;
+    const half2v h2 = q8_pair(b, 0x04010400u) - off, h3 = q8_pair(b, 0x04030402u) - off;
     return half8{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
 }
 

@@ -113,23 +113,40 @@ void launch_final_rows(hipStream_t s, const float* x, const int32_t* wanted, int
 void launch_gather_out(hipStream_t s, const half_t* a, int64_t wa, const float* x, int64_t wx, const int32_t* rows,
                        int64_t r0, int64_t n, half_t* aw, float* xw, const float* p = nullptr, int64_t ps = 0,
                        int64_t po = 0, int64_t wp = 0, float* pw = nullptr);
-// out[r][j] = rows[r] . deq(E[col(j)]) in f32 (+ softcap), col(j) = cols ? cols[j] : j.
-// logits[r][j] = rows[r] . deq(E[cols ? cols[j] : j]) (softcap applied),
-// f32 [nrows][ncols]; with `part` (logits_blocks(ncols) x nrows pairs) each
-// workgroup's (max, sum of exp) per row for the log-sum-exp.
+// Where launch_logits puts a row's logits: the full rows `out`
+// [nrows][ncols]; per row and 32 columns (max, sum of exp) into `part`
+// [logits_blocks(ncols)][nrows] for the log-sum-exp; the columns named by
+// `labels` into lab_out [nrows][nlabels + 1] (ids past the columns are left
+// alone).  Null: not wanted.
+struct LogitsOut {
+    float* out = nullptr;
+    float2* part = nullptr;
+    const uint32_t* labels = nullptr;
+    int64_t nlabels = 0;
+    float* lab_out = nullptr;
+};
+// logits[r][j] = rows[r] . deq(E[cols ? cols[j] : j]) (softcap applied), at
+// f32 precision, from E's stage tiles.  `scratch` (split_rows_bytes, used
+// above 32 rows) may be null: then the workgroups split the rows themselves.
 void launch_logits(hipStream_t s, const DevWeight& E, const float* rows, int64_t nrows, const uint32_t* cols,
-                   int64_t ncols, float softcap, float* out, float2* part = nullptr);
+                   int64_t ncols, float softcap, const LogitsOut& o, void* scratch);
 int64_t logits_blocks(int64_t ncols);
-// The label readout (logits, then launch_label_lse) with its scratch in a
-// fixed device array instead of allocated memory: nothing is allocated;
-// nrows x vocab + 2 x nrows x logits_blocks(vocab) floats must fit
-// label_readout_scratch_floats().
+int64_t split_rows_bytes(int64_t nrows, int64_t K);
+// The label readout (launch_logits, then launch_label_lse) into out
+// [nrows][nlabels + 1], its scratch (label_readout_bytes, 256-byte aligned)
+// the caller's.
+void launch_label_readout(hipStream_t s, const DevWeight& E, const float* rows, int64_t nrows, const uint32_t* labels,
+                          int64_t nlabels, float softcap, float* out, void* scratch);
+int64_t label_readout_bytes(int64_t nrows, int64_t vocab, int64_t nlabels, int64_t K);
+// The same with its scratch in a fixed device array instead of allocated
+// memory: nothing is allocated; nrows x vocab + 2 x nrows x ceil(vocab / 64)
+// floats must fit its 4,194,304.
 void launch_label_readout_noalloc(hipStream_t s, const DevWeight& E, const float* rows, int64_t nrows,
                                   const uint32_t* labels, int64_t nlabels, float softcap, float* out);
-int64_t label_readout_scratch_floats();
-// Per row of full-vocabulary logits [nrows][vocab] and the logits kernel's
-// partials: the columns `labels`, then log-sum-exp over the whole row, into
-// out [nrows][nlabels + 1].
+// Per row the log-sum-exp over the logits kernel's partials into column
+// nlabels of out [nrows][nlabels + 1]; the label columns from the full rows
+// `logits` [nrows][vocab] (null: already written), NaN for ids past the
+// vocabulary.
 void launch_label_lse(hipStream_t s, const float* logits, int64_t nrows, int64_t vocab, const float2* part,
                       int64_t nblocks, const uint32_t* labels, int64_t nlabels, float* out);
 // Readout::Pointer (readout.rs:30-44): proj[r] = W_m h_r + b_m for each row

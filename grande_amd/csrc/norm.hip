@@ -625,148 +625,472 @@ void launch_gather_out(hipStream_t s, const half_t* a, int64_t wa, const float* 
     OMG_HIP(hipGetLastError());
 }
 
-// logits.wgsl:38-79's product, rows . deq(E[col])^T in f32 (no f16
-// rounding on this path, as in the reference), on v_mfma_f32_16x16x4_f32.
-// A workgroup owns 64 output columns (vocabulary rows of E, or the label
-// ids in `cols`), 16 per wave, and up to LG_R = 16 readout rows at a time:
-// D[col][row] = sum_k E[col][k] x[row][k] with A = the decoded weights
-// (lane l: column l % 16) and B = the rows from LDS.  Inside a 32-element
-// block the K order is permuted alike in both operands: MFMA step s of
-// lane group G = l / 16 takes element 8 G + s, so a lane decodes one Q4
-// word (one Q8 pair, 16 bytes of f16) per block.  A column's sums do not
-// depend on which columns share its wave: full rows, label columns and the
-// log-sum-exp path give bit-equal logits.  With `part`, every workgroup
-// also writes each row's (max, sum of exp(z - max)) over its 64 columns.
-constexpr int LG_R = 16;     // readout rows per pass over K
-constexpr int LG_KC = 512;   // K elements of the rows staged in LDS at once
+// logits.wgsl:38-79's product, rows . deq(E[col])^T at f32 precision (no f16
+// rounding on this path, as in the reference), on v_mfma_f32_32x32x16_f16.
+//
+// The f32 MFMA runs at a sixteenth of the f16 one, so each row is scaled by
+// a power of two (its largest finite |x| into [2^14, 2^15)) and written as
+// two f16 parts, x 2^e = hi + lo: lo is the residual of a rounding to
+// nearest, so what is left out is at most 2^-24 |x|, one f32 rounding.  The
+// weights enter as what their codes say exactly (q - 8, q, or the f16
+// itself), so every product is exact and the sums are f32: per 32-element
+// block, four MFMAs (lo, hi of two 16-wide k-steps) give s_b = sum_k q_k
+// x_k, and acc += d_b s_b is one fma per element (f16 weights: straight
+// into acc).
+//
+// Measured (MI355X, 25,000 columns, Q4): 208 rows of 2,560 (26.6 GFLOP)
+// 647 -> 82 us with its two neighbours, 12 rows of 640 17.3 -> 9.9 us; the
+// distance to float64 fell from 3.8e-7 and 2.0e-7 to 0.9e-7 and 0.7e-7 of
+// the rows' 2-norm.  What bounds it now is VALU issue (decode, the scale
+// fmas) beside the MFMAs.
+//
+// Operands: the rows are A (from LDS), the weights B, straight from the
+// stage tiles (kernels.h) into registers; lane l holds vocabulary column
+// l % 32 of its wave's tile, output rows 8 j + 4 (l / 32) + i in element
+// 4 j + i, so a column's block scale is one value per lane.  The sums of
+// an element do not depend on which rows, columns or tile shapes share the
+// launch: full rows, label columns and the log-sum-exp path give bit-equal
+// logits.  With `part`, each wave also writes every row's (max, sum of
+// exp(z - max)) over its 32 columns.
+constexpr int LG_R = 32;      // readout rows per workgroup (an MFMA row tile)
+constexpr int LG_COLS = 32;   // columns per partial (an MFMA column tile)
+constexpr int LG_ST = 64;     // K per stage, as the weights' stage tiles
+constexpr int LG_FRAG = 1024; // bytes of one A fragment: 64 lanes x 8 f16
+constexpr int LG_PARTS = 2;
+constexpr int LG_STAGE = 4 * LG_PARTS * LG_FRAG;  // one stage of a row tile: 4 k-steps x the parts
+constexpr int LG_KC = 4;      // stages converted at once when the rows are split in the kernel
+constexpr int LG_NS = 3;      // ring slots when they arrive split
 
-// Elements 8 g .. 8 g + 7 of block b of column `col`, f32.
-template <int DT>
-__device__ inline void logit_octet(const DevWeight& E, int64_t col, int64_t b, int g, float w[8]) {
-    const int64_t K = E.cols;
-    if constexpr (DT == Q4_DT) {
-        const float d = half_bits_to_f32(E.scales[col * E.sld + b]);
-        const uint32_t word = static_cast<const uint32_t*>(E.data)[(col * (K / 32) + b) * 4 + g];
+// The power of two that brings |x| <= m into f16's upper range, and its
+// inverse (both normal f32).
+__device__ inline float2 row_scale(float m) {
+    int e = int((__builtin_bit_cast(uint32_t, m) >> 23) & 255) - 127;
+    e = m > 0.0f ? (e < -112 ? -112 : e) : 0;
+    return make_float2(__builtin_bit_cast(float, uint32_t(127 + 14 - e) << 23),
+                       __builtin_bit_cast(float, uint32_t(127 - 14 + e) << 23));
+}
+__device__ inline float finite_abs(float v) {
+    const float a = fabsf(v);
+    return a < INFINITY ? a : 0.0f;
+}
+// v = hi + lo; infinities and NaNs stay in hi alone.
+__device__ inline void split2(const float (&v)[8], half8 (&p)[LG_PARTS]) {
 #pragma unroll
-        for (int p = 0; p < 8; ++p) w[p] = q4_elem_f32(word, p, d);
-    } else if constexpr (DT == Q8_DT) {
-        const float d = half_bits_to_f32(E.scales[col * E.sld + b]);
-        const uint2 u = *reinterpret_cast<const uint2*>(static_cast<const uint8_t*>(E.data) + col * K + b * 32 + 8 * g);
+    for (int i = 0; i < 8; ++i) {
+        const half_t h = half_t(v[i]);
+        p[0][i] = h;
+        p[1][i] = half_t(fabsf(v[i]) < INFINITY ? v[i] - float(h) : 0.0f);
+    }
+}
+
+// The rows split ahead of the product, a workgroup per row (rows past the
+// end and columns past K as zeros): part p of row r, elements
+// 64 st + 16 ks + 8 h .. + 7 at fragment ((r / 32 * stages + st) * 4 + ks) *
+// parts + p, lane 32 h + r % 32; inv[r] undoes the row's scale.
+__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ rows, int64_t nrows, int64_t K,
+                                                         int64_t stages, half_t* __restrict__ frag,
+                                                         float* __restrict__ inv) {
+    __shared__ float red[4];
+    const int tid = int(threadIdx.x), wave = tid / WAVE, lane = tid % WAVE;
+    const int64_t r = blockIdx.x;
+    const bool live = r < nrows;
+    const float* x = rows + r * K;
+    auto group = [&](int64_t g, float (&v)[8]) {
+        float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
+        if (live && 8 * g < K) {
+            a = *reinterpret_cast<const float4*>(x + 8 * g);
+            b = *reinterpret_cast<const float4*>(x + 8 * g + 4);
+        }
+        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+    };
+    // (the first group of each thread stays in registers: the whole row up
+    // to 2,048 wide)
+    float first[8];
+    group(tid, first);
+    float m = 0.0f;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            w[k] = float(int8_t(u.x >> (8 * k))) * d;
-            w[4 + k] = float(int8_t(u.y >> (8 * k))) * d;
+    for (int i = 0; i < 8; ++i) m = fmaxf(m, finite_abs(first[i]));
+    for (int64_t g = tid + 256; g < stages * 8; g += 256) {
+        float v[8];
+        group(g, v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) m = fmaxf(m, finite_abs(v[i]));
+    }
+    m = wave_max(m);
+    if (lane == 0) red[wave] = m;
+    __syncthreads();
+    const float2 sc = row_scale(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+    if (tid == 0) inv[r] = sc.y;
+    for (int64_t g = tid; g < stages * 8; g += 256) {
+        float v[8];
+        if (g == tid) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = first[i];
+        } else {
+            group(g, v);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] *= sc.x;
+        half8 p[LG_PARTS];
+        split2(v, p);
+        const int64_t f = (r / LG_R * stages + g / 8) * 4 + (g % 8) / 2;
+        const int ln = int(32 * (g % 2) + r % LG_R);
+#pragma unroll
+        for (int k = 0; k < LG_PARTS; ++k)
+            *reinterpret_cast<half8*>(frag + (f * LG_PARTS + k) * (LG_FRAG / 2) + ln * 8) = p[k];
+    }
+}
+
+struct LogitArgs {
+    DevWeight E;
+    const float* rows;    // f32 rows, split in the kernel (SPLIT_IN)
+    const half_t* frag;   // split_rows_kernel's fragments
+    const float* inv;     // and row scales
+    int64_t nrows;
+    const uint32_t* cols; // vocabulary rows of the columns, null: all in order
+    int64_t ncols;
+    float softcap;
+    float* out;           // [nrows][ncols] or null
+    float2* part;         // [ceil(ncols / 32)][nrows] or null
+    const uint32_t* labels;  // columns wanted in lab_out [nrows][nlabels + 1] (null: none)
+    int64_t nlabels;
+    float* lab_out;
+};
+
+// Four waves, each CT column tiles of 32 on one row tile of 32.  Per stage
+// a wave has 8 CT MFMAs (32 cycles of its SIMD's matrix core each) against
+// 8 fragment reads, 36 CT decode and 32 CT scale instructions.  A block's
+// scale instructions run one block late, behind the next block's MFMAs:
+// right after their own they would wait out the matrix core's latency.
+// SPLIT_IN: the workgroup splits the rows itself, LG_KC stages at a time,
+// for callers without scratch; otherwise the fragments stream through an
+// LDS ring by DMA.
+template <int DT, int CT, bool SPLIT_IN>
+__global__ __launch_bounds__(256) void logits_kernel(LogitArgs a) {
+    constexpr int CL = tile_packet_bytes(DT) / 1024;  // 16-byte code loads per lane and stage
+    constexpr int PK = tile_packet_bytes(DT);
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = int(threadIdx.x), lane = tid % WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int lc = lane % 32, lh = lane / 32;
+    // Workgroup b runs on XCD b % 8: the row tiles of one column block go to
+    // one XCD, whose L2 then holds those weights for all of them.
+    const int64_t nrt = (a.nrows + LG_R - 1) / LG_R, ncb = (a.ncols + 4 * CT * LG_COLS - 1) / (4 * CT * LG_COLS);
+    const int64_t item = int64_t(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+    if (item >= nrt * ncb) return;
+    const int64_t rt = item % nrt, r0 = rt * LG_R, c0 = (item / nrt * 4 + wave) * CT * LG_COLS;
+    const int64_t K = a.E.cols;
+    const int stages = int(a.E.stages);
+
+    // This lane's columns: their packets' lane run and scale.
+    const uint8_t* wp[CT];
+    const uint8_t* sp[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        const int64_t j = c0 + c * LG_COLS + lc;
+        const int64_t col = j < a.ncols ? (a.cols ? int64_t(a.cols[j]) : j) : 0;  // idle columns: row 0, dropped
+        wp[c] = a.E.tiles + (col / 32) * stages * PK + (32 * lh + col % 32) * (PK / 64);
+        sp[c] = DT == F16_DT ? nullptr : a.E.tscales + (col / 32) * stages * TILE_SCALE_BYTES + (col % 32) * 4;
+    }
+    struct W {
+        uint4 code[CT][CL];
+        uint32_t sc[CT];
+    };
+    auto load_w = [&](int st, W& w) {
+        st = st < stages ? st : stages - 1;
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+#pragma unroll
+            for (int i = 0; i < CL; ++i)
+                w.code[c][i] = *reinterpret_cast<const uint4*>(wp[c] + int64_t(st) * PK + 16 * i);
+            if constexpr (DT != F16_DT)
+                w.sc[c] = *reinterpret_cast<const uint32_t*>(sp[c] + int64_t(st) * TILE_SCALE_BYTES);
+        }
+    };
+    floatx16 acc[CT], late[CT];  // late: the last block's sums, not yet scaled by
+    float ld[CT];                // its scale and added
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        acc[c] = floatx16{};
+        late[c] = floatx16{};
+        ld[c] = 0.0f;
+    }
+    auto add_late = [&] {
+        if constexpr (DT != F16_DT)
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[c][e] = fmaf(late[c][e], ld[c], acc[c][e]);
+    };
+    auto compute = [&](const uint8_t* S, const W& w) {
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
+            // A block's fragment reads go out together.
+            half8 xf[2][LG_PARTS];
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                for (int p = LG_PARTS - 1; p >= 0; --p)
+                    xf[k][p] = *reinterpret_cast<const half8*>(S + ((2 * blk + k) * LG_PARTS + p) * LG_FRAG + lane * 16);
+            half8 wf[CT][2];
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const int ks = 2 * blk + k;
+                    if constexpr (DT == Q4_DT) {
+                        const uint4 u = w.code[c][0];
+                        wf[c][k] = q4_word_codes(ks == 0 ? u.x : ks == 1 ? u.y : ks == 2 ? u.z : u.w);
+                    } else if constexpr (DT == Q8_DT) {
+                        const uint4 u = w.code[c][blk];
+                        wf[c][k] = k == 0 ? q8_words_codes(u.x, u.y) : q8_words_codes(u.z, u.w);
+                    } else {
+                        wf[c][k] = __builtin_bit_cast(half8, w.code[c][ks]);
+                    }
+                }
+            floatx16 s[CT];
+#pragma unroll
+            for (int c = 0; c < CT; ++c) s[c] = DT == F16_DT ? acc[c] : floatx16{};
+#pragma unroll
+            for (int p = LG_PARTS - 1; p >= 0; --p)
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+#pragma unroll
+                    for (int c = 0; c < CT; ++c)
+                        s[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[k][p], wf[c][k], s[c], 0, 0, 0);
+            if constexpr (DT == F16_DT) {
+#pragma unroll
+                for (int c = 0; c < CT; ++c) acc[c] = s[c];
+            } else {
+                add_late();
+#pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    late[c] = s[c];
+                    ld[c] = half_bits_to_f32(uint16_t(w.sc[c] >> (16 * blk)));
+                }
+            }
+        }
+    };
+
+    // Weights R - 1 stages ahead in registers.
+    constexpr int R = DT == Q4_DT ? 4 : 2;
+    W w[R];
+    __shared__ float sinv[LG_R];
+    auto first_w = [&] {
+#pragma unroll
+        for (int u = 0; u < R - 1; ++u) load_w(u, w[u]);
+    };
+    if constexpr (SPLIT_IN) {
+        first_w();
+        // Eight threads per row: its largest finite |x|, then the parts of
+        // LG_KC stages at a time (thread: four 8-element groups).
+        const int64_t row = r0 + tid / 8;
+        const int sub = tid % 8, rr = tid / 8;
+        const bool live = row < a.nrows;
+        const float* x = a.rows + row * K;
+        float m = 0.0f;
+        if (live)
+            for (int64_t q = sub; q < K / 4; q += 8) {
+                const float4 v = *reinterpret_cast<const float4*>(x + 4 * q);
+                m = fmaxf(m, fmaxf(fmaxf(finite_abs(v.x), finite_abs(v.y)), fmaxf(finite_abs(v.z), finite_abs(v.w))));
+            }
+#pragma unroll
+        for (int o = 4; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, WAVE));
+        const float2 sc = row_scale(m);
+        if (sub == 0) sinv[rr] = sc.y;
+        float4 raw[LG_KC][2];
+        auto load_x = [&](int st0) {
+#pragma unroll
+            for (int g = 0; g < LG_KC; ++g) {
+                const int64_t k = int64_t(st0 + g) * LG_ST + 8 * sub;
+                const bool in = live && k < K;
+                raw[g][0] = in ? *reinterpret_cast<const float4*>(x + k) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                raw[g][1] = in ? *reinterpret_cast<const float4*>(x + k + 4) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+        };
+        load_x(0);
+        for (int st0 = 0; st0 < stages; st0 += LG_KC) {
+            __syncthreads();  // the previous stages' reads are done
+#pragma unroll
+            for (int g = 0; g < LG_KC; ++g) {
+                const float4 u = raw[g][0], v = raw[g][1];
+                const float e[8] = {u.x * sc.x, u.y * sc.x, u.z * sc.x, u.w * sc.x,
+                                    v.x * sc.x, v.y * sc.x, v.z * sc.x, v.w * sc.x};
+                half8 p[LG_PARTS];
+                split2(e, p);
+#pragma unroll
+                for (int k = 0; k < LG_PARTS; ++k)
+                    *reinterpret_cast<half8*>(smem + g * LG_STAGE + ((sub / 2) * LG_PARTS + k) * LG_FRAG +
+                                              (32 * (sub % 2) + rr) * 16) = p[k];
+            }
+            __syncthreads();
+            if (st0 + LG_KC < stages) load_x(st0 + LG_KC);
+            const int n = stages - st0 < LG_KC ? stages - st0 : LG_KC;
+#pragma unroll
+            for (int g = 0; g < LG_KC; ++g) {
+                if (g >= n) break;
+                load_w(st0 + g + R - 1, w[(g + R - 1) % R]);
+                compute(smem + g * LG_STAGE, w[g % R]);
+            }
         }
     } else {
-        const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const half_t*>(E.data) + col * K + b * 32 + 8 * g);
-        const uint32_t words[4] = {u.x, u.y, u.z, u.w};
+        if (tid < LG_R) sinv[tid] = a.inv[r0 + tid];
+        const uint8_t* src = reinterpret_cast<const uint8_t*>(a.frag) + rt * stages * int64_t(LG_STAGE);
+        constexpr int XI = LG_STAGE / 4096;  // this wave's DMA instructions per stage
+        auto issue = [&](int st) {
+            uint8_t* base = smem + (unsigned(st) % unsigned(LG_NS)) * LG_STAGE;
+            const uint8_t* g = src + int64_t(st < stages ? st : stages - 1) * LG_STAGE;
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(g), (short)0,
+                                                                                LG_STAGE, 0x00020000);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const half2v h = as_half2(words[k]);
-            w[2 * k] = float(h.x);
-            w[2 * k + 1] = float(h.y);
+            for (int i = 0; i < XI; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    rs, (__attribute__((address_space(3))) void*)(base + (i * 4 + wave) * WAVE * 16), 16,
+                    uint32_t((i * 256 + tid) * 16), 0, 0, 0);
+        };
+        constexpr int WL = CT * (CL + (DT == F16_DT ? 0 : 1));  // and its weight loads
+        static_assert(XI + WL <= 15, "vmcnt field");
+        // The wait below counts the memory instructions after a stage's DMA,
+        // so their order is pinned by compiler fences: W, DMA, W, DMA, ...
+        auto fence = [] { asm volatile("" ::: "memory"); };
+        issue(0);
+        fence();
+        first_w();
+        fence();
+        issue(1);
+        for (int st0 = 0; st0 < stages; st0 += R)
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                const int st = st0 + u;
+                if (st >= stages) break;
+                // Stage st's fragments landed once only what follows their
+                // DMA is out: one stage's weights and the next stage's DMA.
+                // Past the barrier everyone's have, and everyone is done
+                // with stage st - 1, whose slot stage st + 2 takes.
+                fence();
+                __builtin_amdgcn_s_waitcnt((XI + WL) | (7 << 4) | (15 << 8));
+                __builtin_amdgcn_s_waitcnt(0xc07f);
+                __builtin_amdgcn_s_barrier();
+                fence();
+                load_w(st + R - 1, w[(u + R - 1) % R]);
+                fence();
+                issue(st + 2);
+                fence();
+                compute(smem + (unsigned(st) % unsigned(LG_NS)) * LG_STAGE, w[u]);
+            }
+        __builtin_amdgcn_s_waitcnt(0);  // no DMA into LDS outlives the workgroup
+    }
+
+    add_late();
+    // Each wave's tile through LDS (its own 32 rows of 33 floats, where the
+    // fragments were): the row statistics then take two lanes per row
+    // instead of a 32-lane reduction per element.
+    __syncthreads();
+    constexpr int TS = LG_COLS + 1;
+    float* T = reinterpret_cast<float*>(smem) + wave * LG_R * TS;
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        const int64_t j0 = c0 + c * LG_COLS, j = j0 + lc;
+        if (j0 >= a.ncols) break;
+        float z[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) z[e] = acc[c][e] * sinv[8 * (e / 4) + 4 * lh + e % 4];
+        if (a.softcap > 0.0f)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) z[e] = a.softcap * tanhf(z[e] / a.softcap);
+        if (a.out && j < a.ncols)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int64_t r = r0 + 8 * (e / 4) + 4 * lh + e % 4;
+                if (r < a.nrows) a.out[r * a.ncols + j] = z[e];
+            }
+        if (!a.part && a.nlabels == 0) continue;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) T[(8 * (e / 4) + 4 * lh + e % 4) * TS + lc] = z[e];
+        // The wanted labels among this tile's columns.
+        for (int64_t l0 = 0; l0 < a.nlabels; l0 += WAVE) {
+            const int64_t mine = l0 + lane < a.nlabels ? int64_t(a.labels[l0 + lane]) : -1;
+            uint64_t hits = __ballot(mine >= j0 && mine < j0 + LG_COLS && mine < a.ncols);
+            while (hits) {
+                const int i = __builtin_ctzll(hits);
+                hits &= hits - 1;
+                const int col = __builtin_amdgcn_readlane(int(mine - j0), i);
+                if (lh == 0 && r0 + lc < a.nrows) a.lab_out[(r0 + lc) * (a.nlabels + 1) + l0 + i] = T[lc * TS + col];
+            }
+        }
+        if (a.part) {
+            // per row: max and sum of exp over the tile's 32 columns, two
+            // lanes of 16 columns each
+            const int row = lane / 2, h = lane % 2;
+            float v[16];
+            float m = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                v[i] = j0 + 16 * h + i < a.ncols ? T[row * TS + 16 * h + i] : -INFINITY;
+                m = fmaxf(m, v[i]);
+            }
+            m = fmaxf(m, dpp_f32<0xb1>(m));
+            float s = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s += j0 + 16 * h + i < a.ncols ? expf(v[i] - m) : 0.0f;
+            s += dpp_f32<0xb1>(s);
+            if (h == 0 && r0 + row < a.nrows) a.part[(j0 / LG_COLS) * a.nrows + r0 + row] = make_float2(m, s);
         }
     }
 }
 
+int64_t logits_blocks(int64_t ncols) { return (ncols + LG_COLS - 1) / LG_COLS; }
+
+// Bytes of the fragments and scales of nrows split rows.
+int64_t split_rows_bytes(int64_t nrows, int64_t K) {
+    return (nrows + LG_R - 1) / LG_R * (((K + LG_ST - 1) / LG_ST) * LG_STAGE + LG_R * 4);
+}
+
+template <int DT, int CT, bool SPLIT_IN>
+static void run_logits(hipStream_t s, const LogitArgs& a) {
+    constexpr int lds = (SPLIT_IN ? LG_KC : LG_NS) * LG_STAGE;
+    static_assert(lds >= 4 * LG_R * (LG_COLS + 1) * 4, "the waves' output tiles fit the ring");
+    const int64_t items = (a.nrows + LG_R - 1) / LG_R * ((a.ncols + 4 * CT * LG_COLS - 1) / (4 * CT * LG_COLS));
+    logits_kernel<DT, CT, SPLIT_IN><<<dim3(unsigned((items + 7) / 8 * 8)), dim3(256), lds, s>>>(a);
+}
+
 template <int DT>
-__global__ __launch_bounds__(256) void logits_kernel(DevWeight E, const float* __restrict__ rows, int64_t nrows,
-                                                     const uint32_t* __restrict__ cols, int64_t ncols, float softcap,
-                                                     float* __restrict__ out, float2* __restrict__ part) {
-    __shared__ __attribute__((aligned(16))) float xs[LG_R][LG_KC];
-    __shared__ float red[4][LG_R][2];
-    const int tid = int(threadIdx.x), lane = tid % WAVE;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-    const int lr = lane % 16, G = lane / 16;
-    // A operand: column wave * 16 + lr of the workgroup's 64
-    const int64_t ja = int64_t(blockIdx.x) * 64 + wave * 16 + lr;
-    const int64_t col = ja < ncols ? (cols ? int64_t(cols[ja]) : ja) : 0;  // idle columns read row 0, dropped
-    // D: columns wave * 16 + 4 G + r, row lr
-    const int64_t jd = int64_t(blockIdx.x) * 64 + wave * 16 + 4 * G;
-    const int64_t K = E.cols;
-    for (int64_t r0 = 0; r0 < nrows; r0 += LG_R) {
-        const int nr = int(nrows - r0 < LG_R ? nrows - r0 : LG_R);
-        floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int64_t k0 = 0; k0 < K; k0 += LG_KC) {
-            const int kc = int(K - k0 < LG_KC ? K - k0 : LG_KC);
-            __syncthreads();  // the previous chunk's reads are done
-            for (int i = tid; i < LG_R * (kc / 4); i += 256) {
-                const int r = i / (kc / 4), c4 = i % (kc / 4);
-                const float4 v = r < nr ? *reinterpret_cast<const float4*>(rows + (r0 + r) * K + k0 + 4 * c4)
-                                        : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                *reinterpret_cast<float4*>(&xs[r][4 * c4]) = v;
-            }
-            __syncthreads();
-            for (int bl = 0; bl < kc / 32; ++bl) {
-                float w[8];
-                logit_octet<DT>(E, col, k0 / 32 + bl, G, w);
-                const float4 x0 = *reinterpret_cast<const float4*>(&xs[lr][bl * 32 + 8 * G]);
-                const float4 x1 = *reinterpret_cast<const float4*>(&xs[lr][bl * 32 + 8 * G + 4]);
-                const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-#pragma unroll
-                for (int st = 0; st < 8; ++st) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[st], x[st], acc, 0, 0, 0);
-            }
-        }
-        // lane: row lr, columns jd .. jd + 3
-        const bool row_ok = lr < nr;
-        float z[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            z[r] = acc[r];
-            if (softcap > 0.0f) z[r] = softcap * tanhf(z[r] / softcap);
-        }
-        if (row_ok) {
-            float* dst = out + (r0 + lr) * ncols + jd;
-            // (rows of a width that is not a multiple of 4 start off the
-            // 16-byte grid: those go out as single floats)
-            if (jd + 3 < ncols && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-                *reinterpret_cast<float4*>(dst) = make_float4(z[0], z[1], z[2], z[3]);
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (jd + r < ncols) dst[r] = z[r];
-            }
-        }
-        if (part) {
-            // per row: max and sum of exp over the workgroup's 64 columns,
-            // lanes (row, G) then waves in a fixed order
-            float m = -INFINITY;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) m = fmaxf(m, jd + r < ncols ? z[r] : -INFINITY);
-            m = max_lanes_16_32(m);
-            if (G == 0) red[wave][lr][0] = m;
-            __syncthreads();
-            m = fmaxf(fmaxf(red[0][lr][0], red[1][lr][0]), fmaxf(red[2][lr][0], red[3][lr][0]));
-            float e = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) e += jd + r < ncols ? expf(z[r] - m) : 0.0f;
-            e = sum_lanes_16_32(e);
-            if (G == 0) red[wave][lr][1] = e;
-            __syncthreads();
-            if (wave == 0 && G == 0 && row_ok)
-                part[int64_t(blockIdx.x) * nrows + r0 + lr] =
-                    make_float2(m, ((red[0][lr][1] + red[1][lr][1]) + red[2][lr][1]) + red[3][lr][1]);
-        }
-    }
+static void dispatch_logits(hipStream_t s, const LogitArgs& a, void* scratch) {
+    if (!scratch) return run_logits<DT, 1, true>(s, a);
+    const int64_t nrt = (a.nrows + LG_R - 1) / LG_R, st = a.E.stages;
+    LogitArgs b = a;
+    half_t* frag = static_cast<half_t*>(scratch);
+    float* inv = reinterpret_cast<float*>(static_cast<uint8_t*>(scratch) + nrt * st * LG_STAGE);
+    split_rows_kernel<<<dim3(unsigned(nrt * LG_R)), dim3(256), 0, s>>>(a.rows, a.nrows, a.E.cols, st, frag, inv);
+    OMG_HIP(hipGetLastError());
+    b.frag = frag;
+    b.inv = inv;
+    // Two column tiles per wave (half the fragment reads per MFMA) once that
+    // leaves every CU two workgroups: 208 rows of the 4B width 85 -> 82 us;
+    // below it one, for the workgroups (60 rows, d 1,536, f16: 36 -> 32 us).
+    if (nrt * ((a.ncols + 8 * LG_COLS - 1) / (8 * LG_COLS)) >= 512) return run_logits<DT, 2, false>(s, b);
+    run_logits<DT, 1, false>(s, b);
 }
 
 void launch_logits(hipStream_t s, const DevWeight& E, const float* rows, int64_t nrows, const uint32_t* cols,
-                   int64_t ncols, float softcap, float* out, float2* part) {
+                   int64_t ncols, float softcap, const LogitsOut& o, void* scratch) {
     if (nrows <= 0 || ncols <= 0) return;
     if (E.cols % 32 != 0) fail(E_INVALID, "logits: width must be a multiple of 32");
-    if (reinterpret_cast<uintptr_t>(rows) % 16 != 0 || reinterpret_cast<uintptr_t>(out) % 4 != 0 ||
-        reinterpret_cast<uintptr_t>(part) % 8 != 0)
+    if (!E.tiles || E.stages != (E.cols + LG_ST - 1) / LG_ST || (E.dtype != F16_DT && !E.tscales))
+        fail(E_INVALID, "logits: weight without stage tiles");
+    if (reinterpret_cast<uintptr_t>(rows) % 16 != 0 || reinterpret_cast<uintptr_t>(o.out) % 4 != 0 ||
+        reinterpret_cast<uintptr_t>(o.part) % 8 != 0 || reinterpret_cast<uintptr_t>(scratch) % 16 != 0)
         fail(E_INVALID, "logits: rows must be 16-byte aligned, the output 4-byte and the partials 8-byte aligned");
-    const dim3 grid(unsigned((ncols + WAVE - 1) / WAVE)), block(256);
+    const LogitArgs a{E,       rows,     nullptr, nullptr,  nrows,
+                      cols,    ncols,    softcap, o.out,    o.part,
+                      o.labels, o.labels ? o.nlabels : 0, o.lab_out};
     switch (E.dtype) {
-        case F16_DT: logits_kernel<F16_DT><<<grid, block, 0, s>>>(E, rows, nrows, cols, ncols, softcap, out, part); break;
-        case Q8_DT: logits_kernel<Q8_DT><<<grid, block, 0, s>>>(E, rows, nrows, cols, ncols, softcap, out, part); break;
-        default: logits_kernel<Q4_DT><<<grid, block, 0, s>>>(E, rows, nrows, cols, ncols, softcap, out, part); break;
+        case F16_DT: dispatch_logits<F16_DT>(s, a, scratch); break;
+        case Q8_DT: dispatch_logits<Q8_DT>(s, a, scratch); break;
+        default: dispatch_logits<Q4_DT>(s, a, scratch); break;
     }
     OMG_HIP(hipGetLastError());
 }
-
-int64_t logits_blocks(int64_t ncols) { return (ncols + WAVE - 1) / WAVE; }
 
 // Readout::distribution's inputs per row (readout.rs:124-146): the label
 // columns of a full logits row and the row's log-sum-exp, from the logits
@@ -799,11 +1123,13 @@ __global__ __launch_bounds__(256) void label_lse_kernel(const float* __restrict_
     sum = wave_sum(sum);
     if (lane == 0) red[wave] = sum;
     __syncthreads();
-    const float* row = logits + r * vocab;
     float* o = out + r * (nlabels + 1);
     for (int64_t i = tid; i < nlabels; i += 256) {
         const uint32_t c = labels[i];
-        o[i] = int64_t(c) < vocab ? row[c] : __builtin_nanf("");
+        if (int64_t(c) >= vocab)
+            o[i] = __builtin_nanf("");
+        else if (logits)  // null: the logits kernel wrote the label columns
+            o[i] = logits[r * vocab + c];
     }
     if (tid == 0) o[nlabels] = m + logf((red[0] + red[1]) + (red[2] + red[3]));
 }
@@ -875,12 +1201,16 @@ void launch_pointer(hipStream_t s, const float* rows, int64_t nrows, int64_t d, 
 
 // Scratch of launch_label_readout_noalloc: the full logits rows, then the
 // logits kernel's (max, sum of exp) pairs.  A file-scope device array, so
-// every GPU the library runs on holds its own copy (16 MiB) until the
+// every GPU the library runs on holds its own copy (17 MiB) until the
 // process ends; calls that overlap on one GPU share it and race.  Nothing
 // in it needs to start at zero: both parts are written whole before they
 // are read.
+// The limit counts a pair per row and 64 columns; the kernel writes one per
+// 32, at most 2 / 35 of the limit more (vocabularies of 33 to 64 rows).
 constexpr int64_t READOUT_SCRATCH_FLOATS = int64_t(4) << 20;
-static __device__ __align__(256) float scratch[READOUT_SCRATCH_FLOATS];
+constexpr int64_t READOUT_SCRATCH_EXTRA = int64_t(1) << 18;
+static_assert(READOUT_SCRATCH_EXTRA * 35 >= READOUT_SCRATCH_FLOATS * 2, "partials of 32 columns fit");
+static __device__ __align__(256) float scratch[READOUT_SCRATCH_FLOATS + READOUT_SCRATCH_EXTRA];
 
 // The array's device address on the current GPU, looked up once per device
 // (in host code `scratch` names a host-side stand-in, not device memory).
@@ -901,20 +1231,70 @@ static float* readout_scratch() {
     return ptr[dev];
 }
 
-int64_t label_readout_scratch_floats() { return READOUT_SCRATCH_FLOATS; }
+// The label readout's two launches.  With up to LABEL_SCAN labels every
+// column tile looks its own columns up among them and writes those logits
+// itself; with more, the full rows go to `logits` [nrows][vocab] and are
+// picked from there (a scan per tile would cost more than the rows).
+constexpr int64_t LABEL_SCAN = 512;
+
+static void label_readout(hipStream_t s, const DevWeight& E, const float* rows, int64_t nrows, const uint32_t* labels,
+                          int64_t nlabels, float softcap, float* out, float* logits, float2* part, void* split) {
+    LogitsOut o;
+    o.part = part;
+    if (nlabels <= LABEL_SCAN) {
+        o.labels = labels;
+        o.nlabels = nlabels;
+        o.lab_out = out;
+        logits = nullptr;
+    } else {
+        o.out = logits;
+    }
+    launch_logits(s, E, rows, nrows, nullptr, E.rows, softcap, o, split);
+    launch_label_lse(s, logits, nrows, E.rows, part, logits_blocks(E.rows), labels, nlabels, out);
+}
+
+// Scratch layout: partials, then (more labels than a scan takes) the full
+// rows, then the split rows.
+static int64_t a256(int64_t n) { return (n + 255) / 256 * 256; }
+int64_t label_readout_bytes(int64_t nrows, int64_t vocab, int64_t nlabels, int64_t K) {
+    return a256(logits_blocks(vocab) * nrows * 8) + (nlabels > LABEL_SCAN ? a256(nrows * vocab * 4) : 0) +
+           split_rows_bytes(nrows, K);
+}
+void launch_label_readout(hipStream_t s, const DevWeight& E, const float* rows, int64_t nrows, const uint32_t* labels,
+                          int64_t nlabels, float softcap, float* out, void* scratch) {
+    if (nrows <= 0 || nlabels <= 0) fail(E_INVALID, "label readout: no rows or no labels");
+    uint8_t* p = static_cast<uint8_t*>(scratch);
+    float2* part = reinterpret_cast<float2*>(p);
+    p += a256(logits_blocks(E.rows) * nrows * 8);
+    float* logits = reinterpret_cast<float*>(p);
+    if (nlabels > LABEL_SCAN) p += a256(nrows * E.rows * 4);
+    label_readout(s, E, rows, nrows, labels, nlabels, softcap, out, logits, part, p);
+}
 
 void launch_label_readout_noalloc(hipStream_t s, const DevWeight& E, const float* rows, int64_t nrows,
                                   const uint32_t* labels, int64_t nlabels, float softcap, float* out) {
     if (nrows <= 0 || nlabels <= 0) fail(E_INVALID, "label readout: no rows or no labels");
-    const int64_t vocab = E.rows, nb = logits_blocks(vocab);
+    // What is accepted: full rows and a pair per row and 64 columns in the
+    // scratch.  The partials alone (a pair per 32 columns) always fit then;
+    // the split rows go behind them where they fit, else the workgroups
+    // split the rows themselves.
+    const int64_t vocab = E.rows;
     const int64_t nlog = (nrows * vocab + 1) / 2 * 2;  // float2 partials on an 8-byte boundary
-    if (nlog + 2 * nb * nrows > READOUT_SCRATCH_FLOATS)
+    if (nlog + 2 * ((vocab + 63) / 64) * nrows > READOUT_SCRATCH_FLOATS)
         fail(E_CAPACITY, "label_readout_noalloc: " + std::to_string(nrows) + " rows x " + std::to_string(vocab) +
                              " logits exceed the " + std::to_string(READOUT_SCRATCH_FLOATS) + "-float scratch");
-    float* base = readout_scratch();
-    float2* part = reinterpret_cast<float2*>(base + nlog);
-    launch_logits(s, E, rows, nrows, nullptr, vocab, softcap, base, part);
-    launch_label_lse(s, base, nrows, vocab, part, nb, labels, nlabels, out);
+    uint8_t* p = reinterpret_cast<uint8_t*>(readout_scratch());
+    if (nlabels > LABEL_SCAN) {
+        // The full rows first, the labels read from them; then the partials.
+        float* base = reinterpret_cast<float*>(p);
+        label_readout(s, E, rows, nrows, labels, nlabels, softcap, out, base, reinterpret_cast<float2*>(base + nlog),
+                      nullptr);
+        return;
+    }
+    float2* part = reinterpret_cast<float2*>(p);
+    const int64_t used = a256(logits_blocks(vocab) * nrows * 8);
+    const bool fits = used + split_rows_bytes(nrows, E.cols) <= READOUT_SCRATCH_FLOATS * 4;
+    label_readout(s, E, rows, nrows, labels, nlabels, softcap, out, nullptr, part, fits ? p + used : nullptr);
 }
 
 // ---------------------------------------------------------- state rows

@@ -272,13 +272,15 @@ int omg_dev_gemm_geglu(const omg_weight *wg, const omg_weight *wu, const void *x
  * 16-byte aligned.  Label ids must be below vocab; the device-resident ids
  * are not checked before the launch, and an id past the vocabulary gives
  * NaN in its column.  The full logits and per-workgroup partials live in
- * scratch device memory the call allocates and frees in stream order. */
+ * scratch device memory: up to 64 MiB kept with the weight for the first
+ * stream it is read out on, otherwise (another stream, under capture, more)
+ * allocated and freed by the call in stream order. */
 int omg_dev_label_readout(const omg_weight *embed, const float *rows, int64_t nrows, const uint32_t *labels,
                           int64_t nlabels, float softcap, float *out, void *stream);
 /* No counterpart in the reference.  omg_dev_label_readout for callers that
  * cannot allocate (code under HIP graph capture, tight serving loops):
  * same arguments and results, nothing allocated; its scratch is a fixed
- * 16 MiB device array per GPU (4,194,304 floats), which must hold
+ * 17 MiB device array per GPU, of which 4,194,304 floats must hold
  * nrows * vocab (rounded up to even) + 2 * nrows * ceil(vocab / 64) floats,
  * else OMG_E_CAPACITY.
  * Calls that overlap on one GPU share that array and race. */

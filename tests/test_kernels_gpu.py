@@ -200,3 +200,75 @@ def test_label_readout_odd_shapes_and_out_of_vocab_labels():
     assert np.isnan(got[:, :-1][:, ~ok]).all()
     assert np.max(np.abs(got[:, :-1][:, ok] - z[:, labels[ok]])) < 1e-4 * max(1.0, np.abs(z).max())
     assert np.max(np.abs(got[:, -1] - lse) / np.maximum(np.abs(lse), 1.0)) < 1e-5
+
+
+# The split-row readout's edges: row tiles of 32 (31, 32, 33, 65 rows), K
+# stages of 64 (32: half a stage, 96: a half last stage, 1,312: past the
+# converted chunks), column tiles of 32 / 128 / 256 (31, 257, 1,025, 31,000
+# columns: two column tiles per wave), more labels than a tile scans.
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("vocab,d,nrows,nlabels", [(31, 32, 31, 3), (257, 96, 32, 26), (1025, 1312, 33, 600),
+                                                   (31000, 64, 130, 26), (640, 4096, 65, 5)])
+def test_split_readout_edges(vocab, d, nrows, nlabels, dtype):
+    """Two f16 parts per row element leave out at most 2^-24 of it, products
+    are exact and a column's sums are f32 over at most 2 d / 16 + d / 32
+    roundings: 2^-24 (2 + d / 8) of sum |x||w| bounds a logit's error (and
+    the log-sum-exp's, plus its own few ulps).  Rows of very different
+    magnitudes share a launch; with and without scratch the logits are the
+    same bits."""
+    rng = np.random.default_rng(vocab * 7 + d + nrows + dtype)
+    t, _ = weight(rng, vocab, d, dtype, "embed")
+    e = t.to_f32().astype(np.float64)
+    rows = rng.standard_normal((nrows, d)).astype(np.float32)
+    rows[0] *= 1e-20
+    rows[nrows // 2] = 0.0
+    rows[-1, ::7] *= 50.0
+    labels = rng.integers(0, vocab, nlabels).astype(np.uint32)
+    w = g.DeviceWeight(t)
+    rd, lab = dev(rows), dev(labels.view(np.int32))
+    outs = []
+    for f in (w.label_readout, w.label_readout_noalloc):
+        out = torch.full((nrows, nlabels + 1), float("nan"), dtype=torch.float32, device="cuda")
+        f(rd.data_ptr(), nrows, lab.data_ptr(), nlabels, 0.0, out.data_ptr())
+        torch.cuda.synchronize()
+        outs.append(out.cpu().numpy())
+    assert np.array_equal(outs[0], outs[1])
+    z = rows.astype(np.float64) @ e.T
+    bound = 2.0 ** -24 * (2 + d / 8) * (np.abs(rows).astype(np.float64) @ np.abs(e).T)
+    assert (np.abs(outs[0][:, :-1] - z[:, labels]) <= bound[:, labels] + 1e-45).all()
+    m = z.max(1)
+    lse = m + np.log(np.exp(z - m[:, None]).sum(1))
+    assert (np.abs(outs[0][:, -1] - lse) <= bound.max(1) + 1e-6 * np.maximum(1.0, np.abs(lse))).all()
+
+
+def test_readout_of_non_finite_rows_and_streams():
+    """An infinity or a NaN in a row stays in that row; calls on two streams
+    with one weight keep apart."""
+    rng = np.random.default_rng(9)
+    vocab, d, nrows = 500, 128, 40
+    t, _ = weight(rng, vocab, d, g.Q8, "embed")
+    w = g.DeviceWeight(t)
+    rows = rng.standard_normal((nrows, d)).astype(np.float32)
+    labels = dev(np.arange(26, dtype=np.int32))
+    streams = [torch.cuda.Stream() for _ in range(2)]
+
+    def readout(r, s=None):
+        rd = dev(r)
+        out = torch.zeros((nrows, 27), dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        w.label_readout(rd.data_ptr(), nrows, labels.data_ptr(), 26, 0.0, out.data_ptr(), s.cuda_stream if s else None)
+        return rd, out
+
+    ref = readout(rows)[1]
+    other = readout(rows[::-1].copy())[1]
+    held = [readout(rows if i % 2 == 0 else rows[::-1].copy(), streams[i % 2]) for i in range(8)]
+    torch.cuda.synchronize()
+    for i, (_, out) in enumerate(held):
+        assert torch.equal(out, ref if i % 2 == 0 else other)
+    bad = rows.copy()
+    bad[3, 5], bad[17, 100] = np.inf, np.nan
+    got = readout(bad)[1].cpu().numpy()
+    torch.cuda.synchronize()
+    live = [r for r in range(nrows) if r not in (3, 17)]
+    assert np.array_equal(got[live], ref.cpu().numpy()[live])
+    assert not np.isfinite(got[3, :26]).any() and np.isnan(got[17]).all()
