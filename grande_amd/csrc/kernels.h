@@ -225,6 +225,25 @@ void launch_add_ln_final(hipStream_t s, float* x, const float* a, const float* w
 void launch_gather_rows(hipStream_t s, const float* x, const float* a, const float* bias, const int32_t* rows,
                         int64_t n, int64_t d, float* out);
 
+// The decision head's scorer (laya.rs:1442-1485).  z[j] = LayerNorm of
+// marker row mrow[j]; h = z . l1^T (launch_logits); then per sequence (its
+// rows: [CLS], then its markers; markers first[s] .. first[s + 1]) the
+// marker logits gelu(h + l1_b) . l2 + l2_b and, with an act head, softmax(
+// gelu([CLS, features] . w1 + b1) . w2^T + b2)[0].
+void launch_score_norm(hipStream_t s, const float* rows, const int32_t* mrow, int64_t n, int64_t d, const float* w,
+                       const float* b, float eps, float* z);
+struct ScoreArgs {
+    const float* rows;     // [sequences + markers][d]
+    const float* h;        // [markers][d]
+    const int32_t* first;  // [sequences + 1]
+    int64_t d;
+    const float *l1_b, *l2, *l2_b;
+    const float *w1t, *b1, *w2, *b2;  // w1t [d + 4][act_hidden], w2 [act_out][act_hidden]
+    int64_t act_hidden, act_out;      // act_out 0: no act head
+    float *logits, *act;
+};
+void launch_score(hipStream_t s, const ScoreArgs& a, int64_t n);
+
 // Column of cache row `row` inside its 64-row V^T tile.  Within each half
 // of 32 keys, key k sits at 8 * ((k % 16) / 4) + 4 * (k / 16) + k % 4: the
 // eight keys one MFMA lane holds probabilities for (4g..4g+3 and

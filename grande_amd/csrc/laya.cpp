@@ -1,5 +1,6 @@
 // The encoder path's host side: config, seeded weights, builder, the pass
-// plan (laya.rs:1138-1432) and the host scorer (laya.rs:1442-1547).
+// plan (laya.rs:1138-1432) and the scorer's launches (laya.rs:1442-1485,
+// which the reference runs on the host).
 #include "laya.h"
 
 #include <algorithm>
@@ -24,58 +25,6 @@ int64_t count(const std::vector<int64_t>& s) {
 bool ends_with(const std::string& s, const char* suf) {
     const size_t n = std::strlen(suf);
     return s.size() >= n && s.compare(s.size() - n, n, suf) == 0;
-}
-
-// laya.rs:1496-1547: the host half in f32, sums in order.
-std::vector<float> layer_norm(const float* x, int64_t n, const float* w, const float* b, float eps) {
-    float mean = 0.0f;
-    for (int64_t i = 0; i < n; ++i) mean += x[i];
-    mean /= float(n);
-    float var = 0.0f;
-    for (int64_t i = 0; i < n; ++i) var += (x[i] - mean) * (x[i] - mean);
-    var /= float(n);
-    const float inv = 1.0f / std::sqrt(var + eps);
-    std::vector<float> y(static_cast<size_t>(n));
-    for (int64_t i = 0; i < n; ++i) y[size_t(i)] = (x[i] - mean) * inv * w[i] + b[i];
-    return y;
-}
-
-float dot(const float* a, const float* b, int64_t n) {
-    float s = 0.0f;
-    for (int64_t i = 0; i < n; ++i) s += a[i] * b[i];
-    return s;
-}
-
-std::vector<float> linear(const std::vector<float>& x, const std::vector<float>& w, const std::vector<float>& b) {
-    const int64_t k = int64_t(x.size()), out = int64_t(b.size());
-    std::vector<float> y(static_cast<size_t>(out));
-    for (int64_t r = 0; r < out; ++r) y[size_t(r)] = dot(w.data() + r * k, x.data(), k) + b[size_t(r)];
-    return y;
-}
-
-// Abramowitz & Stegun 7.1.26 (|error| < 1.5e-7), the reference's erf.
-float erf_as(float x) {
-    const float s = x > 0.0f ? 1.0f : (x < 0.0f ? -1.0f : 0.0f);
-    const float a = std::fabs(x);
-    const float t = 1.0f / (1.0f + 0.3275911f * a);
-    const float poly = ((((1.061405429f * t - 1.453152027f) * t + 1.421413741f) * t - 0.284496736f) * t +
-                        0.254829592f) * t;
-    return s * (1.0f - poly * std::exp(-a * a));
-}
-
-float gelu_erf_host(float x) { return 0.5f * x * (1.0f + erf_as(x * 0.70710678118654752f)); }
-
-std::vector<float> softmax(const std::vector<float>& z) {
-    float m = -INFINITY;
-    for (float v : z) m = std::max(m, v);
-    std::vector<float> e(z.size());
-    float s = 0.0f;
-    for (size_t i = 0; i < z.size(); ++i) {
-        e[i] = std::exp(z[i] - m);
-        s += e[i];
-    }
-    for (float& v : e) v /= s;
-    return e;
 }
 
 DevBuf upload(const void* src, size_t n) {
@@ -222,7 +171,7 @@ std::vector<TensorSpec> LayaConfig::tensors() const {
     return v;
 }
 
-bool laya_host_tensor(const std::string& name) { return name.rfind("scorer.", 0) == 0 || name.rfind("act.", 0) == 0; }
+bool laya_scorer_tensor(const std::string& name) { return name.rfind("scorer.", 0) == 0 || name.rfind("act.", 0) == 0; }
 
 LayaWeights synth_laya(const LayaConfig& cfg, uint64_t seed, Dtype linear, Dtype embed) {
     cfg.validate();
@@ -246,7 +195,7 @@ LayaWeights synth_laya(const LayaConfig& cfg, uint64_t seed, Dtype linear, Dtype
         // saturate its softmax.
         const float scale = nm == "embed" ? 1.0f : (nm == "type_emb" ? 0.15f : 1.0f / std::sqrt(float(spec.shape[1])));
         for (int64_t i = 0; i < n; ++i) buf[size_t(i)] = r.next() * scale;
-        const Dtype dt = nm == "embed" ? embed : ((laya_host_tensor(nm) || nm == "type_emb") ? F16 : linear);
+        const Dtype dt = nm == "embed" ? embed : ((laya_scorer_tensor(nm) || nm == "type_emb") ? F16 : linear);
         switch (dt) {
             case F16: w.tensors[nm] = from_f32(spec.shape, buf.data()); break;
             case Q8: w.tensors[nm] = quantize_q8(spec.shape, buf.data()); break;
@@ -292,9 +241,22 @@ void LayaBuilder::push(const std::string& name, const QTensor& t) {
     if (t.dtype != F16 && int64_t(t.scales.size()) != n / BLOCK * 2) fail(E_INVALID, name + ": scale size mismatch");
     linears_.erase(name);
     vecs_.erase(name);
-    host_.erase(name);
-    if (laya_host_tensor(name)) {
-        host_[name] = to_f32(t);
+    if (laya_scorer_tensor(name)) {
+        // Read in f32 by the scorer's kernels; its first layer's product
+        // takes the stored weights, the act head's first layer transposed.
+        if (name == "scorer.l1") {
+            linears_[name] = upload_weight(t);
+            return;
+        }
+        std::vector<float> v = to_f32(t);
+        if (name == "act.l1") {
+            const int64_t rows = t.shape[0], cols = t.shape[1];
+            std::vector<float> tr(v.size());
+            for (int64_t r = 0; r < rows; ++r)
+                for (int64_t c = 0; c < cols; ++c) tr[size_t(c * rows + r)] = v[size_t(r * cols + c)];
+            v.swap(tr);
+        }
+        vecs_[name] = upload(v.data(), v.size() * 4);
         return;
     }
     if (t.shape.size() == 1 && t.dtype != F16) fail(E_INVALID, name + ": 1-D tensors must be f16");
@@ -314,7 +276,7 @@ void LayaBuilder::push(const std::string& name, const QTensor& t) {
 std::vector<std::string> LayaBuilder::missing() const {
     std::vector<std::string> v;
     for (const auto& kv : expected_)
-        if (!linears_.count(kv.first) && !vecs_.count(kv.first) && !host_.count(kv.first)) v.push_back(kv.first);
+        if (!linears_.count(kv.first) && !vecs_.count(kv.first)) v.push_back(kv.first);
     return v;
 }
 
@@ -376,7 +338,18 @@ std::unique_ptr<LayaEngine> LayaBuilder::finish(int64_t capacity, int64_t max_ro
         H.l2_b = vec(n("l2_b"));
         E.head_.push_back(std::move(H));
     }
-    E.host_ = std::move(host_);
+    E.scorer_.norm_w = vec("scorer.norm_w");
+    E.scorer_.norm_b = vec("scorer.norm_b");
+    E.scorer_.l1 = lin("scorer.l1");
+    E.scorer_.l1_b = vec("scorer.l1_b");
+    E.scorer_.l2 = vec("scorer.l2");
+    E.scorer_.l2_b = vec("scorer.l2_b");
+    if (c.act_out > 0) {
+        E.scorer_.act1_t = vec("act.l1");
+        E.scorer_.act1_b = vec("act.l1_b");
+        E.scorer_.act2 = vec("act.l2");
+        E.scorer_.act2_b = vec("act.l2_b");
+    }
 
     // RoPE (cos, sin) per position below max_len: inv_freq[i] =
     // theta^(-2i / 64) (rope_bi.wgsl:34).
@@ -394,9 +367,10 @@ std::unique_ptr<LayaEngine> LayaBuilder::finish(int64_t capacity, int64_t max_ro
     E.rope_global_ = table(c.theta_global);
 
     const int64_t cap = E.rows_cap_, d = c.d, tp = E.tpad_;
-    E.ids_ = DevBuf(size_t(cap) * 4);
-    E.qtypes_ = DevBuf(size_t(cap) * 4);
-    E.meta_ = DevBuf(size_t(cap) * 16, true);
+    // a pass's inputs: ids, question types, row metadata, rows to read back,
+    // marker rows, each sequence's first marker
+    E.h_in_bytes_ = size_t(cap) * (4 + 4 + 16) + size_t(3 * max_rows + 1) * 4 + 6 * 16;
+    E.in_ = DevBuf(E.h_in_bytes_, true);
     E.x_ = DevBuf(size_t(cap * d) * 4);
     E.a_ = DevBuf(size_t(cap * d) * 4);
     E.h16_ = DevBuf(size_t(cap * d) * 2);
@@ -408,13 +382,16 @@ std::unique_ptr<LayaEngine> LayaBuilder::finish(int64_t capacity, int64_t max_ro
     E.attn16_ = DevBuf(size_t(cap * d) * 2);
     E.act16_ = DevBuf(size_t(cap * std::max(c.ff, 4 * d)) * 2);
     E.rows_ = DevBuf(size_t(max_rows * d) * 4);
-    E.wanted_ = DevBuf(size_t(max_rows) * 4);
     E.attn_w_ = DevBuf(size_t(max_rows * d) * 2);
     E.x_w_ = DevBuf(size_t(max_rows * d) * 4);
     E.a_w_ = DevBuf(size_t(max_rows * d) * 4);
     E.h16_w_ = DevBuf(size_t(max_rows * d) * 2);
     E.act_w_ = DevBuf(size_t(max_rows * 4 * d) * 2);
-    E.h_in_bytes_ = size_t(cap) * (4 + 4 + 16) + size_t(max_rows) * 4;
+    // the scorer: normed marker rows, hidden units, scores, split rows
+    E.score_z_ = DevBuf(size_t(max_rows * d) * 4);
+    E.score_h_ = DevBuf(size_t(max_rows * d) * 4);
+    E.scores_ = DevBuf(size_t(max_rows) * 2 * 4);
+    E.score_split_ = DevBuf(size_t(split_rows_bytes(max_rows, d)));
     OMG_HIP(hipHostMalloc(&E.h_in_, E.h_in_bytes_, hipHostMallocDefault));
     E.h_out_bytes_ = size_t(max_rows * d) * 4;
     OMG_HIP(hipHostMalloc(&E.h_out_, E.h_out_bytes_, hipHostMallocDefault));
@@ -501,11 +478,30 @@ int64_t LayaEngine::pack(const LayaSeq* seqs, int64_t n) {
     if (total > capacity_)
         fail(E_CAPACITY, std::to_string(total) + " tokens exceed the engine capacity " + std::to_string(capacity_));
     sync();
+    // The inputs as one block, each part at its size for this pass (the
+    // loop below refuses a request before it could write past one).
+    int64_t rows = 0, want = 0;
+    for (int64_t i = 0; i < n; ++i) {
+        rows = (rows + 31) / 32 * 32 + seqs[i].n;
+        want += 1 + seqs[i].nmarkers;
+    }
+    rows = std::min(rows, rows_cap_);
+    want = std::min(want, max_rows_);
+    size_t bytes = 0;
+    auto part = [&](int64_t count, size_t size) {
+        const size_t o = bytes;
+        bytes += (size_t(count) * size + 15) / 16 * 16;
+        return o;
+    };
+    const size_t o_ids = part(rows, 4), o_qt = part(rows, 4), o_meta = part(rows, 16), o_wanted = part(want, 4),
+                 o_mrow = part(want, 4), o_first = part(std::min(n, max_rows_) + 1, 4);
     uint8_t* h = static_cast<uint8_t*>(h_in_);
-    uint32_t* ids = reinterpret_cast<uint32_t*>(h);
-    uint32_t* qt = ids + rows_cap_;
-    int32_t* meta = reinterpret_cast<int32_t*>(qt + rows_cap_);
-    int32_t* wanted = meta + 4 * rows_cap_;
+    uint32_t* ids = reinterpret_cast<uint32_t*>(h + o_ids);
+    uint32_t* qt = reinterpret_cast<uint32_t*>(h + o_qt);
+    int32_t* meta = reinterpret_cast<int32_t*>(h + o_meta);
+    int32_t* wanted = reinterpret_cast<int32_t*>(h + o_wanted);
+    int32_t* mrow = reinterpret_cast<int32_t*>(h + o_mrow);
+    int32_t* first = reinterpret_cast<int32_t*>(h + o_first);
     int64_t at = 0, nw = 0;
     for (int64_t si = 0; si < n; ++si) {
         const LayaSeq& s = seqs[si];
@@ -540,18 +536,25 @@ int64_t LayaEngine::pack(const LayaSeq* seqs, int64_t n) {
         }
         if (nw + 1 + s.nmarkers > max_rows_)
             fail(E_CAPACITY, "more rows requested than the engine reads back (" + std::to_string(max_rows_) + ")");
+        first[si] = int32_t(nw - si);  // markers so far
         wanted[nw++] = int32_t(start);
         for (int64_t j = 0; j < s.nmarkers; ++j) {
             if (int64_t(s.markers[j]) >= s.n)
                 fail(E_INVALID, "sequence " + std::to_string(si) + ": marker " + std::to_string(s.markers[j]) +
                                     " past its " + std::to_string(s.n) + " tokens");
+            mrow[nw - si - 1] = int32_t(nw);
             wanted[nw++] = int32_t(start + s.markers[j]);
         }
     }
-    OMG_HIP(hipMemcpyAsync(ids_.p, ids, size_t(at) * 4, hipMemcpyHostToDevice, stream_));
-    OMG_HIP(hipMemcpyAsync(qtypes_.p, qt, size_t(at) * 4, hipMemcpyHostToDevice, stream_));
-    OMG_HIP(hipMemcpyAsync(meta_.p, meta, size_t(at) * 16, hipMemcpyHostToDevice, stream_));
-    OMG_HIP(hipMemcpyAsync(wanted_.p, wanted, size_t(nw) * 4, hipMemcpyHostToDevice, stream_));
+    first[n] = int32_t(nw - n);
+    OMG_HIP(hipMemcpyAsync(in_.p, h, bytes, hipMemcpyHostToDevice, stream_));
+    const uint8_t* dv = in_.as<uint8_t>();
+    d_ids_ = reinterpret_cast<const uint32_t*>(dv + o_ids);
+    d_qtypes_ = reinterpret_cast<const uint32_t*>(dv + o_qt);
+    d_meta_ = reinterpret_cast<const int32_t*>(dv + o_meta);
+    d_wanted_ = reinterpret_cast<const int32_t*>(dv + o_wanted);
+    d_mrow_ = reinterpret_cast<const int32_t*>(dv + o_mrow);
+    d_first_ = reinterpret_cast<const int32_t*>(dv + o_first);
     t_ = at;
     nrows_ = nw;
     return total;
@@ -571,7 +574,7 @@ void LayaEngine::forward() {
     half_t* h16 = h16_.as<half_t>();
     half_t* attn = attn16_.as<half_t>();
     half_t* act = act16_.as<half_t>();
-    const int32_t* meta = meta_.as<int32_t>();
+    const int32_t* meta = d_meta_;
     QkvHeads qh{};
     qh.meta = meta;
     qh.dq = d;
@@ -579,7 +582,7 @@ void LayaEngine::forward() {
     qh.q16 = q16_.as<half_t>();
     qh.k16 = k16_.as<half_t>();
     qh.vt = vt_.as<half_t>();
-    step("embed_ln", [&] { launch_embed_ln(stream_, embed_.w, ids_.as<uint32_t>(), t, embed_norm_.as<float>(), c.eps, x, h16); });
+    step("embed_ln", [&] { launch_embed_ln(stream_, embed_.w, d_ids_, t, embed_norm_.as<float>(), c.eps, x, h16); });
     const Head* h0 = head_.empty() ? nullptr : &head_[0];
     for (size_t l = 0; l < enc_.size(); ++l) {
         const Enc& L = enc_[l];
@@ -601,7 +604,7 @@ void LayaEngine::forward() {
         } else {
             step("final_norm", [&] {
                 launch_add_ln_final(stream_, x, a, final_norm_.as<float>(), c.type_emb ? type_emb_.as<float>() : nullptr,
-                                    qtypes_.as<uint32_t>(), h0 ? h0->norm1_w.as<float>() : nullptr,
+                                    d_qtypes_, h0 ? h0->norm1_w.as<float>() : nullptr,
                                     h0 ? h0->norm1_b.as<float>() : nullptr, c.eps, t, d, h16);
             });
         }
@@ -626,7 +629,7 @@ void LayaEngine::forward() {
             float* pw = a_w_.as<float>();
             half_t* hw = h16_w_.as<half_t>();
             half_t* actw = act_w_.as<half_t>();
-            step("gather_out", [&] { launch_gather_out(stream_, attn, d, x, d, wanted_.as<int32_t>(), 0, n, aw, xw); });
+            step("gather_out", [&] { launch_gather_out(stream_, attn, d, x, d, d_wanted_, 0, n, aw, xw); });
             step("mm_out_out", [&] { launch_gemm(stream_, aw, d, H.out_proj.w, pw, d, n); });
             step("add_out_norm2_out", [&] {
                 launch_add_ln(stream_, xw, pw, H.out_proj_b.as<float>(), H.norm2_w.as<float>(), H.norm2_b.as<float>(),
@@ -652,13 +655,13 @@ void LayaEngine::forward() {
             });
         } else {
             step("rows", [&] {
-                launch_gather_rows(stream_, x, a, H.l2_b.as<float>(), wanted_.as<int32_t>(), nrows_, d,
+                launch_gather_rows(stream_, x, a, H.l2_b.as<float>(), d_wanted_, nrows_, d,
                                    rows_.as<float>());
             });
         }
     }
     if (head_.empty())
-        step("rows", [&] { launch_gather_rows(stream_, x, nullptr, nullptr, wanted_.as<int32_t>(), nrows_, d, rows_.as<float>()); });
+        step("rows", [&] { launch_gather_rows(stream_, x, nullptr, nullptr, d_wanted_, nrows_, d, rows_.as<float>()); });
 }
 
 void LayaEngine::prepare(const LayaSeq* seqs, int64_t n) { pack(seqs, n); }
@@ -684,64 +687,55 @@ void LayaEngine::hidden(const LayaSeq* seqs, int64_t n, float* out, int64_t out_
     std::memcpy(out, h_out_, size_t(nrows_ * cfg_.d) * 4);
 }
 
-void LayaEngine::score(const float* rows, int64_t nmarkers, float* logits, float* act) const {
+// The scorer on the read-out rows of the pass just queued: n sequences'
+// act probabilities after their nrows_ - n marker logits in scores_.
+void LayaEngine::score(int64_t n) {
     const LayaConfig& c = cfg_;
-    const int64_t d = c.d;
-    const auto& nw = host_.at("scorer.norm_w");
-    const auto& nb = host_.at("scorer.norm_b");
-    const auto& l1 = host_.at("scorer.l1");
-    const auto& l1b = host_.at("scorer.l1_b");
-    const auto& l2 = host_.at("scorer.l2");
-    const float l2b = host_.at("scorer.l2_b")[0];
-    std::vector<float> lg(static_cast<size_t>(nmarkers));
-    for (int64_t j = 0; j < nmarkers; ++j) {
-        std::vector<float> z = layer_norm(rows + (1 + j) * d, d, nw.data(), nb.data(), c.eps);
-        z = linear(z, l1, l1b);
-        for (float& v : z) v = gelu_erf_host(v);
-        lg[size_t(j)] = dot(z.data(), l2.data(), d) + l2b;
-        logits[j] = lg[size_t(j)];
+    const int64_t d = c.d, nm = nrows_ - n;
+    const Scorer& S = scorer_;
+    if (nm > 0) {
+        step("score_norm", [&] {
+            launch_score_norm(stream_, rows_.as<float>(), d_mrow_, nm, d, S.norm_w.as<float>(), S.norm_b.as<float>(),
+                              c.eps, score_z_.as<float>());
+        });
+        LogitsOut o;
+        o.out = score_h_.as<float>();
+        step("score_l1", [&] {
+            launch_logits(stream_, S.l1.w, score_z_.as<float>(), nm, nullptr, d, 0.0f, o, score_split_.p);
+        });
     }
-    if (c.act_out == 0) {
-        *act = NAN;
-        return;
-    }
-    // Confidence features of the untempered softmax, one-option questions
-    // padded to two slots (laya.rs:1464-1480).
-    const int64_t k = std::max<int64_t>(nmarkers, 2);
-    std::vector<float> padded = lg;
-    padded.resize(size_t(k), -1e4f);
-    const std::vector<float> p = softmax(padded);
-    float ent = 0.0f;
-    for (float v : p) ent += v * std::log(std::max(v, 1e-9f));
-    const float entropy = -ent / std::log(float(k));
-    std::vector<float> sorted = p;
-    std::sort(sorted.begin(), sorted.end());
-    const float top1 = sorted[size_t(k - 1)], top2 = sorted[size_t(k - 2)];
-    std::vector<float> pooled(rows, rows + d);
-    pooled.push_back(top1);
-    pooled.push_back(top1 - top2);
-    pooled.push_back(entropy);
-    pooled.push_back(float(k) / 255.0f);
-    std::vector<float> h = linear(pooled, host_.at("act.l1"), host_.at("act.l1_b"));
-    for (float& v : h) v = gelu_erf_host(v);
-    *act = softmax(linear(h, host_.at("act.l2"), host_.at("act.l2_b")))[0];
+    ScoreArgs a{};
+    a.rows = rows_.as<float>();
+    a.h = score_h_.as<float>();
+    a.first = d_first_;
+    a.d = d;
+    a.l1_b = S.l1_b.as<float>();
+    a.l2 = S.l2.as<float>();
+    a.l2_b = S.l2_b.as<float>();
+    a.w1t = S.act1_t.as<float>();
+    a.b1 = S.act1_b.as<float>();
+    a.w2 = S.act2.as<float>();
+    a.b2 = S.act2_b.as<float>();
+    a.act_hidden = c.act_hidden;
+    a.act_out = c.act_out;
+    a.logits = scores_.as<float>();
+    a.act = scores_.as<float>() + nm;
+    step("score", [&] { launch_score(stream_, a, n); });
 }
 
 void LayaEngine::evaluate(const LayaSeq* seqs, int64_t n, float* logits, int64_t nlogits, float* act, int64_t nact) {
-    int64_t want = 0, rows = 0;
-    for (int64_t i = 0; i < n; ++i) {
-        want += seqs[i].nmarkers;
-        rows += 1 + seqs[i].nmarkers;
-    }
+    int64_t want = 0;
+    for (int64_t i = 0; i < n; ++i) want += seqs[i].nmarkers;
     if (nlogits < want || nact < n) fail(E_INVALID, "output buffer too small");
-    std::vector<float> h(size_t(rows * cfg_.d));
-    hidden(seqs, n, h.data(), int64_t(h.size()));
-    int64_t r = 0, j = 0;
-    for (int64_t i = 0; i < n; ++i) {
-        score(h.data() + r * cfg_.d, seqs[i].nmarkers, logits + j, act + i);
-        r += 1 + seqs[i].nmarkers;
-        j += seqs[i].nmarkers;
-    }
+    pack(seqs, n);
+    forward();
+    score(n);
+    const int64_t got = want + (cfg_.act_out > 0 ? n : 0);
+    OMG_HIP(hipMemcpyAsync(h_out_, scores_.p, size_t(got) * 4, hipMemcpyDeviceToHost, stream_));
+    sync();
+    const float* h = static_cast<const float*>(h_out_);
+    if (want) std::memcpy(logits, h, size_t(want) * 4);
+    for (int64_t i = 0; i < n; ++i) act[i] = cfg_.act_out > 0 ? h[want + i] : NAN;
 }
 
 void LayaEngine::warmup() {

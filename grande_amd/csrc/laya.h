@@ -46,7 +46,7 @@ struct LayaConfig {
     float temperature_for(int qtype, int64_t k) const;  // laya.rs:234-248
 };
 
-bool laya_host_tensor(const std::string& name);  // laya.rs:326-328
+bool laya_scorer_tensor(const std::string& name);  // laya.rs:326-328
 
 // A host checkpoint of the encoder path (laya.rs:331-464).
 struct LayaWeights {
@@ -93,8 +93,7 @@ class LayaBuilder {
     LayaConfig cfg_;
     std::map<std::string, std::vector<int64_t>> expected_;
     std::map<std::string, DevTensor> linears_;
-    std::map<std::string, DevBuf> vecs_;                 // f32 on the device
-    std::map<std::string, std::vector<float>> host_;     // scorer / act head
+    std::map<std::string, DevBuf> vecs_;  // f32 on the device
 };
 
 class LayaEngine {
@@ -129,7 +128,7 @@ class LayaEngine {
     LayaEngine() = default;
     int64_t pack(const LayaSeq* seqs, int64_t n);  // returns the token count; fills wanted
     void forward();
-    void score(const float* rows, int64_t nmarkers, float* logits, float* act) const;
+    void score(int64_t n);
     template <class F>
     void step(const char* name, F&& f);
 
@@ -150,10 +149,18 @@ class LayaEngine {
     };
     std::vector<Enc> enc_;
     std::vector<Head> head_;
-    std::map<std::string, std::vector<float>> host_;
+    struct Scorer {
+        DevTensor l1;
+        DevBuf norm_w, norm_b, l1_b, l2, l2_b, act1_t, act1_b, act2, act2_b;
+    };
+    Scorer scorer_;
     DevBuf rope_local_, rope_global_;
     // workspace
-    DevBuf ids_, qtypes_, meta_, x_, a_, h16_, q16_, k16_, vt_, attn16_, act16_, rows_, wanted_;
+    DevBuf in_, x_, a_, h16_, q16_, k16_, vt_, attn16_, act16_, rows_;
+    // a pass's inputs inside in_
+    const uint32_t *d_ids_ = nullptr, *d_qtypes_ = nullptr;
+    const int32_t *d_meta_ = nullptr, *d_wanted_ = nullptr, *d_mrow_ = nullptr, *d_first_ = nullptr;
+    DevBuf score_z_, score_h_, scores_, score_split_;
     // The last head layer on the read-out rows: [max_rows] rows of the
     // attention output, stream, product, normed stream and activations.
     bool full_last_layer_ = false;

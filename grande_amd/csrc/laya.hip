@@ -396,6 +396,149 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const float* __restric
     }
 }
 
+// ------------------------------------------------------------- the scorer
+
+// laya.rs:1442-1463, first half: z[j] = LayerNorm(rows[mrow[j]]; w, b), f32,
+// one wave per marker row.
+template <int NV>
+__global__ __launch_bounds__(256) void score_norm_kernel(const float* __restrict__ rows, const int32_t* __restrict__ mrow,
+                                                         int64_t n, int64_t d, const float* __restrict__ w,
+                                                         const float* __restrict__ b, float eps,
+                                                         float* __restrict__ z) {
+    const int lane = int(threadIdx.x) % WAVE;
+    const int64_t j = int64_t(blockIdx.x) * 4 + threadIdx.x / WAVE;
+    if (j >= n) return;
+    const float* row = rows + int64_t(mrow[j]) * d;
+    float4 v[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        const int64_t c = (k * WAVE + lane) * 4;
+        v[k] = c < d ? *reinterpret_cast<const float4*>(row + c) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    float mean, inv;
+    ln_stats<NV>(v, d, lane, eps, mean, inv);
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        const int64_t c = (k * WAVE + lane) * 4;
+        if (c < d) *reinterpret_cast<float4*>(z + j * d + c) = ln_apply(v[k], mean, inv, w, b, c);
+    }
+}
+
+// Abramowitz & Stegun 7.1.26 (|error| < 1.5e-7), the reference scorer's erf.
+__device__ inline float score_gelu(float x) {
+    const float y = x * 0.70710678118654752f;
+    const float a = fabsf(y);
+    const float t = 1.0f / (1.0f + 0.3275911f * a);
+    const float poly = ((((1.061405429f * t - 1.453152027f) * t + 1.421413741f) * t - 0.284496736f) * t +
+                        0.254829592f) * t;
+    const float e = 1.0f - poly * expf(-a * a);
+    return 0.5f * x * (1.0f + (y < 0.0f ? -e : e));
+}
+
+// laya.rs:1442-1485, the rest, one workgroup per sequence: each marker's
+// logit from its hidden units (a wave per marker), then the act head on the
+// [CLS] row and the confidence features of the untempered softmax
+// (one-option questions padded to two slots with -1e4).  The act head's
+// first layer comes transposed [d + 4][hidden], so that a workgroup's reads
+// are whole rows; four threads share a unit's sum.
+constexpr int SC_T = 1024, SC_W = SC_T / WAVE;
+constexpr int SC_HID = 256;  // the act head's hidden units
+constexpr int SC_D = 2048;   // widest row
+
+__global__ __launch_bounds__(SC_T) void score_kernel(ScoreArgs a) {
+    __shared__ float pooled[SC_D + 4];
+    __shared__ float part[SC_T / SC_HID][SC_HID];
+    __shared__ __attribute__((aligned(16))) float hid[SC_HID];
+    __shared__ float stat[SC_W][2], first_out;
+    const int tid = int(threadIdx.x), wave = tid / WAVE, lane = tid % WAVE;
+    const int64_t s = blockIdx.x, d = a.d;
+    const int64_t j0 = a.first[s], nm = a.first[s + 1] - j0;
+    for (int64_t j = j0 + wave; j < j0 + nm; j += SC_W) {
+        float acc = 0.0f;
+        for (int64_t c = lane * 4; c < d; c += WAVE * 4) {
+            const float4 h = *reinterpret_cast<const float4*>(a.h + j * d + c);
+            const float4 b = *reinterpret_cast<const float4*>(a.l1_b + c);
+            const float4 w = *reinterpret_cast<const float4*>(a.l2 + c);
+            acc += (score_gelu(h.x + b.x) * w.x + score_gelu(h.y + b.y) * w.y) +
+                   (score_gelu(h.z + b.z) * w.z + score_gelu(h.w + b.w) * w.w);
+        }
+        acc = wave_sum(acc);
+        if (lane == 0) a.logits[j] = acc + a.l2_b[0];
+    }
+    if (a.act_out == 0) return;
+    // (row of the sequence's [CLS]: every earlier sequence has one too)
+    for (int64_t c = tid; c < d; c += SC_T) pooled[c] = a.rows[(j0 + s) * d + c];
+    __syncthreads();  // the workgroup's logits are written
+    if (wave == 0) {
+        const int64_t k = nm > 2 ? nm : 2;
+        auto logit = [&](int64_t j) { return j < nm ? a.logits[j0 + j] : -1e4f; };
+        // The two largest: per lane, then across lanes.
+        float t1 = -INFINITY, t2 = -INFINITY;
+        auto add = [&](float v) {
+            t2 = fmaxf(t2, fminf(t1, v));
+            t1 = fmaxf(t1, v);
+        };
+        for (int64_t j = lane; j < k; j += WAVE) add(logit(j));
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const float u1 = __shfl_xor(t1, o, WAVE), u2 = __shfl_xor(t2, o, WAVE);
+            t2 = fmaxf(fmaxf(t2, u2), fminf(t1, u1));
+            t1 = fmaxf(t1, u1);
+        }
+        float sum = 0.0f;
+        for (int64_t j = lane; j < k; j += WAVE) sum += expf(logit(j) - t1);
+        sum = wave_sum(sum);
+        float ent = 0.0f;
+        for (int64_t j = lane; j < k; j += WAVE) {
+            const float p = expf(logit(j) - t1) / sum;
+            ent += p * logf(fmaxf(p, 1e-9f));
+        }
+        ent = wave_sum(ent);
+        if (lane == 0) {
+            const float p1 = 1.0f / sum, p2 = expf(t2 - t1) / sum;
+            pooled[d] = p1;
+            pooled[d + 1] = p1 - p2;
+            pooled[d + 2] = -ent / logf(float(k));
+            pooled[d + 3] = float(k) / 255.0f;
+        }
+    }
+    __syncthreads();
+    {
+        const int o = tid % SC_HID, p = tid / SC_HID;
+        const int n = int(d) + 4, step = (n + SC_T / SC_HID - 1) / (SC_T / SC_HID);
+        const int hi = min(n, (p + 1) * step);
+        float acc = 0.0f;
+#pragma unroll 8
+        for (int i = p * step; i < hi; ++i) acc += a.w1t[int64_t(i) * SC_HID + o] * pooled[i];
+        part[p][o] = acc;
+    }
+    __syncthreads();
+    if (tid < SC_HID) hid[tid] = score_gelu(((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid] + a.b1[tid]);
+    __syncthreads();
+    // The outputs, a wave each, with a running softmax per wave.
+    float m = -INFINITY, sum = 0.0f;
+    for (int64_t q = wave; q < a.act_out; q += SC_W) {
+        const float4 w = *reinterpret_cast<const float4*>(a.w2 + q * SC_HID + lane * 4);
+        const float4 h = *reinterpret_cast<const float4*>(hid + lane * 4);
+        const float v = wave_sum((w.x * h.x + w.y * h.y) + (w.z * h.z + w.w * h.w)) + a.b2[q];
+        if (q == 0 && lane == 0) first_out = v;
+        const float mn = fmaxf(m, v);
+        sum = sum * expf(m - mn) + expf(v - mn);
+        m = mn;
+    }
+    if (lane == 0) {
+        stat[wave][0] = m;
+        stat[wave][1] = sum;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        float M = -INFINITY, S = 0.0f;
+        for (int w = 0; w < SC_W; ++w) M = fmaxf(M, stat[w][0]);
+        for (int w = 0; w < SC_W; ++w) S += stat[w][0] == -INFINITY ? 0.0f : stat[w][1] * expf(stat[w][0] - M);
+        a.act[s] = expf(first_out - M) / S;
+    }
+}
+
 int row_nv(int64_t d, const char* what) {
     if (d <= 0 || d % 4 != 0 || d > 2048) fail(E_INVALID, std::string(what) + ": row width must be 4..2048, a multiple of 4");
     return int((d / 4 + WAVE - 1) / WAVE);
@@ -469,6 +612,23 @@ void launch_gather_rows(hipStream_t s, const float* x, const float* a, const flo
     if (a && !bias) fail(E_INVALID, "gather_rows: bias required with a");
     if (n <= 0) return;
     gather_rows_kernel<<<dim3(unsigned((n + 3) / 4)), dim3(256), 0, s>>>(x, a, bias, rows, n, d, out);
+    OMG_HIP(hipGetLastError());
+}
+
+void launch_score_norm(hipStream_t s, const float* rows, const int32_t* mrow, int64_t n, int64_t d, const float* w,
+                       const float* b, float eps, float* z) {
+    const int nv = row_nv(d, "score_norm");
+    if (n <= 0) return;
+    const dim3 grid(unsigned((n + 3) / 4)), block(256);
+    OMG_NV_SWITCH(nv, (score_norm_kernel<NV><<<grid, block, 0, s>>>(rows, mrow, n, d, w, b, eps, z)));
+    OMG_HIP(hipGetLastError());
+}
+
+void launch_score(hipStream_t s, const ScoreArgs& a, int64_t n) {
+    if (a.d <= 0 || a.d % 4 != 0 || a.d > SC_D) fail(E_INVALID, "score: row width");
+    if (a.act_out > 0 && a.act_hidden != SC_HID) fail(E_INVALID, "score: act head of 256 hidden units");
+    if (n <= 0) return;
+    score_kernel<<<dim3(unsigned(n)), dim3(SC_T), 0, s>>>(a);
     OMG_HIP(hipGetLastError());
 }
 

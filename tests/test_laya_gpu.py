@@ -372,3 +372,47 @@ def test_open_exported_directory(tmp_path):
     seqs = random_seqs(np.random.default_rng(6), 300, 3, 20, 90)
     for x, y in zip(a.hidden(seqs), b.hidden(seqs)):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("counts,act,dtype", [([1], {"ask": 1.0}, g.Q8), ([0, 1, 2, 3], {"ask": 1.0, "wait": 0.5}, g.Q8),
+                                              ([33, 1, 70, 2], {str(i): 1.0 for i in range(19)}, g.Q4),
+                                              ([5, 0, 31], None, g.F16)])
+def test_scorer_on_device_matches_float64(counts, act, dtype):
+    """The scorer and the act head (laya.rs:1442-1485) on the engine's own
+    rows against numpy float64: marker counts around the 32-row tile, none,
+    one (padded to two slots), more than a wave of options, more outputs
+    than waves.  f32 sums of up to d + 4 terms with |x w| summing to a few
+    units: 1e-5."""
+    from math import erf
+    cfg = tiny(act_costs=act, max_len=512)
+    w = ly.synth_weights(cfg, 31, dtype, dtype)
+    eng = ly.LayaEngine.new(w, 2048, 256)
+    T = {t.name: t.to_f32().astype(np.float64) for t in w.tensors() if t.name.startswith(("scorer.", "act."))}
+    rng = np.random.default_rng(sum(counts))
+    seqs = [ly.Sequence(rng.integers(5, 300, max(8, k + 2)).tolist(), list(range(1, 1 + k)), i % 3)
+            for i, k in enumerate(counts)]
+    outs, rows = eng.evaluate(seqs), eng.hidden(seqs)
+
+    def gelu(x):
+        return 0.5 * x * (1.0 + np.vectorize(erf)(x / np.sqrt(2.0)))
+
+    for k, o, r in zip(counts, outs, rows):
+        r = r.astype(np.float64)
+        z = r[1:]
+        z = (z - z.mean(1, keepdims=True)) / np.sqrt(z.var(1, keepdims=True) + 1e-5)
+        z = z * T["scorer.norm_w"] + T["scorer.norm_b"]
+        z = gelu(z @ T["scorer.l1"].T + T["scorer.l1_b"]) @ T["scorer.l2"][0] + T["scorer.l2_b"][0] if k else np.zeros(0)
+        assert o.logits.shape == (k,) and np.max(np.abs(o.logits - z), initial=0.0) < 1e-5
+        if act is None:
+            assert o.act_probability is None
+            continue
+        p = np.concatenate([z, np.full(max(0, 2 - k), -1e4)])
+        p = np.exp(p - p.max())
+        p /= p.sum()
+        top = np.sort(p)[::-1]
+        ent = -(p * np.log(np.maximum(p, 1e-9))).sum() / np.log(len(p))
+        h = np.concatenate([r[0], [top[0], top[0] - top[1], ent, len(p) / 255.0]])
+        a = gelu(T["act.l1"] @ h + T["act.l1_b"])
+        a = T["act.l2"] @ a + T["act.l2_b"]
+        a = np.exp(a - a.max())
+        assert abs(o.act_probability - a[0] / a.sum()) < 1e-5
