@@ -38,6 +38,7 @@
 // past M or N read as zero in hardware; in the K tail (K % 64 == 32) the X
 // lanes and weight lanes past K are sent out of range by their lane offset
 // (a zero activation times a zero weight).
+#include <climits>
 #include <string>
 #include <utility>
 
@@ -136,348 +137,6 @@ __device__ inline float gelu_tanh(float x) {
     return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
-template <int QUANT, int MI, int NJ, int EPI, int NS, int NW_ = 4, int WM_ = 1>
-struct Cfg {
-    static constexpr bool GATED = EPI == EPI_GELU_TANH || EPI == EPI_GELU_ERF;
-    static constexpr int NW = NW_, T = NW * WAVE;
-    static constexpr int WM = WM_, WN = NW / WM;       // waves along M and along N
-    static constexpr int BM = 16 * MI * WM;
-    static constexpr int WR = 16 * NJ;                 // weight rows per wave
-    static constexpr int BNW = WN * WR;                // weight rows per tile
-    static constexpr int BN = GATED ? BNW / 2 : BNW;   // output columns per tile
-    static constexpr int X_CH = BM * 8, X_I = (X_CH + T - 1) / T;  // padded lanes go out of range
-    static constexpr int W_CPR = QUANT == Q4_DT ? 2 : (QUANT == Q8_DT ? 4 : 8);
-    static constexpr int W_CH = BNW * W_CPR, W_I = (W_CH + T - 1) / T;
-    static constexpr int S_I = QUANT == F16_DT ? 0 : (BNW + T - 1) / T;
-    static constexpr int C = X_I + W_I + S_I;  // DMA instructions per wave per stage
-    static constexpr int X_BYTES = X_I * T * 16, W_BYTES = W_I * T * 16, S_BYTES = S_I * T * 4;
-    static constexpr int STAGE = X_BYTES + W_BYTES + S_BYTES;
-    static constexpr int LDS = NS * STAGE;
-    static_assert(LDS <= 160 * 1024, "ring larger than the LDS");
-    static_assert(!GATED || NJ % 2 == 0, "gated tiles pair gate and up row blocks");
-    static_assert(BN % 64 == 0 || !GATED, "a scale DMA instruction must stay in one matrix");
-    static_assert(NS >= 2, "ring needs >= 2 slots");
-    static_assert(NW % WM == 0, "waves split evenly over M");
-    static_assert(C <= 63, "vmcnt range");
-    static_assert(EPI != EPI_QKV || WR == 64, "the Q/K/V epilogue gives each wave one 64-wide head");
-};
-
-template <int QUANT, int MI, int NJ, int EPI, int NS, int NW_, int WM_>
-__global__ __launch_bounds__(NW_ * WAVE) void gemm_kernel(GemmArgs g) {
-    using P = Cfg<QUANT, MI, NJ, EPI, NS, NW_, WM_>;
-    constexpr bool GATED = P::GATED;
-    constexpr int NW = P::NW, BM = P::BM, BN = P::BN, WR = P::WR;
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const int tid = int(threadIdx.x), lane = tid % WAVE;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-    // The wave's place in the tile: activation row blocks wm * MI .. + MI,
-    // weight rows of block column wn.
-    const int wn = wave % P::WN, wm = wave / P::WN;
-
-    // Workgroups are dispatched round-robin over the 8 XCDs (each with its
-    // own L2): workgroup b runs on XCD b % 8.  Give each XCD a contiguous run
-    // of tiles, row-tile major, so the activation rows it reads stay in its
-    // L2 while it sweeps the (small) weight matrix.
-    const int64_t N = g.w0.rows, K = g.w0.cols, KB = K / 32, M = g.m;
-    const int ntn = int((N + BN - 1) / BN);
-    const int ntiles = ntn * int((M + BM - 1) / BM);
-    const int per_xcd = int(gridDim.x) / 8;
-    const int tile = (int(blockIdx.x) % 8) * per_xcd + int(blockIdx.x) / 8;
-    if (tile >= ntiles) return;
-    const int64_t n0 = int64_t(tile % ntn) * BN, m0 = int64_t(tile / ntn) * BM;
-    const int kbeg = int(blockIdx.y) * int(K / g.ksplit);  // this split's K range (multiples of G_BK)
-    const int nk = int((K / g.ksplit + G_BK - 1) / G_BK);
-    const int K32 = int(K);
-    const int64_t rows_m = M - m0 < BM ? M - m0 : BM;
-    const int64_t rows_n = N - n0 < BN ? N - n0 : BN;
-
-    const int64_t wrow = QUANT == Q4_DT ? KB * 16 : (QUANT == Q8_DT ? K : 2 * K);
-    const uint8_t* const wbase0 = static_cast<const uint8_t*>(g.w0.data) + n0 * wrow;
-    const uint8_t* const wbase1 = static_cast<const uint8_t*>(g.w1.data) + n0 * wrow;
-    const uint16_t* const sbase0 = g.w0.scales ? g.w0.scales + n0 * g.w0.sld : nullptr;
-    const uint16_t* const sbase1 = g.w1.scales ? g.w1.scales + n0 * g.w1.sld : nullptr;
-    const int64_t sbytes = g.w0.scales ? rows_n * g.w0.sld * 2 : 0;
-
-    uint32_t xoff[P::X_I];
-    int xcol[P::X_I];
-#pragma unroll
-    for (int i = 0; i < P::X_I; ++i) {
-        const int slot = (i * NW + wave) * WAVE + lane;
-        const int r = slot / 8, lc = (slot % 8) ^ swz(r);
-        xcol[i] = lc * 8;
-        xoff[i] = slot < P::X_CH ? uint32_t((r * g.ldx + lc * 8) * 2) : OOB;
-    }
-    uint32_t woff[P::W_I], wtail[P::W_I];  // wtail: the lane's offset in the K-tail stage
-    bool wup[P::W_I];
-#pragma unroll
-    for (int i = 0; i < P::W_I; ++i) {
-        const int blk = i * NW + wave;
-        const int slot = blk * WAVE + lane;
-        const int rw = slot / P::W_CPR, c = slot % P::W_CPR;
-        wup[i] = GATED && blk * WAVE / P::W_CPR >= BN;
-        const int n = GATED && rw >= BN ? rw - BN : rw;
-        uint32_t o;
-        bool past;  // chunk past K when only the stage's first 32 k exist
-        if constexpr (QUANT == Q4_DT) {
-            o = uint32_t((n * KB + c) * 16);
-            past = c >= 1;
-        } else if constexpr (QUANT == Q8_DT) {
-            o = uint32_t(n * K + c * 16);
-            past = c >= 2;
-        } else {
-            const int lc = c ^ swz(rw);
-            o = uint32_t((n * K + lc * 8) * 2);
-            past = lc >= 4;
-        }
-        woff[i] = slot < P::W_CH ? o : OOB;
-        wtail[i] = slot < P::W_CH && !past ? o : OOB;
-    }
-    uint32_t soff[P::S_I > 0 ? P::S_I : 1];
-    bool sup[P::S_I > 0 ? P::S_I : 1];
-#pragma unroll
-    for (int i = 0; i < P::S_I; ++i) {
-        const int rw = (i * NW + wave) * WAVE + lane;  // one scale dword per weight row
-        sup[i] = GATED && (i * NW + wave) * WAVE >= BN;
-        const int n = GATED && rw >= BN ? rw - BN : rw;
-        soff[i] = rw < P::BNW ? uint32_t(n * g.w0.sld * 2) : OOB;
-    }
-
-    // Issue stage s's DMA into its ring slot.  The stage's K offset rides in
-    // the scalar offset, so the lane offsets stay fixed; only the K-tail
-    // stage (K % 64 == 32) masks X lanes per lane.  Stages past the end
-    // repeat the last one (in range, never consumed), so every wave always
-    // issues P::C instructions per stage and the resources do not change.
-    auto slot_base = [&](int s) { return smem + (unsigned(s) % unsigned(NS)) * P::STAGE; };
-    const int last = nk - 1;
-    const int64_t xbytes = rows_m * g.ldx * 2;
-    const bool ktail = (K32 & (G_BK - 1)) != 0;
-    auto issue = [&](int s) {
-        uint8_t* base = slot_base(s);
-        const int k0 = __builtin_amdgcn_readfirstlane(kbeg + (s < last ? s : last) * G_BK);
-        // (Range checks cover the lane offset only: a row's offset plus the
-        // stage offset stays inside the row, and rows past M are out of
-        // range by their lane offset.  Each resource is a named value built
-        // at its use: passed inline, or held across branches, it is not
-        // accepted by the host-side compile of this kernel.)
-        const bool tail = ktail && k0 + G_BK > K32;
-#pragma unroll
-        for (int i = 0; i < P::X_I; ++i) {
-            const uint32_t o = tail && xcol[i] >= K32 - k0 ? OOB : xoff[i];
-            const __amdgpu_buffer_rsrc_t r = rsrc(g.x + m0 * g.ldx, xbytes);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(base + (i * NW + wave) * WAVE * 16), 16, o,
-                                                     k0 * 2, 0, 0);
-        }
-        // (So in the K-tail stage the weight lanes past K are masked by
-        // offset as well.)
-        const int wstep = QUANT == Q4_DT ? k0 / 2 : (QUANT == Q8_DT ? k0 : k0 * 2);
-#pragma unroll
-        for (int i = 0; i < P::W_I; ++i) {
-            const uint32_t o = tail ? wtail[i] : woff[i];
-            const __amdgpu_buffer_rsrc_t r = rsrc(wup[i] ? wbase1 : wbase0, rows_n * wrow);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(base + P::X_BYTES + (i * NW + wave) * WAVE * 16),
-                                                     16, o, wstep, 0, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < P::S_I; ++i) {
-            const __amdgpu_buffer_rsrc_t r = rsrc(sup[i] ? sbase1 : sbase0, sbytes);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                r, (lds_ptr_t)(base + P::X_BYTES + P::W_BYTES + (i * NW + wave) * WAVE * 4), 4, soff[i], k0 / 16, 0, 0);
-        }
-    };
-
-    // Tile-local weight row of this wave's row block j.
-    auto wrow_of = [&](int j) {
-        if constexpr (GATED)
-            return j < NJ / 2 ? wn * (WR / 2) + 16 * j : BN + wn * (WR / 2) + 16 * (j - NJ / 2);
-        else
-            return wn * WR + 16 * j;
-    };
-
-    floatx4 acc[MI][NJ];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    const int lr = lane % 16, lg = lane / 16;
-    int foff[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) foff[ks] = lr * G_ROW + (((ks * 4 + lg) ^ swz(lr)) * 16);
-
-#pragma unroll
-    for (int s = 0; s < NS - 1; ++s) issue(s);
-
-    for (int kt = 0; kt < nk; ++kt) {
-        // This wave's DMA of stage kt landed, then everyone's; everyone is
-        // done reading stage kt - 1, whose slot the next DMA reuses.
-        wait_vm<(NS - 2) * P::C>();
-        lds_barrier();
-        issue(kt + NS - 1);
-        const uint8_t* X = slot_base(kt);
-        const uint8_t* Wr = X + P::X_BYTES;
-        const uint8_t* S = Wr + P::W_BYTES;
-        // Every LDS read of the stage goes out first (X fragments, this
-        // wave's codes and scales), so their latencies overlap; then the
-        // decode and the MFMAs.
-        half8 xf[2][MI];
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-                xf[ks][i] = *reinterpret_cast<const half8*>(X + (wm * MI + i) * 16 * G_ROW + foff[ks]);
-        uint32_t sc[NJ];
-        uint2 code[2][NJ];  // Q4: .x only; Q8: both words
-        half8 wf16[2][NJ];
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int rw = wrow_of(j) + lr;
-            if constexpr (QUANT != F16_DT) sc[j] = *reinterpret_cast<const uint32_t*>(S + rw * 4);
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                if constexpr (QUANT == F16_DT)
-                    wf16[ks][j] = *reinterpret_cast<const half8*>(Wr + wrow_of(j) * G_ROW + foff[ks]);
-                else if constexpr (QUANT == Q4_DT)
-                    code[ks][j].x = *reinterpret_cast<const uint32_t*>(Wr + rw * 32 + ks * 16 + lg * 4);
-                else
-                    code[ks][j] = *reinterpret_cast<const uint2*>(Wr + rw * 64 + ks * 32 + lg * 8);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            half8 wf[NJ];
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                if constexpr (QUANT == F16_DT) {
-                    wf[j] = wf16[ks][j];
-                } else {
-                    const half_t d = __builtin_bit_cast(half_t, uint16_t(sc[j] >> (16 * ks)));
-                    if constexpr (QUANT == Q4_DT)
-                        wf[j] = dq4_word(code[ks][j].x, half2v{d, d});
-                    else
-                        wf[j] = dq8_words(code[ks][j].x, code[ks][j].y, half2v{d, d});
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int j = 0; j < NJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[j], xf[ks][i], acc[i][j], 0, 0, 0);
-        }
-    }
-    wait_vm<0>();
-
-    // Epilogue: lane (lr, lg) holds output columns 4 lg..4 lg + 3 of row lr
-    // of each 16 x 16 block.
-    if constexpr (EPI == EPI_QKV) {
-        // The wave's 64 columns are one head of q, k or v (the q width and
-        // the tile edges are multiples of 64).  RoPE pairs dims (c, c + 32),
-        // which sit in blocks j and j + 2 of the same lane.
-        const QkvHeads& o = g.qkv;
-        const int64_t c0 = n0 + wn * WR;
-        if (c0 >= N) return;
-        const int sec = int(c0 / o.dq);
-        const int64_t head = (c0 % o.dq) / 64;
-        float bias[NJ][4];
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                bias[j][r] = g.bias ? float(__builtin_bit_cast(half_t, g.bias[c0 + 16 * j + 4 * lg + r])) : 0.0f;
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-            const int64_t m = m0 + (wm * MI + i) * 16 + lr;
-            if (m >= M) continue;
-            float v[NJ][4];
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) v[j][r] = acc[i][j][r] + bias[j][r];
-            if (sec < 2 && o.rope) {
-                // rope_bi.wgsl:30-49: a' = a cos - b sin, b' = b cos + a sin.
-                const float2* rp = o.rope + int64_t(o.meta[4 * m]) * 32;
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float2 cs = rp[16 * j + 4 * lg + r];
-                        const float a = v[j][r], b = v[j + 2][r];
-                        v[j][r] = a * cs.x - b * cs.y;
-                        v[j + 2][r] = b * cs.x + a * cs.y;
-                    }
-            }
-            if (sec < 2) {
-                const float sc = sec == 0 ? o.qscale : 1.0f;
-                half_t* dst = (sec == 0 ? o.q16 : o.k16) + (head * o.tpad + m) * 64;
-#pragma unroll
-                for (int j = 0; j < NJ; ++j)
-                    *reinterpret_cast<half4*>(dst + 16 * j + 4 * lg) =
-                        half4{half_t(v[j][0] * sc), half_t(v[j][1] * sc), half_t(v[j][2] * sc), half_t(v[j][3] * sc)};
-            } else {
-                half_t* dst = o.vt + (head * (o.tpad / 32) + m / 32) * (64 * 32) + vt_col32(int(m % 32));
-#pragma unroll
-                for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) dst[(16 * j + 4 * lg + r) * 32] = half_t(v[j][r]);
-            }
-        }
-        return;
-    }
-    constexpr int NO = GATED ? NJ / 2 : NJ;
-    const int64_t nw0 = n0 + (GATED ? wn * (WR / 2) : wn * WR);
-    float cbias[EPI == EPI_RELU_F16 ? NO : 1][4];
-    if constexpr (EPI == EPI_RELU_F16) {
-#pragma unroll
-        for (int j = 0; j < NO; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t n = nw0 + j * 16 + lg * 4 + r;
-                cbias[j][r] = n < N ? float(__builtin_bit_cast(half_t, g.bias[n])) : 0.0f;
-            }
-    }
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-        const int64_t m = m0 + (wm * MI + i) * 16 + lr;
-        if (m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < NO; ++j) {
-            const int64_t n = nw0 + j * 16 + lg * 4;
-            float v[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if constexpr (EPI == EPI_GELU_TANH)
-                    v[r] = gelu_tanh(acc[i][j][r]) * acc[i][j + NJ / 2][r];
-                else if constexpr (EPI == EPI_GELU_ERF)
-                    v[r] = gelu_erf(acc[i][j][r]) * acc[i][j + NJ / 2][r];
-                else if constexpr (EPI == EPI_RELU_F16)
-                    v[r] = fmaxf(acc[i][j][r] + cbias[j][r], 0.0f);
-                else
-                    v[r] = acc[i][j][r];
-            }
-            constexpr bool F16_OUT = EPI != EPI_F32;
-            if (n + 3 < N) {
-                if constexpr (F16_OUT) {
-                    *reinterpret_cast<half4*>(static_cast<half_t*>(g.y) + m * g.ldy + n) =
-                        half4{half_t(v[0]), half_t(v[1]), half_t(v[2]), half_t(v[3])};
-                } else {
-                    *reinterpret_cast<float4*>(static_cast<float*>(g.y) + int64_t(blockIdx.y) * g.part_stride +
-                                               m * g.ldy + n) =
-                        make_float4(v[0], v[1], v[2], v[3]);
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (n + r >= N) break;
-                    if constexpr (F16_OUT)
-                        static_cast<half_t*>(g.y)[m * g.ldy + n + r] = half_t(v[r]);
-                    else
-                        static_cast<float*>(g.y)[int64_t(blockIdx.y) * g.part_stride + m * g.ldy + n + r] = v[r];
-                }
-            }
-        }
-    }
-}
-
 // ------------------------------------------------------ 32x32x16 tiles
 
 // The decoder's products (f32 out and the gated GeGLU) on
@@ -545,6 +204,191 @@ struct Cfg32 {
     static_assert(NS >= 3, "ring needs >= 3 slots: one read into registers, one landing, one in flight");
     static_assert(WL + (NS - 2) * C <= 63, "vmcnt range");
 };
+
+// A pair of four-value f16 groups, columns c .. c + 3 in lanes l < 32 and
+// c + 4 .. c + 7 in lanes l + 32 for group a (c) and group b (c + 8), turned
+// into eight consecutive columns per lane: c .. c + 7 of the row in lanes
+// l < 32, c + 8 .. c + 15 in lanes l + 32.
+__device__ inline uint4 wide8(half4 a, half4 b) {
+    const uint2 ua = __builtin_bit_cast(uint2, a), ub = __builtin_bit_cast(uint2, b);
+    const auto x = __builtin_amdgcn_permlane32_swap(ua.x, ub.x, false, false);
+    const auto y = __builtin_amdgcn_permlane32_swap(ua.y, ub.y, false, false);
+    return uint4{uint32_t(x[0]), uint32_t(y[0]), uint32_t(x[1]), uint32_t(y[1])};
+}
+
+// What the 32x32 tiles do with their sums: lane (lr, lh) holds, for
+// activation row m0 + 32 i + lr, columns nw0 + 32 j + 8 q + 4 lh + 0..3 of
+// weight block j in elements 4 q .. 4 q + 3 (gated: blocks NJ / 2 .. of the
+// up matrix).  Every f16 is converted from a value first rounded to f32 and
+// every multiply-add that rounds once is an explicit fmaf, so the outputs of
+// a row do not depend on the tile shape that computed it.
+template <int MI, int NJ, int EPI, bool W8 = false>
+__device__ inline void finish32(const GemmArgs& g, const floatx16 (&acc)[MI][NJ], int64_t m0, int64_t nw0, int lane) {
+    constexpr bool GATED = EPI == EPI_GELU_TANH || EPI == EPI_GELU_ERF;
+    constexpr int NO = GATED ? NJ / 2 : NJ;
+    const int lr = lane % 32, lh = lane / 32;
+    const int64_t M = g.m, N = g.w0.rows;
+    if constexpr (EPI == EPI_QKV) {
+        // The wave's 64 columns are one head of q, k or v.  RoPE pairs dims
+        // (c, c + 32): blocks 0 and 1 of the same lane and element.
+        static_assert(NJ == 2, "one 64-wide head per wave");
+        const QkvHeads& o = g.qkv;
+        if (nw0 >= N) return;
+        const int sec = int(nw0 / o.dq);
+        const int64_t head = (nw0 % o.dq) / 64;
+        float bias[2][16];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                bias[j][e] = g.bias ? float(__builtin_bit_cast(half_t, g.bias[nw0 + 32 * j + 8 * (e / 4) + 4 * lh + e % 4]))
+                                    : 0.0f;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            const int64_t m = m0 + 32 * i + lr;
+            const bool live = m >= 0 && m < M;
+            float v[2][16];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) v[j][e] = acc[i][j][e] + bias[j][e];
+            if (sec < 2) {
+                if (o.rope) {
+                    // rope_bi.wgsl:30-49: a' = a cos - b sin, b' = b cos + a sin.
+                    const float2* rp = o.rope + int64_t(live ? o.meta[4 * m] : 0) * 32 + 4 * lh;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const float4 c01 = *reinterpret_cast<const float4*>(rp + 8 * q);
+                        const float4 c23 = *reinterpret_cast<const float4*>(rp + 8 * q + 2);
+                        const float cs[4] = {c01.x, c01.z, c23.x, c23.z}, sn[4] = {c01.y, c01.w, c23.y, c23.w};
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float a = v[0][4 * q + r], b = v[1][4 * q + r];
+                            v[0][4 * q + r] = fmaf(a, cs[r], -(b * sn[r]));
+                            v[1][4 * q + r] = fmaf(b, cs[r], a * sn[r]);
+                        }
+                    }
+                }
+                const float sc = sec == 0 ? o.qscale : 1.0f;
+                half_t* dst = (sec == 0 ? o.q16 : o.k16) + (head * o.tpad + m) * 64;
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; q += 2) {
+                        half4 h[2];
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+                            h[u] = half4{f16_rounded(v[j][4 * (q + u)] * sc), f16_rounded(v[j][4 * (q + u) + 1] * sc),
+                                         f16_rounded(v[j][4 * (q + u) + 2] * sc), f16_rounded(v[j][4 * (q + u) + 3] * sc)};
+                        const uint4 w = wide8(h[0], h[1]);
+                        if (live) *reinterpret_cast<uint4*>(dst + 32 * j + 8 * (q + lh)) = w;
+                    }
+            } else {
+                // V^T: lanes 2 k and 2 k + 1 hold neighbouring keys of a
+                // dimension, two f16 of one word; the even lane writes the
+                // pair of one dimension, the odd lane the next one's.
+                half_t* dst = o.vt + (head * (o.tpad / 32) + m / 32) * (64 * 32) + vt_col32(lr & ~1);
+                const bool odd = lane & 1;
+                const bool pair = __shfl_xor(int(live), 1, WAVE) && live;
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; e += 2) {
+                        const uint32_t a = __builtin_bit_cast(uint16_t, f16_rounded(v[j][e]));
+                        const uint32_t b = __builtin_bit_cast(uint16_t, f16_rounded(v[j][e + 1]));
+                        const int dim = 32 * j + 8 * (e / 4) + 4 * lh + e % 4;
+                        const uint32_t got = uint32_t(__builtin_amdgcn_update_dpp(0, int(odd ? a : b), 0xb1, 0xf, 0xf, false));
+                        const uint32_t w = odd ? (got | b << 16) : (a | got << 16);
+                        if (pair) {
+                            *reinterpret_cast<uint32_t*>(dst + (dim + int(odd)) * 32) = w;
+                        } else if (live) {  // the pass's last key: alone
+                            dst[dim * 32 + int(odd)] = __builtin_bit_cast(half_t, uint16_t(a));
+                            dst[(dim + 1) * 32 + int(odd)] = __builtin_bit_cast(half_t, uint16_t(b));
+                        }
+                    }
+            }
+        }
+        return;
+    }
+    float cbias[EPI == EPI_RELU_F16 ? NO : 1][16];
+    if constexpr (EPI == EPI_RELU_F16) {
+#pragma unroll
+        for (int j = 0; j < NO; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int64_t n = nw0 + 32 * j + 8 * (e / 4) + 4 * lh + e % 4;
+                cbias[j][e] = n < N ? float(__builtin_bit_cast(half_t, g.bias[n])) : 0.0f;
+            }
+    }
+    auto value = [&](int i, int j, int x) {
+        if constexpr (EPI == EPI_GELU_TANH)
+            return gelu_tanh(acc[i][j][x]) * acc[i][j + NJ / 2][x];
+        else if constexpr (EPI == EPI_GELU_ERF)
+            return gelu_erf(acc[i][j][x]) * acc[i][j + NJ / 2][x];
+        else if constexpr (EPI == EPI_RELU_F16)
+            return fmaxf(acc[i][j][x] + cbias[j][x], 0.0f);
+        else
+            return acc[i][j][x];
+    };
+    // f16 rows: whole 32-column blocks of 16-byte-aligned rows go out eight
+    // columns per store, others as the lane's own four.
+    const bool aligned = EPI != EPI_F32 && g.ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(g.y) & 15) == 0;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int64_t m = m0 + 32 * i + lr;
+        const bool live = m >= 0 && m < M;
+#pragma unroll
+        for (int j = 0; j < NO; ++j) {
+            const int64_t n0 = nw0 + 32 * j;
+            if constexpr (EPI == EPI_F32) {
+                if (!live) continue;
+                float* dst = static_cast<float*>(g.y) + int64_t(blockIdx.y) * g.part_stride + m * g.ldy;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int64_t n = n0 + 8 * q + 4 * lh;
+                    if (n + 3 < N) {
+                        *reinterpret_cast<float4*>(dst + n) = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1],
+                                                                          acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (n + r < N) dst[n + r] = acc[i][j][4 * q + r];
+                    }
+                }
+            } else if (W8 && aligned && n0 + 32 <= N) {
+                half_t* dst = static_cast<half_t*>(g.y) + m * g.ldy;
+#pragma unroll
+                for (int q = 0; q < 4; q += 2) {
+                    half4 h[2];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) h[u][r] = f16_rounded(value(i, j, 4 * (q + u) + r));
+                    const uint4 w = wide8(h[0], h[1]);
+                    if (live) *reinterpret_cast<uint4*>(dst + n0 + 8 * (q + lh)) = w;
+                }
+            } else {
+                if (!live) continue;
+                half_t* dst = static_cast<half_t*>(g.y) + m * g.ldy;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int64_t n = n0 + 8 * q + 4 * lh;
+                    float v[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = value(i, j, 4 * q + r);
+                    if (n + 3 < N) {
+                        *reinterpret_cast<half4*>(dst + n) =
+                            half4{f16_rounded(v[0]), f16_rounded(v[1]), f16_rounded(v[2]), f16_rounded(v[3])};
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (n + r < N) dst[n + r] = f16_rounded(v[r]);
+                    }
+                }
+            }
+        }
+    }
+}
 
 template <class F, size_t... I>
 __device__ inline bool run_phases(F& f, std::index_sequence<I...>) {
@@ -967,7 +811,6 @@ __global__ __launch_bounds__(NW_ * WAVE) void gemm32_kernel(GemmArgs g) {
 
     // PAIR: the gate waves' sums to the up waves, element for element (the
     // same lane layout), through LDS that every wave has finished with.
-    floatx16 gsum[PAIR ? MI : 1][PAIR ? NJ : 1];
     if constexpr (PAIR) {
         float* E = reinterpret_cast<float*>(smem);
         lds_barrier();
@@ -981,62 +824,218 @@ __global__ __launch_bounds__(NW_ * WAVE) void gemm32_kernel(GemmArgs g) {
         }
         lds_barrier();
         if (wave < NW / 2) return;
+        floatx16 both[MI][2 * NJ];
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                both[i][NJ + j] = acc[i][j];
+#pragma unroll
+                for (int e = 0; e < 16; ++e) both[i][j][e] = E[(((pw * MI + i) * NJ + j) * 16 + e) * WAVE + lane];
+            }
+        finish32<MI, 2 * NJ, EPI>(g, both, m0, n0 + pw * WR, lane);
+    } else if constexpr (EPI != EPI_QKPREP) {
+        finish32<MI, NJ, EPI>(g, acc, m0, n0 + (GATED ? wave * (WR / 2) : wave * WR), lane);
+    }
+}
+
+// Wide tiles for long passes: the same products, operand layouts and K order
+// as gemm32_kernel (so the same sums), with 128 x 64 results per wave.  A
+// 32-row block per wave reads each X fragment from LDS for one MFMA, which
+// takes the LDS its whole bandwidth; two blocks halve that and share the
+// decode over four row blocks.  The accumulators take half the registers,
+// so the X fragments and the decoded weights are double buffered one k-step
+// (16 K) at a time instead of a stage.  Iteration kt, k-step ks:
+//   read the fragments and decode the weights of the next k-step (of stage
+//   kt + 1 after a wait for its X DMA and a barrier, which also frees stage
+//   kt's ring slot: the DMA of stage kt + NS goes out), between the MFMAs
+//   of this one; after the last decode, load stage kt + 2's weights.
+template <int QUANT, int MI, int NJ, int EPI, int NS, int NW_>
+__global__ __launch_bounds__(NW_ * WAVE, 2) void gemm32w_kernel(GemmArgs g) {
+    using P = Cfg32<QUANT, MI, NJ, EPI, NS, NW_, false>;
+    constexpr bool GATED = P::GATED;
+    constexpr int NW = P::NW, BM = P::BM, BN = P::BN, WR = P::WR, PK = P::PK;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = int(threadIdx.x), lane = tid % WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int64_t N = g.w0.rows, K = g.w0.cols, M = g.m;
+    const int ntn = int((N + BN - 1) / BN);
+    const int ntiles = ntn * int((M + BM - 1) / BM);
+    const int per_xcd = int(gridDim.x) / 8;
+    const int tile = (int(blockIdx.x) % 8) * per_xcd + int(blockIdx.x) / 8;
+    if (tile >= ntiles) return;
+    const int64_t n0 = int64_t(tile % ntn) * BN, m0 = int64_t(tile / ntn) * BM;
+    const int kbeg = int(blockIdx.y) * int(K / g.ksplit);
+    const int nk = int((K / g.ksplit + G_BK - 1) / G_BK);
+    const int K32 = int(K), last = nk - 1;
+
+    uint32_t xoff[P::X_I];
+    int xcol[P::X_I];
+#pragma unroll
+    for (int i = 0; i < P::X_I; ++i) {
+        const int slot = (i * NW + wave) * WAVE + lane;
+        const int r = slot / 8, lc = (slot % 8) ^ swz(r);
+        xcol[i] = lc * 8;
+        xoff[i] = slot < P::X_CH && m0 + r < M ? uint32_t(((m0 + r) * g.ldx + lc * 8) * 2) : OOB;
+    }
+    const int64_t stages = g.w0.stages, rblocks = (N + 31) / 32, rb0 = n0 / 32;
+    const int64_t live_blocks = rblocks - rb0;
+    auto mat_of = [&](int j) { return GATED && j >= NJ / 2 ? 1 : 0; };
+    auto blk_of = [&](int j) { return GATED ? wave * (NJ / 2) + (j % (NJ / 2)) : wave * NJ + j; };
+    uint32_t coff[NJ], scoff[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        coff[j] = blk_of(j) < live_blocks ? uint32_t(blk_of(j) * stages * PK + lane * (PK / 64)) : OOB;
+        scoff[j] = blk_of(j) < live_blocks ? uint32_t(blk_of(j) * stages * TILE_SCALE_BYTES + (lane % 32) * 4) : OOB;
+    }
+    auto slot_base = [&](int s) { return smem + (unsigned(s) % unsigned(NS)) * P::X_BYTES; };
+    const int64_t xbytes = M * g.ldx * 2;
+    const bool ktail = (K32 & (G_BK - 1)) != 0;
+    auto issue_x = [&](int s) {
+        uint8_t* base = slot_base(s);
+        const int k0 = __builtin_amdgcn_readfirstlane(kbeg + (s < last ? s : last) * G_BK);
+        const bool tail = ktail && k0 + G_BK > K32;
+#pragma unroll
+        for (int i = 0; i < P::X_I; ++i) {
+            const uint32_t o = tail && xcol[i] >= K32 - k0 ? OOB : xoff[i];
+            const __amdgpu_buffer_rsrc_t r = rsrc(g.x, xbytes);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(base + (i * NW + wave) * WAVE * 16), 16, o,
+                                                     k0 * 2, 0, 0);
+        }
+    };
+    struct WRegs {
+        uint4 code[NJ][P::CL];
+        uint32_t sc[NJ];
+    };
+    const int st0 = kbeg / G_BK;
+    auto issue_w = [&](int s, WRegs& w) {
+        const int st = __builtin_amdgcn_readfirstlane(st0 + (s < last ? s : last));
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const DevWeight& wt = mat_of(j) ? g.w1 : g.w0;
+            const __amdgpu_buffer_rsrc_t r = rsrc(wt.tiles + rb0 * stages * PK, live_blocks * stages * PK);
+#pragma unroll
+            for (int c = 0; c < P::CL; ++c)
+                w.code[j][c] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                             r, coff[j] + 16 * c, st * PK, 0));
+            if constexpr (QUANT != F16_DT) {
+                const __amdgpu_buffer_rsrc_t rs = rsrc(wt.tscales + rb0 * stages * TILE_SCALE_BYTES,
+                                                       live_blocks * stages * TILE_SCALE_BYTES);
+                w.sc[j] = __builtin_amdgcn_raw_buffer_load_b32(rs, scoff[j], st * TILE_SCALE_BYTES, 0);
+            }
+        }
+    };
+    // The memory instructions' order (X of a stage, then weights) is what the
+    // wait counts rely on: compiler fences keep it.
+    auto fence = [] { asm volatile("" ::: "memory"); };
+
+    floatx16 acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = floatx16{};
+    const int lr = lane % 32, lh = lane / 32;
+    int foff[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) foff[ks] = lr * G_ROW + (((2 * ks + lh) ^ swz(lr)) * 16);
+
+    struct Frag {
+        half8 x[MI], w[NJ];
+    };
+    auto read_x = [&](int s, int ks, Frag& f) {
+        const uint8_t* X = slot_base(s);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) f.x[i] = *reinterpret_cast<const half8*>(X + i * 32 * G_ROW + foff[ks]);
+    };
+    auto decode = [&](const WRegs& w, int ks, Frag& f) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            if constexpr (QUANT == F16_DT) {
+                f.w[j] = __builtin_bit_cast(half8, w.code[j][ks]);
+            } else {
+                const half_t d = __builtin_bit_cast(half_t, uint16_t(w.sc[j] >> (16 * (ks / 2))));
+                if constexpr (QUANT == Q4_DT) {
+                    const uint4 u = w.code[j][0];
+                    f.w[j] = dq4_word(ks == 0 ? u.x : ks == 1 ? u.y : ks == 2 ? u.z : u.w, half2v{d, d});
+                } else {
+                    const uint4 u = w.code[j][ks / 2];
+                    f.w[j] = ks % 2 == 0 ? dq8_words(u.x, u.y, half2v{d, d}) : dq8_words(u.z, u.w, half2v{d, d});
+                }
+            }
+        }
+    };
+    auto mfmas = [&](const Frag& f) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) gsum[i][j][e] = E[(((pw * MI + i) * NJ + j) * 16 + e) * WAVE + lane];
-    }
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.w[j], f.x[i], acc[i][j], 0, 0, 0);
+    };
 
-    // Epilogue: lane (lr, lh) holds, for activation row lr of block i,
-    // output columns 8 q + 4 lh + 0..3 of weight block j (q = 0..3).
-    constexpr int NO = GATED && !PAIR ? NJ / 2 : NJ;
-    const int64_t nw0 = n0 + (PAIR ? pw * WR : GATED ? wave * (WR / 2) : wave * WR);
+    constexpr int VPM = (NJ * (QUANT == F16_DT ? 0 : 14) + MI * NJ - 1) / (MI * NJ) + 1;  // decode per MFMA
+    WRegs wr[2];
+    Frag fa, fb;
+    issue_x(0);
+    fence();
 #pragma unroll
-    for (int i = 0; i < MI; ++i) {
-        const int64_t m = m0 + i * 32 + lr;
-        if (m < 0 || m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < NO; ++j)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int64_t n = nw0 + j * 32 + 8 * q + 4 * lh;
-                float v[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if constexpr (PAIR && EPI == EPI_GELU_TANH)
-                        v[r] = gelu_tanh(gsum[i][j][4 * q + r]) * acc[i][j][4 * q + r];
-                    else if constexpr (PAIR)
-                        v[r] = gelu_erf(gsum[i][j][4 * q + r]) * acc[i][j][4 * q + r];
-                    else if constexpr (EPI == EPI_GELU_TANH)
-                        v[r] = gelu_tanh(acc[i][j][4 * q + r]) * acc[i][j + NJ / 2][4 * q + r];
-                    else if constexpr (EPI == EPI_GELU_ERF)
-                        v[r] = gelu_erf(acc[i][j][4 * q + r]) * acc[i][j + NJ / 2][4 * q + r];
-                    else
-                        v[r] = acc[i][j][4 * q + r];
-                }
-                if (n + 3 < N) {
-                    // f16 from the f32 value in every tile shape (no fused
-                    // multiply-convert in one instance and not another)
-                    if constexpr (GATED)
-                        *reinterpret_cast<half4*>(static_cast<half_t*>(g.y) + m * g.ldy + n) =
-                            half4{f16_rounded(v[0]), f16_rounded(v[1]), f16_rounded(v[2]), f16_rounded(v[3])};
-                    else
-                        *reinterpret_cast<float4*>(static_cast<float*>(g.y) + int64_t(blockIdx.y) * g.part_stride +
-                                                   m * g.ldy + n) = make_float4(v[0], v[1], v[2], v[3]);
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        if (n + r >= N) break;
-                        if constexpr (GATED)
-                            static_cast<half_t*>(g.y)[m * g.ldy + n + r] = f16_rounded(v[r]);
-                        else
-                            static_cast<float*>(g.y)[int64_t(blockIdx.y) * g.part_stride + m * g.ldy + n + r] = v[r];
-                    }
-                }
-            }
+    for (int s = 1; s < NS; ++s) {
+        issue_x(s);
+        fence();
+        if (s >= NS - 2) {
+            issue_w(s - (NS - 2), wr[s - (NS - 2)]);
+            fence();
+        }
     }
+    wait_vm<(NS - 1) * P::X_I>();  // stage 0's X: at least the other stages' follow it
+    lds_barrier();
+    read_x(0, 0, fa);
+    decode(wr[0], 0, fa);
+    int kt = 0;
+    auto step = [&](auto phase) {
+        constexpr int PH = decltype(phase)::value;
+        WRegs& cw = wr[PH];
+        WRegs& nw = wr[1 - PH];
+        // One k-step: the next one's fragment reads first, its decode spread
+        // between this one's MFMAs; nothing moves across its ends (the
+        // compiler would otherwise pull a later decode, and with it the wait
+        // for its weights, ahead of these MFMAs).
+        auto kstep = [&](const WRegs& w, int s, int ks, const Frag& cur, Frag& nxt) {
+            read_x(s, ks, nxt);
+            decode(w, ks, nxt);
+            mfmas(cur);
+            __builtin_amdgcn_sched_group_barrier(0x100, MI, 0);  // LDS reads
+#pragma unroll
+            for (int u = 0; u < MI * NJ; ++u) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);  // VALU
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        kstep(cw, kt, 1, fa, fb);
+        kstep(cw, kt, 2, fb, fa);
+        kstep(cw, kt, 3, fa, fb);
+        // Stage kt + 1's X landed (this wave's; past the barrier everyone's,
+        // and everyone holds stage kt's last fragments).
+        fence();
+        wait_vm<(NS - 2) * P::C>();
+        lds_barrier();
+        issue_x(kt + NS);
+        fence();
+        issue_w(kt + 2, cw);
+        fence();
+        __builtin_amdgcn_sched_barrier(0);
+        kstep(nw, kt + 1, 0, fb, fa);
+        ++kt;
+    };
+    // (Two stages per iteration and no exit between them: with one, the
+    // compiler's wait counts have to hold on a path that skips a stage.)
+    for (int left = nk; left >= 2; left -= 2) {
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+    }
+    if (nk & 1) step(std::integral_constant<int, 0>{});
+    wait_vm<0>();
+    finish32<MI, NJ, EPI, true>(g, acc, m0, n0 + (GATED ? wave * (WR / 2) : wave * WR), lane);
 }
 
 // Resident X tiles up to this many bytes of LDS (one workgroup per CU
@@ -1074,55 +1073,79 @@ static void run32(hipStream_t s, const GemmArgs& g) {
     OMG_HIP(hipGetLastError());
 }
 
-template <int QUANT, int MI, int NJ, int EPI, int NS, int NW = 4, int WM = 1>
-static void run(hipStream_t s, const GemmArgs& g) {
-    using P = Cfg<QUANT, MI, NJ, EPI, NS, NW, WM>;
+template <int QUANT, int MI, int NJ, int EPI, int NS, int NW = 4>
+static void run32w(hipStream_t s, const GemmArgs& g) {
+    using P = Cfg32<QUANT, MI, NJ, EPI, NS, NW, false>;
+    for (const DevWeight* w : {&g.w0, &g.w1})
+        if (!w->tiles || w->stages != (w->cols + G_BK - 1) / G_BK || (QUANT != F16_DT && !w->tscales))
+            fail(E_INVALID, "gemm: weight without stage tiles");
     static bool lds_set = false;
     if (!lds_set) {
-        OMG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<QUANT, MI, NJ, EPI, NS, NW, WM>),
+        OMG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm32w_kernel<QUANT, MI, NJ, EPI, NS, NW>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, P::LDS));
         lds_set = true;
     }
-    const int64_t N = g.w0.rows;
-    const int64_t tiles = ((N + P::BN - 1) / P::BN) * ((g.m + P::BM - 1) / P::BM);
+    if (g.mshift != 0 || g.kfold != 0) fail(E_INVALID, "gemm: wide tiles take no row shift or K pieces");
+    const int64_t tiles = ((g.w0.rows + P::BN - 1) / P::BN) * ((g.m + P::BM - 1) / P::BM);
     const dim3 grid(unsigned((tiles + 7) / 8 * 8), unsigned(g.ksplit));
-    gemm_kernel<QUANT, MI, NJ, EPI, NS, NW, WM><<<grid, dim3(P::T), P::LDS, s>>>(g);
+    gemm32w_kernel<QUANT, MI, NJ, EPI, NS, NW><<<grid, dim3(P::T), P::LDS, s>>>(g);
     OMG_HIP(hipGetLastError());
 }
 
-// Tile choice, measured on MI355X (tiles are activation rows x weight rows).
-// f32 products (gemm32_kernel, 32x32x16, four waves; whole-pass A/B on the
-// 270M model and an isolated sweep with rotating weight sets): 32 x 128
-// for short passes (M <= 512), 64 x 128, 96 x 128 when K is split (twice
-// the tiles), 128 x 128 for long passes (M >= 8192, the encoder's
-// 49,152-token batches).  The other epilogues (gemm_kernel, 16x16x32):
-//   bias+ReLU: short passes 32 x 32 on two waves; 64 x 64 (96 x 64 from
-//   N = 768) for N <= 1280; 128 x 64, 96 x 128 for K >= 4096; 192 x 128
-//   for long passes.  Q/K/V head scatter (64 weight rows per wave): 32 x
-//   256 short, 96 x 256 otherwise.
-//   Gated: 160 x 128 weight rows (64 output columns; a 2,384-token pass
-//   of the 270M model is 480 tiles, at most two per CU, where 128-row
-//   tiles made 608 and left 96 CUs a third) with three ring slots (two:
-//   the whole pass 0.8% slower, though the product's own event time is
-//   0.4 µs shorter), 128 x 256 with three slots
-//   for very wide layers, 192 x 128 for long passes, 64 x 128 for short
-//   (four slots from K 1,024).
-// One template per product type for every M: rows do not depend on M.
+// Row blocks (of 32) of the wide tile: a workgroup of MI blocks takes about
+// 1 + MI units of time whatever the product, and 256 CUs run a round of
+// tiles at a time, so the MI with the least rounds x (1 + MI) is taken (the
+// larger of equals: less decode and weight traffic).  Measured over 19
+// shapes from 300 to 49,152 rows, K 640 to 2,560, it picks the fastest MI
+// or one within 3% of it; f16 weights take twice the registers of Q8 ones
+// and stop at three blocks.
+template <int QUANT>
+static int wide_blocks(int64_t m, int64_t ntn) {
+    int best = 1;
+    int64_t cost = INT64_MAX;
+    for (int mi = QUANT == F16_DT ? 3 : 4; mi >= 1; --mi) {
+        const int64_t tiles = (m + 32 * mi - 1) / (32 * mi) * ntn, c = (tiles + 255) / 256 * (1 + mi);
+        if (c < cost) cost = c, best = mi;
+    }
+    return best;
+}
+
+// 32 MI rows x 256 weight rows on four waves.
+template <int QUANT, int EPI>
+static void run_wide(hipStream_t s, const GemmArgs& g, int64_t cols_per_tile) {
+    const int mi = wide_blocks<QUANT>(g.m, (g.w0.rows + cols_per_tile - 1) / cols_per_tile * g.ksplit);
+    if constexpr (QUANT != F16_DT)
+        if (mi == 4) return run32w<QUANT, 4, 2, EPI, 3, 4>(s, g);
+    if (mi == 3) return run32w<QUANT, 3, 2, EPI, 3, 4>(s, g);
+    if (mi == 2) return run32w<QUANT, 2, 2, EPI, 4, 4>(s, g);
+    return run32w<QUANT, 1, 2, EPI, 4, 4>(s, g);
+}
+
+// Tile choice, measured on MI355X (tiles are activation rows x weight rows;
+// both kernels give every output element the same sums, so rows never
+// depend on M).  gemm32_kernel, whose K loop has the shorter stages, while
+// its tiles make one round of the 256 CUs; above that the wide tiles.
+// Isolated products, 16x16x32 tiles / gemm32_kernel before -> now:
+//   [q | k | v] heads, N 2,304, K 768, Q8: 49,152 rows 303 -> 236 us, 6,000
+//   53 -> 33, 3,000 32 -> 21, 500 18.5 -> 9.8; erf-gated, N 2 x 1,152: 226
+//   -> 204, 53 -> 28, 33 -> 17, 12.1 -> 9.1; o, N 768: 84 -> 79, 20.8 ->
+//   16.3, 14.5 -> 11.0; tanh-gated, N 2 x 10,240, K 2,560, Q4, 16,320 rows:
+//   1,557 -> 1,444; N 2 x 6,912, K 1,152, Q8, 384 rows: 32.5 -> 20.8.
+// Long products are bound by power: the card runs the 16,320-row one at
+// 1.6 GHz with its matrix cores 67% busy (a library f16 product of 8,192^3:
+// 1.4 GHz, 89%).
 template <int QUANT, int EPI>
 static void dispatch(hipStream_t s, const GemmArgs& g) {
     const int64_t N = g.w0.rows, K = g.w0.cols, M = g.m;
+    auto tiles = [&](int64_t rows, int64_t cols) { return (M + rows - 1) / rows * ((N + cols - 1) / cols) * g.ksplit; };
     if constexpr (EPI == EPI_QKV) {
-        if (M <= 512) return run<QUANT, 2, 4, EPI, 4, 4>(s, g);
-        return run<QUANT, 6, 4, EPI, 2, 4>(s, g);
+        // a 64-wide head per wave
+        if (tiles(32, 256) <= 256) return run32<QUANT, 1, 2, EPI, 4, 4>(s, g);
+        if (tiles(64, 256) <= 256) return run32<QUANT, 2, 2, EPI, 4, 4>(s, g);
+        return run_wide<QUANT, EPI>(s, g, 256);
     } else if constexpr (EPI == EPI_RELU_F16) {
-        if (M <= 512) return run<QUANT, 2, 1, EPI, 4, 2>(s, g);
-        if (M >= 8192) return run<QUANT, 12, 2, EPI, 2, 4>(s, g);
-        if (N <= 1280) {
-            if (N > 768) return run<QUANT, 6, 1, EPI, 4, 4>(s, g);
-            return run<QUANT, 4, 1, EPI, 4, 4>(s, g);
-        }
-        if (K >= 4096) return run<QUANT, 6, 2, EPI, 2, 4>(s, g);
-        return run<QUANT, 8, 1, EPI, 2, 4>(s, g);
+        if (tiles(32, 128) <= 256) return run32<QUANT, 1, 1, EPI, 4, 4>(s, g);
+        return run_wide<QUANT, EPI>(s, g, 256);
     } else if constexpr (EPI == EPI_QKPREP) {
         // One head on eight waves of one 32-row weight block each (half the
         // decode per wave and K stage of the four-wave tile): short passes,
@@ -1134,51 +1157,32 @@ static void dispatch(hipStream_t s, const GemmArgs& g) {
         if (K <= 768) return run32<QUANT, 2, 1, EPI, 4, 8>(s, g);
         return run32<QUANT, 2, 2, EPI, 4, 4>(s, g);
     } else if constexpr (EPI == EPI_F32) {
-        // 32x32x16 tiles (gemm32_kernel) for every M: the same sums per element
         if (g.kfold > 0) {  // K pieces added in registers (up to 96-row tiles: the totals fit)
             if (M <= 512) return run32<QUANT, 1, 1, EPI, 4, 4, true>(s, g);
             return run32<QUANT, 3, 1, EPI, 4, 4, true>(s, g);
         }
-        if (M <= 512) return run32<QUANT, 1, 1, EPI, 4, 4>(s, g);
-        if (M >= 8192) return run32<QUANT, 4, 1, EPI, 3, 4>(s, g);
-        if (g.ksplit > 1) return run32<QUANT, 3, 1, EPI, 4, 4>(s, g);  // split K: twice the tiles
-        return run32<QUANT, 2, 1, EPI, 4, 4>(s, g);
+        if (M <= 512 && tiles(32, 128) <= 512) return run32<QUANT, 1, 1, EPI, 4, 4>(s, g);
+        if (g.ksplit > 1 && tiles(96, 128) <= 256) return run32<QUANT, 3, 1, EPI, 4, 4>(s, g);
+        if (g.ksplit == 1 && tiles(64, 128) <= 256) return run32<QUANT, 2, 1, EPI, 4, 4>(s, g);
+        // 128 x 256 (five units a round) against 96 x 128 (2.4)
+        if (QUANT == F16_DT || 50 * ((tiles(128, 256) + 255) / 256) > 24 * ((tiles(96, 128) + 255) / 256))
+            return run32w<QUANT, 3, 1, EPI, 3, 4>(s, g);
+        if constexpr (QUANT != F16_DT) return run32w<QUANT, 4, 2, EPI, 3, 4>(s, g);
     } else {
-        if constexpr (EPI == EPI_GELU_TANH) {
-            // The decoder's gated products on the 32x32x16 kernel, weights
-            // in registers: 96 x 128 outputs, 32 x 128 for short passes
-            // (same box against the 16x16x32 kernel below: the 270M
-            // model's cold gate/up 20.7 -> 20.2 us, warm 9.7 -> 9.0 us; the
-            // 4B model's cold gate/up 1,890 -> 1,565 us, its cold pass
-            // -4.8%, warm -5.4%; E2B's warm pass -8.5%).  Ring slots: three
-            // for long passes (270M cold pass -0.5%), four for short ones
-            // (three: the flushed one-branch passes 1-5% slower); 128-row
-            // or 64-column tiles and five slots were 3-10% slower.
-            // Branch-sized passes (M <= 64) pair the waves (a gate and an
-            // up wave per 32 columns: half the decode per wave and stage;
-            // flushed one-branch passes, same box, against 32 x 128 on
-            // four waves of gate and up each: the 270M model's gate/up
-            // 9.2 -> 7.4 us and pass 1.064 -> 1.027 ms, the 4B model's
-            // 23.9 -> 21.4 us and 3.60 -> 3.50 ms).  With X resident (K
-            // <= 1,024) nine slots of weights (four: 7.9 us); through the
-            // ring 64 rows on four waves, four slots (32 rows on two: 21.8
-            // us; five to nine slots 26-29 us).
-            if (M <= 64) {
-                if (K <= 1024) return run32<QUANT, 1, 1, EPI, 9, 2, false, true>(s, g);
-                return run32<QUANT, 2, 1, EPI, 4, 4, false, true>(s, g);
-            }
-            if (M <= 512) return run32<QUANT, 1, 2, EPI, 4, 4>(s, g);
-            return run32<QUANT, 3, 2, EPI, 3, 4>(s, g);
+        // Branch-sized passes (M <= 64) pair the waves (a gate and an up
+        // wave per 32 columns: half the decode per wave and stage; flushed
+        // one-branch passes, same box, against 32 x 128 on four waves of
+        // gate and up each: the 270M model's gate/up 9.2 -> 7.4 us and pass
+        // 1.064 -> 1.027 ms, the 4B model's 23.9 -> 21.4 us and 3.60 -> 3.50
+        // ms).  With X resident (K <= 1,024) nine slots of weights (four:
+        // 7.9 us); through the ring 64 rows on four waves, four slots (32
+        // rows on two: 21.8 us; five to nine slots 26-29 us).
+        if (M <= 64 && EPI == EPI_GELU_TANH) {
+            if (K <= 1024) return run32<QUANT, 1, 1, EPI, 9, 2, false, true>(s, g);
+            return run32<QUANT, 2, 1, EPI, 4, 4, false, true>(s, g);
         }
-        // Short passes: four ring slots from K 1,024 (two are better at
-        // K 640).  The ring depth does not change any sum.
-        if (M <= 512) {
-            if (K >= 1024) return run<QUANT, 4, 2, EPI, 4, 4>(s, g);
-            return run<QUANT, 4, 2, EPI, 2, 4>(s, g);
-        }
-        if (N >= 8192) return run<QUANT, 8, 4, EPI, 3, 4>(s, g);
-        if (M >= 8192) return run<QUANT, 12, 2, EPI, 2, 4>(s, g);
-        return run<QUANT, 10, 2, EPI, 3, 4>(s, g);
+        if (tiles(32, 128) <= 256) return run32<QUANT, 1, 2, EPI, 4, 4>(s, g);
+        return run_wide<QUANT, EPI>(s, g, 128);
     }
 }
 

@@ -272,3 +272,55 @@ def test_readout_of_non_finite_rows_and_streams():
     live = [r for r in range(nrows) if r not in (3, 17)]
     assert np.array_equal(got[live], ref.cpu().numpy()[live])
     assert not np.isfinite(got[3, :26]).any() and np.isnan(got[17]).all()
+
+
+# Wide tiles: a 7,944-column product makes more than one round of tiles from
+# a few dozen rows on, so the rows below pass through the short tiles, every
+# wide row-block count and its partial last tile (and columns past the last
+# whole tile); K 96 and 160 end in half a stage, 320 and 640 have an odd and
+# an even stage count.
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("k", [96, 160, 320, 640])
+def test_wide_tiles_give_the_short_tiles_rows(k, dtype):
+    """Products of one type are the same bits for a row whatever M selects
+    (f32, both gated forms, bias + ReLU), and match a float64 product of the
+    same f16 operands: f32 sums of K products bound the error by 2^-23 K of
+    sum |x||w|, f16 outputs add half an ulp (2^-11)."""
+    rng = np.random.default_rng(k + dtype)
+    n = 7944
+    (tg, gd), (tu, ud) = weight(rng, n, k, dtype, "gate"), weight(rng, n, k, dtype, "up")
+    wg, wu = g.DeviceWeight(tg), g.DeviceWeight(tu)
+    bias = rng.uniform(-1, 1, n).astype(np.float16)
+    x = rng.uniform(-1, 1, (700, k)).astype(np.float16)
+    bd = dev(bias)
+
+    def run(m, kind):
+        xd = dev(x[:m])
+        y = torch.zeros((m, n), dtype=torch.float32 if kind == "f32" else torch.float16, device="cuda")
+        if kind == "f32":
+            wg.gemm(xd.data_ptr(), k, m, y.data_ptr(), n)
+        elif kind == "relu":
+            wg.gemm_bias_relu(xd.data_ptr(), k, m, bd.data_ptr(), y.data_ptr(), n)
+        else:
+            (wg.gemm_geglu if kind == "tanh" else wg.gemm_geglu_erf)(wu, xd.data_ptr(), k, m, y.data_ptr(), n)
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    xf = x.astype(np.float64)
+    a, u = xf @ gd.T, xf @ ud.T
+    bound = 2.0 ** -23 * k * (np.abs(xf) @ np.abs(gd).T)
+    for kind in ("f32", "relu", "tanh", "erf"):
+        full = run(700, kind)
+        for m in (1, 33, 95, 130, 257, 480):
+            assert np.array_equal(run(m, kind), full[:m]), f"{kind} rows at M {m}"
+        got = full.astype(np.float64)
+        if kind == "f32":
+            assert (np.abs(got - a) <= bound + 1e-30).all()
+        elif kind == "relu":
+            z = np.maximum(a + bias, 0.0)
+            assert (np.abs(got - z) <= bound + 2.0 ** -11 * np.abs(z) + 1e-7).all()
+        else:
+            from math import erf
+            z = a[:40]
+            z = (gelu(z) if kind == "tanh" else 0.5 * z * (1.0 + np.vectorize(erf)(z / np.sqrt(2.0)))) * u[:40]
+            assert np.max(np.abs(got[:40] - z) / np.maximum(np.abs(z), 1.0)) < 2e-3
