@@ -1,43 +1,41 @@
 // Dequant-fused MFMA GEMMs for the linear layers (matmul.wgsl and
 // matmul_gated.wgsl's job): Y[M,N] = f16(X)[M,K] . deq(W)[N,K]^T with f32
-// accumulation on v_mfma_f32_16x16x32_f16.
+// accumulation on v_mfma_f32_32x32x16_f16.
 //
 // Row-owner tiles: NW wave64s per workgroup over a BM x BN output tile,
-// BM = 16 * MI activation rows.  Each wave owns 16 * NJ weight rows (gated:
-// NJ / 2 row blocks of the gate matrix and the same rows of the up matrix)
-// across all BM rows, so every weight row is decoded by exactly one wave,
-// straight from its codes into MFMA operand registers.  K advances 64 at a
-// time ("stages").  Data path of one stage:
-//
-//   global --LDS DMA--> ring slot (NS slots): X tile f16 [BM][64], raw
-//       weight codes (Q4: [rows][2 blocks][16 B], Q8: [rows][64 B], F16:
-//       [rows][64] f16) and one dword of two block scales per weight row;
-//   ring slot --ds_read--> X fragments (b128) and this wave's codes and
-//       scales --decode in registers--> weight fragments --> MFMA.
-//
-// The DMA (buffer_load ... lds, 16 B or 4 B per lane) keeps NS - 1 stages
-// in flight with no registers held for them; the stage's K offset rides in
-// the instruction's scalar offset, so the per-lane offsets are fixed for
-// the whole loop.  One barrier per stage.  The ring alone sets the LDS
-// footprint, so several workgroups share a CU.  The decode rounds
+// BM = 32 * MI activation rows.  Each wave owns 32 * NJ weight rows (gated:
+// half of them rows of the gate matrix and half the same rows of the up
+// matrix) across all BM rows, so every weight row is decoded by exactly one
+// wave of the tile, straight from its codes into MFMA operand registers.  K
+// advances 64 at a time ("stages").  The X tile of a stage (f16 [BM][64])
+// goes by LDS DMA into a ring of NS slots; the weights come from the tiled
+// copy (one contiguous packet of codes per 32 rows and stage, and one of
+// scales) into the registers of the wave that owns the rows.  The DMA holds
+// no registers for what is in flight, the stage's K offset rides in the
+// instruction's scalar offset, so the per-lane offsets are fixed for the
+// whole loop, and there is one barrier per stage.  The decode rounds
 // (q - 8) * d (or q * d) to f16 once, the reference's f16 rounding point
 // (shaders/weight.wgsl:40-54).
 //
-// X and f16 weight tiles are 128 B per row with the 16 B chunk c of row r
-// stored at c ^ ((r >> 1) & 7), so the 16 rows x 4 chunks of one fragment
-// read hit distinct banks.
+// Two kernels with the same sums: gemm32_kernel (fragments of a whole stage
+// at a time; short products, where a tile's own latency counts) and
+// gemm32w_kernel (fragments one k-step ahead, so twice the tile in the same
+// registers; products of more than one round of tiles).
 //
-// MFMA operand layout (16x16x32 f16): lane l supplies A[l % 16][8*(l/16)..+8)
-// and B[8*(l/16)..+8)[l % 16]; the f32 result D[4*(l/16) + r][l % 16] lands
-// in element r of the lane's float4.  The weight fragment is the A operand
-// and the activation fragment the B operand, so D = (X W^T)^T and each lane
-// ends up with four consecutive output columns of one row: the epilogue
-// stores them as one vector.
+// X tiles are 128 B per row with the 16 B chunk c of row r stored at
+// c ^ ((r >> 1) & 7), so the rows of one fragment read hit distinct banks.
+//
+// MFMA operand layout (32x32x16 f16): lane l supplies A[l % 32][8*(l/32)..+8)
+// and B[8*(l/32)..+8)[l % 32]; D[8*q + 4*(l/32) + r][l % 32] of the f32
+// result lands in element 4 q + r of the lane's sixteen.  The weight fragment
+// is the A operand and the activation fragment the B operand, so D =
+// (X W^T)^T and each lane ends up with runs of four consecutive output
+// columns of one row: the epilogue stores them as vectors.
 //
 // Bounds: every global read is a buffer load on a per-tile resource, so rows
 // past M or N read as zero in hardware; in the K tail (K % 64 == 32) the X
-// lanes and weight lanes past K are sent out of range by their lane offset
-// (a zero activation times a zero weight).
+// lanes past K are sent out of range by their lane offset (a zero activation
+// times the packet's zero padding).
 #include <climits>
 #include <string>
 #include <utility>
@@ -78,10 +76,10 @@ struct GemmArgs {
     // [z K / ksplit, (z + 1) K / ksplit) into y + z * part_stride.
     int ksplit = 1;
     int64_t part_stride = 0;
-    // gemm32_kernel EPI_F32 with FOLD: K pieces of kfold stages counted
+    // EPI_F32 with FOLD: K pieces of kfold stages counted
     // from the split's first stage; see launch_gemm_splitk.
     int kfold = 0;
-    // gemm32_kernel: row tiles start at BM * i - mshift (0 <= mshift < BM)
+    // EPI_QKPREP: row tiles start at BM * i - mshift (0 <= mshift < BM)
     int64_t mshift = 0;
 };
 
@@ -191,8 +189,7 @@ struct Cfg32 {
     // EPI_QKPREP stages the f32 tile [BM][256] (rows padded to 260
     // floats), eight partial sums of squares and a scale per row in LDS
     // after the K loop.
-    static constexpr int QK_TS = 260;
-    static constexpr int QK_LDS = EPI == EPI_QKPREP ? BM * (QK_TS + 17) * 4 : 0;  // + [BM][16] sums, [BM] scales
+    static constexpr int QK_LDS = EPI == EPI_QKPREP ? BM * (260 + 17) * 4 : 0;  // + [BM][16] sums, [BM] scales
     static constexpr int PAIR_LDS = PAIR ? (NW / 2) * MI * NJ * 16 * WAVE * 4 : 0;  // the gate waves' sums
     static constexpr int EPI_LDS = QK_LDS > PAIR_LDS ? QK_LDS : PAIR_LDS;           // LDS after the K loop
     static constexpr int LDS = NS * X_BYTES > EPI_LDS ? NS * X_BYTES : EPI_LDS;
@@ -204,6 +201,159 @@ struct Cfg32 {
     static_assert(NS >= 3, "ring needs >= 3 slots: one read into registers, one landing, one in flight");
     static_assert(WL + (NS - 2) * C <= 63, "vmcnt range");
 };
+
+// The q/k/v epilogue (EPI_QKPREP) for row blocks C0 .. C0 + RB - 1 of a
+// 256-column tile (one head); m0: the first row of those blocks; qpos: the
+// rope row of each of the thread's rows (row p * NW * 2 + tid / 32 of the
+// blocks at p).
+constexpr int QK_TS = 260;  // floats per staged row
+template <int MI, int NJ, int NW, int C0, int RB>
+__device__ inline void finish_qkprep(const GemmArgs& g, const floatx16 (&acc)[MI][NJ], int64_t m0, int64_t n0,
+                                     uint8_t* smem, int wave, int lane, const int* qpos) {
+    // Every multiply-add that rounds once is an explicit fmaf and every
+    // f16 comes from an f32 value (nothing for the compiler to fuse in
+    // one tile shape and not another): a row's outputs are the same
+    // bits from the four-wave and the eight-wave tile.
+    // qk_prep.wgsl:66-114 on the tile's rows, without cross-lane
+    // traffic: each lane's sums of squares over its 16 accumulators of
+    // a row in each 32-column block go to LDS with the f32 tile (the
+    // ring is free: every DMA landed, every read done); a row's RMS is
+    // the sum of its sixteen partials (block, lane half) in a fixed
+    // order, whichever wave held which block.  q and k heads: 32 threads per row,
+    // thread c holding head dimensions 4c..4c+3 and their RoPE partners
+    // 128 + 4c..: RMS norm with the head's weight, RoPE, query scale,
+    // f16 q rows or k cache rows.  v head: (optional) RMS norm, then
+    // the V^T tiles of the cache in whole 16-byte chunks of 8 keys, 8
+    // lanes per 128-byte dimension row (the caller aligns the row tiles
+    // to 32 cache rows, so every chunk belongs to one tile; at the
+    // pass's edges a chunk keeps the cache's other keys).
+    constexpr int HD = 256, TS = QK_TS, HALF = HD / 2, BM = 32 * RB, WR = 32 * NJ;
+    constexpr int QK_RP = NW * WAVE / 32, QK_PASSES = BM / QK_RP;  // 32 threads per row
+    const int tid = wave * WAVE + lane, lr = lane % 32, lh = lane / 32;
+    const int64_t M = g.m;
+    auto row_ok = [&](int64_t r) { return m0 + r >= 0 && m0 + r < M; };
+    const QkArgs& a = g.qk;
+    float* T = reinterpret_cast<float*>(smem);
+    float* ssp = T + BM * TS;  // [BM][16] partial sums of squares
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                *reinterpret_cast<float4*>(T + (i * 32 + lr) * TS + wave * WR + j * 32 + 8 * q + 4 * lh) =
+                    make_float4(acc[C0 + i][j][4 * q], acc[C0 + i][j][4 * q + 1], acc[C0 + i][j][4 * q + 2], acc[C0 + i][j][4 * q + 3]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ss = fmaf(acc[C0 + i][j][4 * q + r], acc[C0 + i][j][4 * q + r], ss);
+            }
+            ssp[(i * 32 + lr) * 16 + 2 * (wave * NJ + j) + lh] = ss;
+        }
+    const int slot = int(n0 / HD);
+    const int H = a.heads, KV = a.kv_heads;
+    const bool is_v = slot >= H + KV;
+    const int c = tid % 32, d0 = 4 * c;
+    // The rope pairs of every pass now, while the tile is staged.
+    float4 r01[QK_PASSES], r23[QK_PASSES];
+    if (!is_v) {
+#pragma unroll
+        for (int p = 0; p < QK_PASSES; ++p) {
+            const float4* rt = reinterpret_cast<const float4*>(a.rope + int64_t(qpos[p]) * HALF + d0);
+            r01[p] = rt[0];
+            r23[p] = rt[1];
+        }
+    }
+    lds_barrier();
+    // Each row's scale once, from the sum of its sixteen partials in
+    // order; the passes below read it.
+    float* rinv = ssp + BM * 16;  // [BM] row scales
+    if (tid < BM) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) ss += ssp[tid * 16 + k];
+        rinv[tid] = 1.0f / sqrtf(ss / float(HD) + a.eps);
+    }
+    lds_barrier();
+    if (!is_v) {
+        const bool is_q = slot < H;
+        const int head = is_q ? slot : slot - H;
+        const float* wn = is_q ? a.q_norm : a.k_norm;
+        const float4 wl = *reinterpret_cast<const float4*>(wn + d0), wh = *reinterpret_cast<const float4*>(wn + HALF + d0);
+        const float w_lo[4] = {wl.x, wl.y, wl.z, wl.w}, w_hi[4] = {wh.x, wh.y, wh.z, wh.w};
+        const float sc = is_q ? a.q_scale : 1.0f;
+        const int rot = int(a.rope_dims / 2);
+#pragma unroll
+        for (int p = 0; p < QK_PASSES; ++p) {
+            const int r = p * QK_RP + tid / 32;
+            if (!row_ok(r)) continue;
+            const float inv = rinv[r];
+            const float4 vl = *reinterpret_cast<const float4*>(T + r * TS + d0);
+            const float4 vh = *reinterpret_cast<const float4*>(T + r * TS + HALF + d0);
+            const float v_lo[4] = {vl.x, vl.y, vl.z, vl.w}, v_hi[4] = {vh.x, vh.y, vh.z, vh.w};
+            const float cs[4] = {r01[p].x, r01[p].z, r23[p].x, r23[p].z};
+            const float sn[4] = {r01[p].y, r01[p].w, r23[p].y, r23[p].w};
+            float o_lo[4], o_hi[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float y0 = v_lo[k] * inv * w_lo[k], y1 = v_hi[k] * inv * w_hi[k];
+                if (d0 + k < rot) {
+                    o_lo[k] = fmaf(y0, cs[k], -(y1 * sn[k]));
+                    o_hi[k] = fmaf(y1, cs[k], y0 * sn[k]);
+                } else {
+                    o_lo[k] = y0;
+                    o_hi[k] = y1;
+                }
+            }
+            const int64_t tok = m0 + r, row = a.base + tok;
+            half_t* dst = is_q ? a.q16 + (tok * H + head) * HD : a.kc + (int64_t(head) * a.cap_pad + row) * HD;
+            *reinterpret_cast<half4*>(dst + d0) =
+                half4{f16_rounded(o_lo[0] * sc), f16_rounded(o_lo[1] * sc), f16_rounded(o_lo[2] * sc),
+                      f16_rounded(o_lo[3] * sc)};
+            *reinterpret_cast<half4*>(dst + HALF + d0) =
+                half4{f16_rounded(o_hi[0] * sc), f16_rounded(o_hi[1] * sc), f16_rounded(o_hi[2] * sc),
+                      f16_rounded(o_hi[3] * sc)};
+        }
+        return;
+    }
+    // V head: per 32-key half of the tile, item (dim, chunk cc) for
+    // 256 dims x 4 chunks; chunk 4 hf + cc of a 64-key cache tile holds
+    // keys 32 hf + 4 cc + {0..3, 16..19} (vt_col).
+    const int head = slot - H - KV;
+#pragma unroll
+    for (int hh = 0; hh < BM / 32; ++hh) {
+        const int64_t kh = a.base + m0 + 32 * hh;  // first cache row of this half (a multiple of 32)
+        if (m0 + 32 * hh + 32 <= 0 || m0 + 32 * hh >= M) continue;
+        const int64_t t0 = kh / 64 * 64;
+        const int hf = int((kh % 64) / 32);
+#pragma unroll
+        for (int u = 0; u < 1024 / (NW * WAVE); ++u) {
+            const int item = tid + NW * WAVE * u;
+            const int dim = item / 4, cc = item % 4;
+            half_t* dst = a.vt + ((int64_t(head) * (a.cap_pad / 64) + t0 / 64) * HD + dim) * 64 + 8 * (4 * hf + cc);
+            half_t h[8];
+            bool all = true;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int r = 32 * hh + 4 * cc + 16 * (e / 4) + e % 4;  // tile row of key e
+                const bool in = row_ok(r);
+                all = all && in;
+                const float v = T[r * TS + dim];
+                h[e] = f16_rounded(a.v_norm ? v * rinv[r] : v);
+            }
+            if (!all) {
+                // a pass edge: the chunk's other keys keep the cache's values
+                const half8 old = *reinterpret_cast<const half8*>(dst);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int r = 32 * hh + 4 * cc + 16 * (e / 4) + e % 4;
+                    if (!row_ok(r)) h[e] = old[e];
+                }
+            }
+            *reinterpret_cast<half8*>(dst) = half8{h[0], h[1], h[2], h[3], h[4], h[5], h[6], h[7]};
+        }
+    }
+}
 
 // A pair of four-value f16 groups, columns c .. c + 3 in lanes l < 32 and
 // c + 4 .. c + 7 in lanes l + 32 for group a (c) and group b (c + 8), turned
@@ -409,9 +559,10 @@ __global__ __launch_bounds__(NW_ * WAVE) void gemm32_kernel(GemmArgs g) {
     const int tid = int(threadIdx.x), lane = tid % WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
 
-    // XCD-aware tile order (see gemm_kernel).  Row tiles start at
-    // BM * i - mshift (mshift < BM: the first tile is short), so a caller
-    // can align the tiles to its own row grid.
+    // XCD-aware tile order: workgroups reach the eight XCDs in turn, so each
+    // XCD is given a contiguous run of tiles (which share rows in its L2).
+    // Row tiles start at BM * i - mshift (mshift < BM: the first tile is
+    // short), so a caller can align the tiles to its own row grid.
     const int64_t N = g.w0.rows, K = g.w0.cols, M = g.m;
     const int ntn = int((N + BN - 1) / BN);
     const int ntiles = ntn * int((M + g.mshift + BM - 1) / BM);
@@ -667,145 +818,7 @@ __global__ __launch_bounds__(NW_ * WAVE) void gemm32_kernel(GemmArgs g) {
     }
 
     if constexpr (EPI == EPI_QKPREP) {
-        // Every multiply-add that rounds once is an explicit fmaf and every
-        // f16 comes from an f32 value (nothing for the compiler to fuse in
-        // one tile shape and not another): a row's outputs are the same
-        // bits from the four-wave and the eight-wave tile.
-        // qk_prep.wgsl:66-114 on the tile's rows, without cross-lane
-        // traffic: each lane's sums of squares over its 16 accumulators of
-        // a row in each 32-column block go to LDS with the f32 tile (the
-        // ring is free: every DMA landed, every read done); a row's RMS is
-        // the sum of its sixteen partials (block, lane half) in a fixed
-        // order, whichever wave held which block.  q and k heads: 32 threads per row,
-        // thread c holding head dimensions 4c..4c+3 and their RoPE partners
-        // 128 + 4c..: RMS norm with the head's weight, RoPE, query scale,
-        // f16 q rows or k cache rows.  v head: (optional) RMS norm, then
-        // the V^T tiles of the cache in whole 16-byte chunks of 8 keys, 8
-        // lanes per 128-byte dimension row (the caller aligns the row tiles
-        // to 32 cache rows, so every chunk belongs to one tile; at the
-        // pass's edges a chunk keeps the cache's other keys).
-        constexpr int HD = 256, TS = P::QK_TS, HALF = HD / 2;
-        const QkArgs& a = g.qk;
-        float* T = reinterpret_cast<float*>(smem);
-        float* ssp = T + BM * TS;  // [BM][16] partial sums of squares
-        lds_barrier();
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                float ss = 0.0f;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    *reinterpret_cast<float4*>(T + (i * 32 + lr) * TS + wave * WR + j * 32 + 8 * q + 4 * lh) =
-                        make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) ss = fmaf(acc[i][j][4 * q + r], acc[i][j][4 * q + r], ss);
-                }
-                ssp[(i * 32 + lr) * 16 + 2 * (wave * NJ + j) + lh] = ss;
-            }
-        const int slot = int(n0 / HD);
-        const int H = a.heads, KV = a.kv_heads;
-        const bool is_v = slot >= H + KV;
-        const int c = tid % 32, d0 = 4 * c;
-        // The rope pairs of every pass now, while the tile is staged.
-        float4 r01[QK_PASSES], r23[QK_PASSES];
-        if (!is_v) {
-#pragma unroll
-            for (int p = 0; p < QK_PASSES; ++p) {
-                const float4* rt = reinterpret_cast<const float4*>(a.rope + int64_t(qpos[p]) * HALF + d0);
-                r01[p] = rt[0];
-                r23[p] = rt[1];
-            }
-        }
-        lds_barrier();
-        // Each row's scale once, from the sum of its sixteen partials in
-        // order; the passes below read it.
-        float* rinv = ssp + BM * 16;  // [BM] row scales
-        if (tid < BM) {
-            float ss = 0.0f;
-#pragma unroll
-            for (int k = 0; k < 16; ++k) ss += ssp[tid * 16 + k];
-            rinv[tid] = 1.0f / sqrtf(ss / float(HD) + a.eps);
-        }
-        lds_barrier();
-        if (!is_v) {
-            const bool is_q = slot < H;
-            const int head = is_q ? slot : slot - H;
-            const float* wn = is_q ? a.q_norm : a.k_norm;
-            const float4 wl = *reinterpret_cast<const float4*>(wn + d0), wh = *reinterpret_cast<const float4*>(wn + HALF + d0);
-            const float w_lo[4] = {wl.x, wl.y, wl.z, wl.w}, w_hi[4] = {wh.x, wh.y, wh.z, wh.w};
-            const float sc = is_q ? a.q_scale : 1.0f;
-            const int rot = int(a.rope_dims / 2);
-#pragma unroll
-            for (int p = 0; p < QK_PASSES; ++p) {
-                const int r = p * QK_RP + tid / 32;
-                if (!row_ok(r)) continue;
-                const float inv = rinv[r];
-                const float4 vl = *reinterpret_cast<const float4*>(T + r * TS + d0);
-                const float4 vh = *reinterpret_cast<const float4*>(T + r * TS + HALF + d0);
-                const float v_lo[4] = {vl.x, vl.y, vl.z, vl.w}, v_hi[4] = {vh.x, vh.y, vh.z, vh.w};
-                const float cs[4] = {r01[p].x, r01[p].z, r23[p].x, r23[p].z};
-                const float sn[4] = {r01[p].y, r01[p].w, r23[p].y, r23[p].w};
-                float o_lo[4], o_hi[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const float y0 = v_lo[k] * inv * w_lo[k], y1 = v_hi[k] * inv * w_hi[k];
-                    if (d0 + k < rot) {
-                        o_lo[k] = fmaf(y0, cs[k], -(y1 * sn[k]));
-                        o_hi[k] = fmaf(y1, cs[k], y0 * sn[k]);
-                    } else {
-                        o_lo[k] = y0;
-                        o_hi[k] = y1;
-                    }
-                }
-                const int64_t tok = m0 + r, row = a.base + tok;
-                half_t* dst = is_q ? a.q16 + (tok * H + head) * HD : a.kc + (int64_t(head) * a.cap_pad + row) * HD;
-                *reinterpret_cast<half4*>(dst + d0) =
-                    half4{f16_rounded(o_lo[0] * sc), f16_rounded(o_lo[1] * sc), f16_rounded(o_lo[2] * sc),
-                          f16_rounded(o_lo[3] * sc)};
-                *reinterpret_cast<half4*>(dst + HALF + d0) =
-                    half4{f16_rounded(o_hi[0] * sc), f16_rounded(o_hi[1] * sc), f16_rounded(o_hi[2] * sc),
-                          f16_rounded(o_hi[3] * sc)};
-            }
-            return;
-        }
-        // V head: per 32-key half of the tile, item (dim, chunk cc) for
-        // 256 dims x 4 chunks; chunk 4 hf + cc of a 64-key cache tile holds
-        // keys 32 hf + 4 cc + {0..3, 16..19} (vt_col).
-        const int head = slot - H - KV;
-#pragma unroll
-        for (int hh = 0; hh < BM / 32; ++hh) {
-            const int64_t kh = a.base + m0 + 32 * hh;  // first cache row of this half (a multiple of 32)
-            if (m0 + 32 * hh + 32 <= 0 || m0 + 32 * hh >= M) continue;
-            const int64_t t0 = kh / 64 * 64;
-            const int hf = int((kh % 64) / 32);
-#pragma unroll
-            for (int u = 0; u < 1024 / (NW * WAVE); ++u) {
-                const int item = tid + NW * WAVE * u;
-                const int dim = item / 4, cc = item % 4;
-                half_t* dst = a.vt + ((int64_t(head) * (a.cap_pad / 64) + t0 / 64) * HD + dim) * 64 + 8 * (4 * hf + cc);
-                half_t h[8];
-                bool all = true;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int r = 32 * hh + 4 * cc + 16 * (e / 4) + e % 4;  // tile row of key e
-                    const bool in = row_ok(r);
-                    all = all && in;
-                    const float v = T[r * TS + dim];
-                    h[e] = f16_rounded(a.v_norm ? v * rinv[r] : v);
-                }
-                if (!all) {
-                    // a pass edge: the chunk's other keys keep the cache's values
-                    const half8 old = *reinterpret_cast<const half8*>(dst);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int r = 32 * hh + 4 * cc + 16 * (e / 4) + e % 4;
-                        if (!row_ok(r)) h[e] = old[e];
-                    }
-                }
-                *reinterpret_cast<half8*>(dst) = half8{h[0], h[1], h[2], h[3], h[4], h[5], h[6], h[7]};
-            }
-        }
+        finish_qkprep<MI, NJ, NW, 0, MI>(g, acc, m0, n0, smem, wave, lane, qpos);
         return;
     }
 
@@ -850,7 +863,7 @@ __global__ __launch_bounds__(NW_ * WAVE) void gemm32_kernel(GemmArgs g) {
 //   kt + 1 after a wait for its X DMA and a barrier, which also frees stage
 //   kt's ring slot: the DMA of stage kt + NS goes out), between the MFMAs
 //   of this one; after the last decode, load stage kt + 2's weights.
-template <int QUANT, int MI, int NJ, int EPI, int NS, int NW_>
+template <int QUANT, int MI, int NJ, int EPI, int NS, int NW_, bool FOLD>
 __global__ __launch_bounds__(NW_ * WAVE, 2) void gemm32w_kernel(GemmArgs g) {
     using P = Cfg32<QUANT, MI, NJ, EPI, NS, NW_, false>;
     constexpr bool GATED = P::GATED;
@@ -860,11 +873,11 @@ __global__ __launch_bounds__(NW_ * WAVE, 2) void gemm32w_kernel(GemmArgs g) {
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int64_t N = g.w0.rows, K = g.w0.cols, M = g.m;
     const int ntn = int((N + BN - 1) / BN);
-    const int ntiles = ntn * int((M + BM - 1) / BM);
+    const int ntiles = ntn * int((M + g.mshift + BM - 1) / BM);
     const int per_xcd = int(gridDim.x) / 8;
     const int tile = (int(blockIdx.x) % 8) * per_xcd + int(blockIdx.x) / 8;
     if (tile >= ntiles) return;
-    const int64_t n0 = int64_t(tile % ntn) * BN, m0 = int64_t(tile / ntn) * BM;
+    const int64_t n0 = int64_t(tile % ntn) * BN, m0 = int64_t(tile / ntn) * BM - g.mshift;
     const int kbeg = int(blockIdx.y) * int(K / g.ksplit);
     const int nk = int((K / g.ksplit + G_BK - 1) / G_BK);
     const int K32 = int(K), last = nk - 1;
@@ -876,7 +889,7 @@ __global__ __launch_bounds__(NW_ * WAVE, 2) void gemm32w_kernel(GemmArgs g) {
         const int slot = (i * NW + wave) * WAVE + lane;
         const int r = slot / 8, lc = (slot % 8) ^ swz(r);
         xcol[i] = lc * 8;
-        xoff[i] = slot < P::X_CH && m0 + r < M ? uint32_t(((m0 + r) * g.ldx + lc * 8) * 2) : OOB;
+        xoff[i] = slot < P::X_CH && m0 + r >= 0 && m0 + r < M ? uint32_t(((m0 + r) * g.ldx + lc * 8) * 2) : OOB;
     }
     const int64_t stages = g.w0.stages, rblocks = (N + 31) / 32, rb0 = n0 / 32;
     const int64_t live_blocks = rblocks - rb0;
@@ -934,6 +947,21 @@ __global__ __launch_bounds__(NW_ * WAVE, 2) void gemm32w_kernel(GemmArgs g) {
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = floatx16{};
+    // FOLD: K pieces of g.kfold stages from zero, added in K order (as in
+    // gemm32_kernel).
+    floatx16 tot[FOLD ? MI : 1][FOLD ? NJ : 1];
+    bool folded = false;
+    int kleft = g.kfold;
+    auto fold = [&] {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                tot[i][j] = folded ? tot[i][j] + acc[i][j] : acc[i][j];
+                acc[i][j] = floatx16{};
+            }
+        folded = true;
+    };
     const int lr = lane % 32, lh = lane / 32;
     int foff[4];
 #pragma unroll
@@ -1026,6 +1054,12 @@ __global__ __launch_bounds__(NW_ * WAVE, 2) void gemm32w_kernel(GemmArgs g) {
         __builtin_amdgcn_sched_barrier(0);
         kstep(nw, kt + 1, 0, fb, fa);
         ++kt;
+        if constexpr (FOLD) {
+            if (--kleft == 0 || kt == nk) {
+                kleft = g.kfold;
+                fold();
+            }
+        }
     };
     // (Two stages per iteration and no exit between them: with one, the
     // compiler's wait counts have to hold on a path that skips a stage.)
@@ -1035,7 +1069,27 @@ __global__ __launch_bounds__(NW_ * WAVE, 2) void gemm32w_kernel(GemmArgs g) {
     }
     if (nk & 1) step(std::integral_constant<int, 0>{});
     wait_vm<0>();
-    finish32<MI, NJ, EPI, true>(g, acc, m0, n0 + (GATED ? wave * (WR / 2) : wave * WR), lane);
+    if constexpr (EPI == EPI_QKPREP) {
+        // One 32-row block at a time: the staged tile then fits the ring.
+        auto block = [&](auto c) {
+            constexpr int C = decltype(c)::value;
+            int pos[4];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const int64_t r = m0 + 32 * C + 8 * p + tid / 32;
+                const int v = g.qk.meta[4 * (g.qk.base + (r < 0 ? 0 : (r < M ? r : M - 1)))];
+                pos[p] = v < 0 ? 0 : (v >= g.qk.rope_rows ? int(g.qk.rope_rows - 1) : v);
+            }
+            finish_qkprep<MI, NJ, NW, C, 1>(g, acc, m0 + 32 * C, n0, smem, wave, lane, pos);
+            return true;
+        };
+        run_phases(block, std::make_index_sequence<MI>{});
+    } else {
+        if constexpr (FOLD)
+            finish32<MI, NJ, EPI, true>(g, tot, m0, n0 + wave * WR, lane);
+        else
+            finish32<MI, NJ, EPI, true>(g, acc, m0, n0 + (GATED ? wave * (WR / 2) : wave * WR), lane);
+    }
 }
 
 // Resident X tiles up to this many bytes of LDS (one workgroup per CU
@@ -1073,52 +1127,58 @@ static void run32(hipStream_t s, const GemmArgs& g) {
     OMG_HIP(hipGetLastError());
 }
 
-template <int QUANT, int MI, int NJ, int EPI, int NS, int NW = 4>
+template <int QUANT, int MI, int NJ, int EPI, int NS, int NW = 4, bool FOLD = false>
 static void run32w(hipStream_t s, const GemmArgs& g) {
+    static_assert(!FOLD || EPI == EPI_F32, "K pieces: f32 products only");
     using P = Cfg32<QUANT, MI, NJ, EPI, NS, NW, false>;
     for (const DevWeight* w : {&g.w0, &g.w1})
         if (!w->tiles || w->stages != (w->cols + G_BK - 1) / G_BK || (QUANT != F16_DT && !w->tscales))
             fail(E_INVALID, "gemm: weight without stage tiles");
+    constexpr int QK = EPI == EPI_QKPREP ? 32 * (QK_TS + 17) * 4 : 0, RING = NS * P::X_BYTES;
+    constexpr int LDS = QK > RING ? QK : RING;
     static bool lds_set = false;
     if (!lds_set) {
-        OMG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm32w_kernel<QUANT, MI, NJ, EPI, NS, NW>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, P::LDS));
+        OMG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm32w_kernel<QUANT, MI, NJ, EPI, NS, NW, FOLD>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
         lds_set = true;
     }
-    if (g.mshift != 0 || g.kfold != 0) fail(E_INVALID, "gemm: wide tiles take no row shift or K pieces");
-    const int64_t tiles = ((g.w0.rows + P::BN - 1) / P::BN) * ((g.m + P::BM - 1) / P::BM);
+    if (FOLD != (g.kfold > 0)) fail(E_INVALID, "gemm: K pieces");
+    const int64_t tiles = ((g.w0.rows + P::BN - 1) / P::BN) * ((g.m + g.mshift + P::BM - 1) / P::BM);
     const dim3 grid(unsigned((tiles + 7) / 8 * 8), unsigned(g.ksplit));
-    gemm32w_kernel<QUANT, MI, NJ, EPI, NS, NW><<<grid, dim3(P::T), P::LDS, s>>>(g);
+    gemm32w_kernel<QUANT, MI, NJ, EPI, NS, NW, FOLD><<<grid, dim3(P::T), LDS, s>>>(g);
     OMG_HIP(hipGetLastError());
 }
 
-// Row blocks (of 32) of the wide tile: a workgroup of MI blocks takes about
-// 1 + MI units of time whatever the product, and 256 CUs run a round of
-// tiles at a time, so the MI with the least rounds x (1 + MI) is taken (the
-// larger of equals: less decode and weight traffic).  Measured over 19
-// shapes from 300 to 49,152 rows, K 640 to 2,560, it picks the fastest MI
-// or one within 3% of it; f16 weights take twice the registers of Q8 ones
-// and stop at three blocks.
-template <int QUANT>
+// Row blocks (of 32) of the wide tile, at least LO: a workgroup of MI blocks
+// takes about 1 + MI units of time whatever the product, and ROUND tiles run
+// at a time, so the MI with the least rounds x (1 + MI) is taken (the larger
+// of equals: less decode and weight traffic).  With 256 to a round it picks
+// the fastest MI or one within 3% of it over 19 shapes from 300 to 49,152
+// rows, K 640 to 2,560; the q/k/v tile, whose epilogue of one workgroup runs
+// beside the K loop of the next on its CU, fits 512 (eight passes of 930 to
+// 16,320 rows, K 1,152 to 2,560).  f16 weights take twice the registers of
+// Q8 ones and stop at three blocks.
+template <int QUANT, int LO, int ROUND>
 static int wide_blocks(int64_t m, int64_t ntn) {
-    int best = 1;
+    int best = LO;
     int64_t cost = INT64_MAX;
-    for (int mi = QUANT == F16_DT ? 3 : 4; mi >= 1; --mi) {
-        const int64_t tiles = (m + 32 * mi - 1) / (32 * mi) * ntn, c = (tiles + 255) / 256 * (1 + mi);
+    for (int mi = QUANT == F16_DT ? 3 : 4; mi >= LO; --mi) {
+        const int64_t tiles = (m + 32 * mi - 1) / (32 * mi) * ntn, c = (tiles + ROUND - 1) / ROUND * (1 + mi);
         if (c < cost) cost = c, best = mi;
     }
     return best;
 }
 
 // 32 MI rows x 256 weight rows on four waves.
-template <int QUANT, int EPI>
+template <int QUANT, int EPI, int LO = 1, int ROUND = 256>
 static void run_wide(hipStream_t s, const GemmArgs& g, int64_t cols_per_tile) {
-    const int mi = wide_blocks<QUANT>(g.m, (g.w0.rows + cols_per_tile - 1) / cols_per_tile * g.ksplit);
+    const int mi = wide_blocks<QUANT, LO, ROUND>(g.m, (g.w0.rows + cols_per_tile - 1) / cols_per_tile * g.ksplit);
     if constexpr (QUANT != F16_DT)
         if (mi == 4) return run32w<QUANT, 4, 2, EPI, 3, 4>(s, g);
     if (mi == 3) return run32w<QUANT, 3, 2, EPI, 3, 4>(s, g);
-    if (mi == 2) return run32w<QUANT, 2, 2, EPI, 4, 4>(s, g);
-    return run32w<QUANT, 1, 2, EPI, 4, 4>(s, g);
+    if constexpr (LO == 1)
+        if (mi == 1) return run32w<QUANT, 1, 2, EPI, 4, 4>(s, g);
+    return run32w<QUANT, 2, 2, EPI, 4, 4>(s, g);
 }
 
 // Tile choice, measured on MI355X (tiles are activation rows x weight rows;
@@ -1150,16 +1210,23 @@ static void dispatch(hipStream_t s, const GemmArgs& g) {
         // One head on eight waves of one 32-row weight block each (half the
         // decode per wave and K stage of the four-wave tile): short passes,
         // and long ones whose 64-row X tile stays resident (K <= 768; the
-        // 270M model's cold q/k/v 15.9 -> 13.3 us, its cold pass -3.2%); at
-        // K 2,560 (the 4B model) eight waves through the ring were slower
-        // (396 -> 522 us a launch) than four of two blocks each.
+        // 270M model's cold q/k/v 15.9 -> 13.3 us, its cold pass -3.2%).
+        // Longer K: wide tiles against 64 rows on four waves of the short
+        // stages, 4B model (K 2,560), 16,320 rows 388 -> 337 us, 8,800 217
+        // -> 198, 4,100 118 -> 105, 1,980 55.0 -> 55.8; 1B (K 1,152), 2,352
+        // rows 23.7 -> 24.1, 992 21.5 -> 19.6.
         if (M <= 512) return run32<QUANT, 1, 1, EPI, 4, 8>(s, g);
         if (K <= 768) return run32<QUANT, 2, 1, EPI, 4, 8>(s, g);
-        return run32<QUANT, 2, 2, EPI, 4, 4>(s, g);
+        return run_wide<QUANT, EPI, 2, 512>(s, g, 256);
     } else if constexpr (EPI == EPI_F32) {
-        if (g.kfold > 0) {  // K pieces added in registers (up to 96-row tiles: the totals fit)
+        if (g.kfold > 0) {
+            // K pieces added in registers (up to 96-row tiles: the totals
+            // fit).  96 rows of the wide kernel against the short stages, 4B
+            // down (N 2,560, K 10,240): 16,320 rows 935 -> 896 us, 8,800 531
+            // -> 512, 3,000 214 -> 192, 1,980 133 -> 137; 128 rows were 884,
+            // 515, 180 and 153.
             if (M <= 512) return run32<QUANT, 1, 1, EPI, 4, 4, true>(s, g);
-            return run32<QUANT, 3, 1, EPI, 4, 4, true>(s, g);
+            return run32w<QUANT, 3, 1, EPI, 3, 4, true>(s, g);
         }
         if (M <= 512 && tiles(32, 128) <= 512) return run32<QUANT, 1, 1, EPI, 4, 4>(s, g);
         if (g.ksplit > 1 && tiles(96, 128) <= 256) return run32<QUANT, 3, 1, EPI, 4, 4>(s, g);

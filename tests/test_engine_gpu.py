@@ -511,6 +511,35 @@ def test_long_groups_bit_equal_to_separate_passes(heads, kv):
                 assert np.array_equal(r, s), f"group {i}"
 
 
+@pytest.mark.parametrize("rows,d,linear", [(1190, 800, "Q4"), (2390, 832, "Q8"), (2390, 800, "F16"), (2890, 832, "Q4"),
+                                           (2890, 800, "Q8")])
+def test_wide_qkv_tiles_bit_equal_to_short_passes(rows, d, linear):
+    """The q/k/v product with K > 768 in passes of 64-, 96- and 128-row
+    wide tiles (20 head slots: 1,190, 2,390 and 2,890 rows; K 800 ends in
+    half a stage), behind a resident prefix of odd length, so that the tiles
+    start before the pass: every group's rows are bit-equal to its rows
+    alone, in passes of at most 512 rows on the eight-wave tile."""
+    rng = np.random.default_rng(rows + d)
+    cfg = gguf_tiny(16, 2, window=90, d=d)
+    eng, _, _, _ = build(cfg, 43, getattr(g, linear), g.Q8, capacity=3072, oracle_models=False)
+    sizes = [500] * (rows // 500) + [rows % 500]
+    groups = [Group([2, 5, 9], [BranchTokens([7, 8], [1])])]
+    groups += [Group(rng.integers(0, 64, n - 31).tolist(), [BranchTokens(rng.integers(0, 64, 31).tolist(), [0, 30])])
+               for n in sizes]
+    alone = []
+    for gr in groups:
+        eng.evict_resident()
+        alone.append(eng.evaluate(gr.prefix, gr.branches, Want.HIDDEN))
+    eng.evict_resident()
+    eng.evaluate(groups[0].prefix, groups[0].branches, Want.HIDDEN)  # resident: base 3
+    together = eng.evaluate_groups(groups, Want.HIDDEN)
+    assert together[0].prefix_source == PrefixSource.RESIDENT
+    for i, (a, t) in enumerate(zip(alone, together)):
+        for x, y in zip(a, t.branches):
+            for r, s in zip(x.rows, y.rows):
+                assert np.array_equal(r, s), f"group {i}"
+
+
 def test_graph_replay_matches_eager_pass():
     """omg_pass_graph: the prepared pass captured once and replayed gives
     the eager launch's rows bit for bit on every replay, with other eager
