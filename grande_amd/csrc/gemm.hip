@@ -545,6 +545,23 @@ __device__ inline bool run_phases(F& f, std::index_sequence<I...>) {
     return (f(std::integral_constant<int, int(I)>{}) && ...);
 }
 
+template <class F, size_t... I>
+__device__ inline void run_all(F& f, std::index_sequence<I...>) {
+    (f(std::integral_constant<int, int(I)>{}), ...);
+}
+
+// f(phase) for nk stages, phase = stage % U; f returns whether a stage is
+// left.  Whole groups of U without an exit among them, then the rest: with
+// an exit after every stage the compiler gave the loop one latch for all of
+// them, could no longer tell which stages' loads were out at the loop head,
+// and waited there for nearly all of them (vmcnt 0 to 4), once every U
+// stages.
+template <int U, class F>
+__device__ inline void run_stages(F& f, int nk) {
+    for (int n = nk / U; n > 0; --n) run_all(f, std::make_index_sequence<U>{});
+    if (nk % U) run_phases(f, std::make_index_sequence<U>{});
+}
+
 // XR (resident X): the workgroup's whole X tile (BM rows x its K range)
 // lands in LDS in the prologue, one slot per stage, and the K loop runs
 // with no barrier and no X wait (the weights are each wave's own).  Same
@@ -720,25 +737,34 @@ __global__ __launch_bounds__(NW_ * WAVE) void gemm32_kernel(GemmArgs g) {
 
     // EPI_QKPREP, q and k heads: the rope rows of the rows this thread
     // finishes (RP rows per pass of the workgroup, row p * RP + tid / 32),
-    // loaded now so their latency hides behind the K loop.
+    // loaded now so their latency hides behind the K loop.  Every thread
+    // loads the position of a row of the pass (its own row, clamped into the
+    // pass); rows outside the pass and the v head take position 0 in
+    // clamp_pos, once the first stages have landed: with the choice made
+    // here the compiler put each load in a branch of its own with its wait.
     constexpr int QK_RP = NW * WAVE / 32;  // rows per pass: 32 threads per row
     constexpr int QK_PASSES = EPI == EPI_QKPREP ? BM / QK_RP : 1;
     int qpos[QK_PASSES];
     if constexpr (EPI == EPI_QKPREP) {
-        const QkArgs& a = g.qk;
-        const bool qk_head = n0 / 256 < a.heads + a.kv_heads;
 #pragma unroll
         for (int p = 0; p < QK_PASSES; ++p) {
-            // Every thread loads the position of a row of the pass (its own
-            // row, clamped into the pass), so the loads go out back to back
-            // with no branch between them; rows outside the pass and the v
-            // head take position 0.
             const int r = p * QK_RP + tid / 32;
             const int64_t m = m0 + r < 0 ? 0 : (m0 + r < M ? m0 + r : M - 1);
-            const int pos = a.meta[4 * (a.base + m)];
-            qpos[p] = qk_head && row_ok(r) ? (pos < 0 ? 0 : (pos >= a.rope_rows ? int(a.rope_rows - 1) : pos)) : 0;
+            qpos[p] = g.qk.meta[4 * (g.qk.base + m)];
         }
     }
+    auto clamp_pos = [&] {
+        if constexpr (EPI == EPI_QKPREP) {
+            const bool qk_head = n0 / 256 < g.qk.heads + g.qk.kv_heads;
+#pragma unroll
+            for (int p = 0; p < QK_PASSES; ++p) asm volatile("" : "+v"(qpos[p]));
+#pragma unroll
+            for (int p = 0; p < QK_PASSES; ++p) {
+                const int v = qpos[p] < 0 ? 0 : (qpos[p] >= g.qk.rope_rows ? int(g.qk.rope_rows - 1) : qpos[p]);
+                qpos[p] = qk_head && row_ok(p * QK_RP + tid / 32) ? v : 0;
+            }
+        }
+    };
 
     WRegs wr[R];
     XRegs xa, xb;
@@ -750,6 +776,7 @@ __global__ __launch_bounds__(NW_ * WAVE) void gemm32_kernel(GemmArgs g) {
 #pragma unroll
         for (int s = 0; s < R; ++s) issue_w(s, wr[s]);
         wait_vm<0>();
+        clamp_pos();
         lds_barrier();
         read_x(0, xa);
         auto xstep = [&](auto phase) {
@@ -770,8 +797,7 @@ __global__ __launch_bounds__(NW_ * WAVE) void gemm32_kernel(GemmArgs g) {
             }
             return ++kt < nk;
         };
-        while (run_phases(xstep, std::make_index_sequence<P::U>{})) {
-        }
+        run_stages<P::U>(xstep, nk);
     }
     // Prologue: stages 0 .. NS - 2 in the same order as the loop issues
     // them (X, then weights), then stage 0's X fragments.
@@ -782,6 +808,7 @@ __global__ __launch_bounds__(NW_ * WAVE) void gemm32_kernel(GemmArgs g) {
         issue_w(s, wr[s]);
     }
     wait_vm<P::WL + (NS - 2) * P::C>();
+    clamp_pos();
     lds_barrier();
     read_x(0, xa);
     }
@@ -806,8 +833,7 @@ __global__ __launch_bounds__(NW_ * WAVE) void gemm32_kernel(GemmArgs g) {
         return ++kt < nk;
     };
     if constexpr (!XR) {
-        while (run_phases(step, std::make_index_sequence<P::U>{})) {
-        }
+        run_stages<P::U>(step, nk);
     }
     wait_vm<0>();
     if constexpr (FOLD) {
