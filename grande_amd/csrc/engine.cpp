@@ -489,9 +489,13 @@ Packed Engine::pack_checked(const GroupIn* groups, int64_t n, int64_t first, boo
     if (int64_t(pk.wanted.size()) > max_rows_)
         fail(E_CAPACITY, std::to_string(pk.wanted.size()) + " rows requested, engine reads back at most " +
                              std::to_string(max_rows_));
-    for (uint32_t id : pk.ids)
+    uint32_t top = 0;  // one branch-free pass; the first offender only when there is one
+    for (uint32_t id : pk.ids) top = std::max(top, id);
+    for (uint32_t id : pk.ids) {
+        if (int64_t(top) < cfg_.vocab) break;
         if (int64_t(id) >= cfg_.vocab)
             fail(E_INVALID, "token id " + std::to_string(id) + " outside the vocabulary of " + std::to_string(cfg_.vocab));
+    }
     return pk;
 }
 

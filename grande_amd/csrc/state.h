@@ -50,7 +50,7 @@ Packed pack_groups(const GroupIn* groups, int64_t n, int64_t first, bool residen
 // query belongs to, so nothing sees them).  Wanted and decoded rows move
 // with their groups.  Returns the packing unchanged when the padded pass
 // would need more than `rows` cache rows.
-Packed align_groups(const Packed& pk, int64_t align, int64_t rows);
+Packed align_groups(Packed pk, int64_t align, int64_t rows);
 
 // engine.rs:503-580: a prefix's K/V rows as f16 per layer that owns K/V.
 struct SavedState {

@@ -14,6 +14,7 @@ from __future__ import annotations
 import ctypes as C
 import itertools
 import enum
+from array import array
 from dataclasses import dataclass, field
 from pathlib import Path
 from typing import Sequence
@@ -160,8 +161,17 @@ class GroupOutput:
     prefix_source: PrefixSource
 
 
+_U32 = np.dtype(np.uint32)
+
+
 def _u32(xs) -> np.ndarray:
+    if isinstance(xs, np.ndarray) and xs.dtype == _U32:
+        return np.ascontiguousarray(xs)
     return np.ascontiguousarray(np.asarray(xs, dtype=np.int64).astype(np.uint32))
+
+
+_SHARED_ROWS_BYTES = 4 << 20
+_BRANCH_P = C.POINTER(L.omg_branch)
 
 
 class _CGroups:
@@ -177,20 +187,20 @@ class _CGroups:
         for gi, g in enumerate(groups):
             p = _u32(g.prefix)
             nb = len(g.branches)
-            br = (L.omg_branch * max(1, nb))()
             nt = [len(b.tokens) for b in g.branches]
             nw = [len(b.want) for b in g.branches]
             t = _u32_joined([b.tokens for b in g.branches], sum(nt))
             w = _u32_joined([b.want for b in g.branches], sum(nw))
-            ta, wa = _addr(t), _addr(w)
-            for bi in range(nb):
-                c = br[bi]
-                c.tokens, c.ntokens, c.want, c.nwant = ta, nt[bi], wa, nw[bi]
-                ta += 4 * nt[bi]
-                wa += 4 * nw[bi]
+            flat, ta, wa = [], _addr(t), _addr(w)
+            for n, m in zip(nt, nw):
+                flat += (ta, n, wa, m)  # omg_branch: tokens, ntokens, want, nwant
+                ta += 4 * n
+                wa += 4 * m
+            br = array("Q", flat or [0])
             self.keep += [p, t, w, br]
             a = self.arr[gi]
-            a.prefix, a.prefix_len, a.branches, a.nbranches = _addr(p), p.size, br, nb
+            a.prefix, a.prefix_len, a.nbranches = _addr(p), p.size, nb
+            a.branches = C.cast(br.buffer_info()[0], _BRANCH_P)
 
 
 def _u32_joined(seqs: Sequence, total: int) -> np.ndarray:
@@ -198,6 +208,10 @@ def _u32_joined(seqs: Sequence, total: int) -> np.ndarray:
     if total == 0:
         return np.zeros(1, np.uint32)
     if all(isinstance(x, np.ndarray) for x in seqs):
+        if all(x.ndim == 1 for x in seqs):
+            x = np.concatenate(seqs)
+            if x.dtype == _U32:
+                return x
         return _u32(np.concatenate([np.asarray(x, dtype=np.int64).ravel() for x in seqs]))
     return np.fromiter(itertools.chain.from_iterable(seqs), np.int64, total).astype(np.uint32)
 
@@ -288,12 +302,19 @@ class Engine:
         L.check(L.lib().omg_evaluate_groups(self._h, cg.arr, cg.n, int(want),
                                             lab.ctypes.data_as(C.POINTER(C.c_uint32)), lab.size,
                                             out.ctypes.data_as(C.POINTER(C.c_float)), out.size, src))
+        # Rows of a small result are views of this call's own array (208 rows
+        # of 2,560: 0.5 ms of copies); of a large one copies, so that a kept
+        # row keeps no more than itself.
+        rows_out = list(out[:rows, :width])
+        if out.nbytes > _SHARED_ROWS_BYTES:
+            rows_out = [x.copy() for x in rows_out]
         res, r = [], 0
         for gi, g in enumerate(groups):
             bo = []
             for b in g.branches:
-                bo.append(BranchOutput(rows=[out[r + s, :width].copy() for s in range(len(b.want))]))
-                r += len(b.want)
+                n = len(b.want)
+                bo.append(BranchOutput(rows=rows_out[r:r + n]))
+                r += n
             res.append(GroupOutput(branches=bo, prefix_source=PrefixSource(src[gi])))
         return res
 

@@ -252,3 +252,29 @@ def test_state_bytes_mutations_fail_cleanly():
         except L.OmgError:
             refused += 1
     assert refused > 0
+
+
+@pytest.mark.parametrize("kind", [list, tuple, np.uint32, np.int64, "mixed", "strided"])
+def test_request_arrays_of_every_kind_pack_alike(kind):
+    """Tokens and wanted rows as lists, tuples, uint32 or other arrays, a
+    mixture of them or strided views, with an empty prefix, a branch that
+    wants nothing and a group without branches: the same packing."""
+    def conv(x, i):
+        if kind in (list, tuple):
+            return kind(x)
+        if kind == "mixed":
+            return list(x) if i % 3 == 0 else np.array(x, np.uint32 if i % 3 == 1 else np.int64)
+        if kind == "strided":
+            return np.repeat(np.array(x, np.uint32), 2)[::2]
+        return np.array(x, kind)
+
+    raw = [([], [([5, 6, 7], [0, 2]), ([8], [])]), ([1, 2, 3], []), (list(range(40)), [([9] * 33, [32]), ([4, 250000], [1])])]
+    groups = [g.Group(conv(p, i), [g.BranchTokens(conv(t, i + j), conv(w, j + 1)) for j, (t, w) in enumerate(bs)])
+              for i, (p, bs) in enumerate(raw)]
+    ids, meta, wanted = g.pack(groups, first=2, align=32, rows=1 << 12)
+    flat = raw[2][0] + [9] * 33 + [4, 250000]
+    assert ids[:len(flat)].tolist() == flat
+    assert sorted(x for x in ids.tolist() if x) == sorted(x for x in flat + [5, 6, 7, 8, 1, 2, 3] if x)
+    at = {tuple(w[:3]): int(ids[w[3]]) for w in wanted.tolist()}
+    assert at == {(2, 0, 0): 9, (2, 1, 0): 250000, (0, 0, 0): 5, (0, 0, 1): 7}
+    assert meta[:len(flat), 3].tolist() == list(range(1, len(flat) + 1))
