@@ -469,22 +469,26 @@ __global__ __launch_bounds__(NW * 64) void attention_kernel(AttnArgs a, const in
 // out = sum_c O_c l_c 2^(m_c - M) / sum_c l_c 2^(m_c - M), M = max_c m_c,
 // over the chunks the row saw anything in.  A row with one such chunk gets
 // that chunk's f16 output unchanged, exactly what an unsplit tile writes.
-// One wave per row (four rows per workgroup); lane l owns columns
-// 256 q + 4l .. 256 q + 4l + 3 (q < HD / 256), so every 256 columns of a
-// partial row are one contiguous 512-byte wave load.
+// Half a wave per row (eight rows per workgroup); lane l of it owns columns
+// 256 q + 8l .. 256 q + 8l + 7 (q < HD / 256), so a wave load is 16 bytes per
+// lane, 512 contiguous bytes of each of its two rows.  Long passes are bound
+// by the partials' bytes (16,320 rows of 8 heads in about five chunks, 400 MB:
+// a wave per row and 8-byte loads 156 us, this 150); the 270M model's cold
+// pass 6.9 -> 6.2 us a launch, its one-branch pass, all latency, 5.5 -> 5.3.
 // The statistics and partial rows of up to MAXC chunks are loaded together
 // (one round trip after the merge record).
 template <int HD, int NW>
 __global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs a, const int4* __restrict__ merges) {
     constexpr int ROWS = NW * 16 * A_QB;  // query rows of a work item
-    static_assert(HD == 256 || HD == 512, "half4 column groups per lane");
+    static_assert(HD == 256 || HD == 512, "half8 column groups per lane");
     constexpr int NQ = HD / 256;
     constexpr int MAXC = 8;  // chunks loaded per round
-    const int4 mg = merges[blockIdx.x / (ROWS / 4)];
+    constexpr int WG_ROWS = 8, LR = WAVE / 2;  // lanes per row
+    const int4 mg = merges[blockIdx.x / (ROWS / WG_ROWS)];
     const int qtile = mg.x, slot0 = mg.y, n = mg.z;
     const int g = int(blockIdx.y);
-    const int wave = int(threadIdx.x) / WAVE, lane = int(threadIdx.x) % WAVE;
-    const int row = int(blockIdx.x % (ROWS / 4)) * 4 + wave;
+    const int lane = int(threadIdx.x) % LR;
+    const int row = int(blockIdx.x % (ROWS / WG_ROWS)) * WG_ROWS + int(threadIdx.x) / LR;
     // Row r of a work item: 16-row block r / 16 (wave-major), 16 / hpg tokens
     // per block, the lane's token (r % 16) / hpg within it.
     const int hpg = a.heads / a.kv_heads, tpq = 16 / hpg, tpb = NW * A_QB * tpq;
@@ -495,16 +499,17 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs a, const 
     // Running merge over rounds of MAXC chunks (one round for n <= MAXC):
     // (M, L, acc) rescaled when a later round raises the max.
     float M = -INFINITY, L = 0.0f;
-    float4 acc[NQ];
-    half4 only[NQ];
+    float acc[NQ][8];
+    half8 only[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        acc[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        only[q] = half4{};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[q][e] = 0.0f;
+        only[q] = half8{};
     }
     int seen = 0;
     for (int c0 = 0; c0 < n; c0 += MAXC) {
-        half4 v[MAXC][NQ];
+        half8 v[MAXC][NQ];
         float2 ml[MAXC];
 #pragma unroll
         for (int c = 0; c < MAXC; ++c) {
@@ -512,7 +517,7 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs a, const 
                 ml[c] = *reinterpret_cast<const float2*>(a.part_ml + base(c0 + c) * 2);
 #pragma unroll
                 for (int q = 0; q < NQ; ++q)
-                    v[c][q] = *reinterpret_cast<const half4*>(a.part_o + base(c0 + c) * HD + q * 256 + lane * 4);
+                    v[c][q] = *reinterpret_cast<const half8*>(a.part_o + base(c0 + c) * HD + q * 256 + lane * 8);
             } else {
                 ml[c] = make_float2(-INFINITY, 0.0f);
             }
@@ -524,12 +529,9 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs a, const 
         const float r = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - Mr);
         L *= r;
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            acc[q].x *= r;
-            acc[q].y *= r;
-            acc[q].z *= r;
-            acc[q].w *= r;
-        }
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[q][e] *= r;
         M = Mr;
 #pragma unroll
         for (int c = 0; c < MAXC; ++c) {
@@ -540,20 +542,19 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs a, const 
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
                 only[q] = v[c][q];
-                acc[q].x += float(v[c][q].x) * w;
-                acc[q].y += float(v[c][q].y) * w;
-                acc[q].z += float(v[c][q].z) * w;
-                acc[q].w += float(v[c][q].w) * w;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[q][e] += float(v[c][q][e]) * w;
             }
         }
     }
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const half4 o = seen == 1 ? only[q]
-                                  : half4{half_t(acc[q].x * inv), half_t(acc[q].y * inv), half_t(acc[q].z * inv),
-                                          half_t(acc[q].w * inv)};
-        *reinterpret_cast<half4*>(a.out + (tq * a.heads + head) * HD + q * 256 + lane * 4) = o;
+        half8 o = only[q];
+        if (seen != 1)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = half_t(acc[q][e] * inv);
+        *reinterpret_cast<half8*>(a.out + (tq * a.heads + head) * HD + q * 256 + lane * 8) = o;
     }
 }
 
@@ -718,7 +719,7 @@ void launch_attention(hipStream_t s, const AttnArgs& a, const int4* items, int64
 void launch_attention_merge(hipStream_t s, const AttnArgs& a, const int4* merges, int64_t nmerges, int nw) {
     if (a.t <= 0 || nmerges <= 0) return;
     if (nw != 2 && nw != A_NW) fail(E_INVALID, "attention_merge: waves per item must be 2 or 4");
-    const dim3 grid(unsigned(nmerges * (nw * 16 * A_QB / 4)), unsigned(a.kv_heads));
+    const dim3 grid(unsigned(nmerges * (nw * 16 * A_QB / 8)), unsigned(a.kv_heads));
     if (a.hd != 512 && a.hd != 256) fail(E_INVALID, "attention_merge: head_dim must be 256 or 512");
     if (a.hd == 512 && nw == 2)
         attention_merge_kernel<512, 2><<<grid, dim3(256), 0, s>>>(a, merges);
