@@ -630,19 +630,29 @@ void launch_gather_out(hipStream_t s, const half_t* a, int64_t wa, const float* 
 //
 // The f32 MFMA runs at a sixteenth of the f16 one, so each row is scaled by
 // a power of two (its largest finite |x| into [2^14, 2^15)) and written as
-// two f16 parts, x 2^e = hi + lo: lo is the residual of a rounding to
-// nearest, so what is left out is at most 2^-24 |x|, one f32 rounding.  The
-// weights enter as what their codes say exactly (q - 8, q, or the f16
-// itself), so every product is exact and the sums are f32: per 32-element
-// block, four MFMAs (lo, hi of two 16-wide k-steps) give s_b = sum_k q_k
-// x_k, and acc += d_b s_b is one fma per element (f16 weights: straight
-// into acc).
+// three f16 parts, x 2^e = hi + 2^-12 (mid + lo), each the rounding of what
+// the parts before it leave: 11 + 11 bits and two signs hold 24, and the
+// lower two in a range of their own hold every f32 down to 2^-27 of the
+// row's largest.  The weights enter as what their codes say exactly (q - 8
+// or q, for the lower parts times 2^-12; or the f16 itself), so every
+// product is exact and the sums are f32: per 32-element block, six MFMAs
+// (lo, mid, hi of two 16-wide k-steps) give s_b = sum_k q_k x_k, and acc +=
+// d_b s_b is one fma per element (f16 weights: straight into an accumulator
+// for hi and one for the lower parts).
 //
-// Measured (MI355X, 25,000 columns, Q4): 208 rows of 2,560 (26.6 GFLOP)
-// 647 -> 82 us with its two neighbours, 12 rows of 640 17.3 -> 9.9 us; the
-// distance to float64 fell from 3.8e-7 and 2.0e-7 to 0.9e-7 and 0.7e-7 of
-// the rows' 2-norm.  What bounds it now is VALU issue (decode, the scale
-// fmas) beside the MFMAs.
+// Rows the parts do not hold in every bit (an element under 2^-27 of the
+// largest with low bits set, an infinity, a NaN) run again on the f32 MFMA
+// and take those sums, as do logits that come out NaN (a zero part times an
+// infinite weight); their row tile alone pays, about one standard normal row
+// in 20,000.  Two parts in one range held 23 bits, and of an element
+// 2^-24 of the row's largest 15.
+//
+// Measured (MI355X, 25,000 columns, Q4, whole calls): 208 rows of 2,560
+// (26.6 GFLOP) on the f32 MFMA 647 us, on two parts 77, on three 96; 12 rows
+// of 640: 26, 16, 18.  Distance to float64 (of the rows' 2-norm): 3.8e-7,
+// 0.87e-7, 0.84e-7 and 2.0e-7, 0.63e-7, 0.61e-7; f16 weights at 2,560 wide
+// 2.0e-7 on two parts, 1.5e-7 on three.  What bounds it is the MFMAs and,
+// beside them, VALU issue (decode, the scale fmas).
 //
 // Operands: the rows are A (from LDS), the weights B, straight from the
 // stage tiles (kernels.h) into registers; lane l holds vocabulary column
@@ -656,7 +666,8 @@ constexpr int LG_R = 32;      // readout rows per workgroup (an MFMA row tile)
 constexpr int LG_COLS = 32;   // columns per partial (an MFMA column tile)
 constexpr int LG_ST = 64;     // K per stage, as the weights' stage tiles
 constexpr int LG_FRAG = 1024; // bytes of one A fragment: 64 lanes x 8 f16
-constexpr int LG_PARTS = 2;
+constexpr int LG_PARTS = 3;
+constexpr float LG_LOW = 4096.0f;  // the scale of the lower parts
 constexpr int LG_STAGE = 4 * LG_PARTS * LG_FRAG;  // one stage of a row tile: 4 k-steps x the parts
 constexpr int LG_KC = 4;      // stages converted at once when the rows are split in the kernel
 constexpr int LG_NS = 3;      // ring slots when they arrive split
@@ -673,20 +684,30 @@ __device__ inline float finite_abs(float v) {
     const float a = fabsf(v);
     return a < INFINITY ? a : 0.0f;
 }
-// v = hi + lo; infinities and NaNs stay in hi alone.
-__device__ inline void split2(const float (&v)[8], half8 (&p)[LG_PARTS]) {
+// v = hi + (mid + lo) / LG_LOW; whether that holds for all eight exactly
+// (never for an infinity or a NaN).
+__device__ inline bool split3(const float (&v)[8], half8 (&p)[LG_PARTS]) {
+    bool held = true;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const half_t h = half_t(v[i]);
-        p[0][i] = h;
-        p[1][i] = half_t(fabsf(v[i]) < INFINITY ? v[i] - float(h) : 0.0f);
+        const half_t hi = half_t(v[i]);
+        const float r = (v[i] - float(hi)) * LG_LOW;  // at most 2^15
+        const half_t mid = half_t(r);
+        const float r2 = r - float(mid);
+        const half_t lo = half_t(r2);
+        p[0][i] = hi;
+        p[1][i] = mid;
+        p[2][i] = lo;
+        held = held && float(lo) == r2;
     }
+    return held;
 }
 
 // The rows split ahead of the product, a workgroup per row (rows past the
 // end and columns past K as zeros): part p of row r, elements
 // 64 st + 16 ks + 8 h .. + 7 at fragment ((r / 32 * stages + st) * 4 + ks) *
-// parts + p, lane 32 h + r % 32; inv[r] undoes the row's scale.
+// parts + p, lane 32 h + r % 32; inv[r] undoes the row's scale, negative
+// where the parts do not hold the row.
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ rows, int64_t nrows, int64_t K,
                                                          int64_t stages, half_t* __restrict__ frag,
                                                          float* __restrict__ inv) {
@@ -720,7 +741,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
     if (lane == 0) red[wave] = m;
     __syncthreads();
     const float2 sc = row_scale(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-    if (tid == 0) inv[r] = sc.y;
+    bool held = true;
     for (int64_t g = tid; g < stages * 8; g += 256) {
         float v[8];
         if (g == tid) {
@@ -732,18 +753,20 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] *= sc.x;
         half8 p[LG_PARTS];
-        split2(v, p);
+        held = split3(v, p) && held;
         const int64_t f = (r / LG_R * stages + g / 8) * 4 + (g % 8) / 2;
         const int ln = int(32 * (g % 2) + r % LG_R);
 #pragma unroll
         for (int k = 0; k < LG_PARTS; ++k)
             *reinterpret_cast<half8*>(frag + (f * LG_PARTS + k) * (LG_FRAG / 2) + ln * 8) = p[k];
     }
+    held = __syncthreads_and(held);
+    if (tid == 0) inv[r] = held ? sc.y : -sc.y;
 }
 
 struct LogitArgs {
     DevWeight E;
-    const float* rows;    // f32 rows, split in the kernel (SPLIT_IN)
+    const float* rows;    // f32 rows
     const half_t* frag;   // split_rows_kernel's fragments
     const float* inv;     // and row scales
     int64_t nrows;
@@ -758,15 +781,15 @@ struct LogitArgs {
 };
 
 // Four waves, each CT column tiles of 32 on one row tile of 32.  Per stage
-// a wave has 8 CT MFMAs (32 cycles of its SIMD's matrix core each) against
-// 8 fragment reads, 36 CT decode and 32 CT scale instructions.  A block's
+// a wave has 12 CT MFMAs (32 cycles of its SIMD's matrix core each) against
+// 12 fragment reads, 52 CT decode and 32 CT scale instructions.  A block's
 // scale instructions run one block late, behind the next block's MFMAs:
 // right after their own they would wait out the matrix core's latency.
 // SPLIT_IN: the workgroup splits the rows itself, LG_KC stages at a time,
 // for callers without scratch; otherwise the fragments stream through an
 // LDS ring by DMA.
 template <int DT, int CT, bool SPLIT_IN>
-__global__ __launch_bounds__(256) void logits_kernel(LogitArgs a) {
+__global__ __launch_bounds__(256, CT == 2 || SPLIT_IN ? 2 : 4) void logits_kernel(LogitArgs a) {
     constexpr int CL = tile_packet_bytes(DT) / 1024;  // 16-byte code loads per lane and stage
     constexpr int PK = tile_packet_bytes(DT);
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -807,8 +830,22 @@ __global__ __launch_bounds__(256) void logits_kernel(LogitArgs a) {
                 w.sc[c] = *reinterpret_cast<const uint32_t*>(sp[c] + int64_t(st) * TILE_SCALE_BYTES);
         }
     };
-    floatx16 acc[CT], late[CT];  // late: the last block's sums, not yet scaled by
-    float ld[CT];                // its scale and added
+    // This lane's eight codes of k-step ks.
+    auto codes = [&](const W& w, int c, int ks) -> half8 {
+        if constexpr (DT == Q4_DT) {
+            const uint4 u = w.code[c][0];
+            return q4_word_codes(ks == 0 ? u.x : ks == 1 ? u.y : ks == 2 ? u.z : u.w);
+        } else if constexpr (DT == Q8_DT) {
+            const uint4 u = w.code[c][ks / 2];
+            return ks % 2 == 0 ? q8_words_codes(u.x, u.y) : q8_words_codes(u.z, u.w);
+        } else {
+            return __builtin_bit_cast(half8, w.code[c][ks]);
+        }
+    };
+    // late: the last block's sums, not yet scaled by its scale ld and added
+    // (f16 weights: the sums of the lower parts)
+    floatx16 acc[CT], late[CT];
+    float ld[CT];
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
         acc[c] = floatx16{};
@@ -832,36 +869,36 @@ __global__ __launch_bounds__(256) void logits_kernel(LogitArgs a) {
 #pragma unroll
                 for (int p = LG_PARTS - 1; p >= 0; --p)
                     xf[k][p] = *reinterpret_cast<const half8*>(S + ((2 * blk + k) * LG_PARTS + p) * LG_FRAG + lane * 16);
-            half8 wf[CT][2];
+            half8 wf[CT][2], wl[CT][2];  // wl: for the lower parts
 #pragma unroll
             for (int c = 0; c < CT; ++c)
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
-                    const int ks = 2 * blk + k;
-                    if constexpr (DT == Q4_DT) {
-                        const uint4 u = w.code[c][0];
-                        wf[c][k] = q4_word_codes(ks == 0 ? u.x : ks == 1 ? u.y : ks == 2 ? u.z : u.w);
-                    } else if constexpr (DT == Q8_DT) {
-                        const uint4 u = w.code[c][blk];
-                        wf[c][k] = k == 0 ? q8_words_codes(u.x, u.y) : q8_words_codes(u.z, u.w);
-                    } else {
-                        wf[c][k] = __builtin_bit_cast(half8, w.code[c][ks]);
-                    }
+                    wf[c][k] = codes(w, c, 2 * blk + k);
+                    wl[c][k] = DT == F16_DT ? wf[c][k] : wf[c][k] * half_t(1.0f / LG_LOW);
                 }
-            floatx16 s[CT];
-#pragma unroll
-            for (int c = 0; c < CT; ++c) s[c] = DT == F16_DT ? acc[c] : floatx16{};
-#pragma unroll
-            for (int p = LG_PARTS - 1; p >= 0; --p)
-#pragma unroll
-                for (int k = 0; k < 2; ++k)
-#pragma unroll
-                    for (int c = 0; c < CT; ++c)
-                        s[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[k][p], wf[c][k], s[c], 0, 0, 0);
             if constexpr (DT == F16_DT) {
 #pragma unroll
-                for (int c = 0; c < CT; ++c) acc[c] = s[c];
+                for (int p = LG_PARTS - 1; p >= 0; --p)
+#pragma unroll
+                    for (int k = 0; k < 2; ++k)
+#pragma unroll
+                        for (int c = 0; c < CT; ++c) {
+                            floatx16& s = p ? late[c] : acc[c];
+                            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[k][p], wf[c][k], s, 0, 0, 0);
+                        }
             } else {
+                floatx16 s[CT];
+#pragma unroll
+                for (int c = 0; c < CT; ++c) s[c] = floatx16{};
+#pragma unroll
+                for (int p = LG_PARTS - 1; p >= 0; --p)
+#pragma unroll
+                    for (int k = 0; k < 2; ++k)
+#pragma unroll
+                        for (int c = 0; c < CT; ++c)
+                            s[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[k][p], p ? wl[c][k] : wf[c][k], s[c], 0, 0,
+                                                                          0);
                 add_late();
 #pragma unroll
                 for (int c = 0; c < CT; ++c) {
@@ -897,7 +934,7 @@ __global__ __launch_bounds__(256) void logits_kernel(LogitArgs a) {
 #pragma unroll
         for (int o = 4; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, WAVE));
         const float2 sc = row_scale(m);
-        if (sub == 0) sinv[rr] = sc.y;
+        bool held = true;
         float4 raw[LG_KC][2];
         auto load_x = [&](int st0) {
 #pragma unroll
@@ -917,7 +954,7 @@ __global__ __launch_bounds__(256) void logits_kernel(LogitArgs a) {
                 const float e[8] = {u.x * sc.x, u.y * sc.x, u.z * sc.x, u.w * sc.x,
                                     v.x * sc.x, v.y * sc.x, v.z * sc.x, v.w * sc.x};
                 half8 p[LG_PARTS];
-                split2(e, p);
+                held = split3(e, p) && held;
 #pragma unroll
                 for (int k = 0; k < LG_PARTS; ++k)
                     *reinterpret_cast<half8*>(smem + g * LG_STAGE + ((sub / 2) * LG_PARTS + k) * LG_FRAG +
@@ -933,6 +970,9 @@ __global__ __launch_bounds__(256) void logits_kernel(LogitArgs a) {
                 compute(smem + g * LG_STAGE, w[g % R]);
             }
         }
+#pragma unroll
+        for (int o = 4; o > 0; o >>= 1) held = __shfl_xor(int(held), o, WAVE) && held;
+        if (sub == 0) sinv[rr] = held ? sc.y : -sc.y;
     } else {
         if (tid < LG_R) sinv[tid] = a.inv[r0 + tid];
         const uint8_t* src = reinterpret_cast<const uint8_t*>(a.frag) + rt * stages * int64_t(LG_STAGE);
@@ -982,10 +1022,65 @@ __global__ __launch_bounds__(256) void logits_kernel(LogitArgs a) {
     }
 
     add_late();
+    if constexpr (DT == F16_DT)
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[c][e] = fmaf(late[c][e], 1.0f / LG_LOW, acc[c][e]);
     // Each wave's tile through LDS (its own 32 rows of 33 floats, where the
     // fragments were): the row statistics then take two lanes per row
     // instead of a 32-lane reduction per element.
     __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const float inv = fabsf(sinv[8 * (e / 4) + 4 * lh + e % 4]);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[c][e] *= inv;
+    }
+    // Rows the parts do not hold: on v_mfma_f32_32x32x2_f32 (lane: row lc of
+    // A, column lc of B, K 8 lh + e of a k-step at step e), for the whole
+    // tile, of which those rows take the result.
+    bool redo = sinv[lc] < 0.0f;
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) redo = redo || acc[c][e] != acc[c][e];
+    if (__any(redo)) {
+        floatx16 sum[CT];
+#pragma unroll
+        for (int c = 0; c < CT; ++c) sum[c] = floatx16{};
+        const float* x = a.rows + (r0 + lc) * K;
+#pragma unroll 1
+        for (int st = 0; st < stages; ++st) {
+            W u;
+            load_w(st, u);
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                const int64_t k = int64_t(st) * LG_ST + 16 * ks + 8 * lh;
+                float4 lo = make_float4(0.0f, 0.0f, 0.0f, 0.0f), hi = lo;
+                if (r0 + lc < a.nrows && k < K) {
+                    lo = *reinterpret_cast<const float4*>(x + k);
+                    hi = *reinterpret_cast<const float4*>(x + k + 4);
+                }
+                const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    const half8 q = codes(u, c, ks);
+                    const float d = DT == F16_DT ? 1.0f : half_bits_to_f32(uint16_t(u.sc[c] >> (16 * (ks / 2))));
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        sum[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[e], float(q[e]) * d, sum[c], 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const bool row = sinv[8 * (e / 4) + 4 * lh + e % 4] < 0.0f;
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+                if (row || acc[c][e] != acc[c][e]) acc[c][e] = sum[c][e];
+        }
+    }
     constexpr int TS = LG_COLS + 1;
     float* T = reinterpret_cast<float*>(smem) + wave * LG_R * TS;
 #pragma unroll
@@ -994,7 +1089,7 @@ __global__ __launch_bounds__(256) void logits_kernel(LogitArgs a) {
         if (j0 >= a.ncols) break;
         float z[16];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) z[e] = acc[c][e] * sinv[8 * (e / 4) + 4 * lh + e % 4];
+        for (int e = 0; e < 16; ++e) z[e] = acc[c][e];
         if (a.softcap > 0.0f)
 #pragma unroll
             for (int e = 0; e < 16; ++e) z[e] = a.softcap * tanhf(z[e] / a.softcap);

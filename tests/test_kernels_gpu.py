@@ -210,12 +210,12 @@ def test_label_readout_odd_shapes_and_out_of_vocab_labels():
 @pytest.mark.parametrize("vocab,d,nrows,nlabels", [(31, 32, 31, 3), (257, 96, 32, 26), (1025, 1312, 33, 600),
                                                    (31000, 64, 130, 26), (640, 4096, 65, 5)])
 def test_split_readout_edges(vocab, d, nrows, nlabels, dtype):
-    """Two f16 parts per row element leave out at most 2^-24 of it, products
-    are exact and a column's sums are f32 over at most 2 d / 16 + d / 32
-    roundings: 2^-24 (2 + d / 8) of sum |x||w| bounds a logit's error (and
-    the log-sum-exp's, plus its own few ulps).  Rows of very different
-    magnitudes share a launch; with and without scratch the logits are the
-    same bits."""
+    """The parts hold a row element exactly, products are exact, and a
+    column's sums are f32 over d / 16 roundings of the high parts' sums (the
+    lower parts' are 2^-11 of those) and d / 32 of the scaled blocks:
+    2^-24 (2 + d / 8) of sum |x||w| bounds a logit's error (and the
+    log-sum-exp's, plus its own few ulps).  Rows of very different magnitudes
+    share a launch; with and without scratch the logits are the same bits."""
     rng = np.random.default_rng(vocab * 7 + d + nrows + dtype)
     t, _ = weight(rng, vocab, d, dtype, "embed")
     e = t.to_f32().astype(np.float64)
@@ -239,6 +239,81 @@ def test_split_readout_edges(vocab, d, nrows, nlabels, dtype):
     m = z.max(1)
     lse = m + np.log(np.exp(z - m[:, None]).sum(1))
     assert (np.abs(outs[0][:, -1] - lse) <= bound.max(1) + 1e-6 * np.maximum(1.0, np.abs(lse))).all()
+
+
+# Split ahead of the product (one and two column tiles per wave, a half last
+# stage) and in the workgroups (more labels than a tile scans, no scratch).
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("vocab,d,nrows,nlabels", [(300, 96, 40, 7), (31, 2560, 33, 3), (31000, 64, 140, 9),
+                                                   (1400, 352, 70, 600)])
+def test_readout_of_rows_with_an_outlier(vocab, d, nrows, nlabels, dtype):
+    """Rows with one element 2^12 to 2^102 times the others, read out at
+    columns whose weight there is zero: their logits are the sums of the
+    small elements and stay f32 sums of f32 values, whatever the range of the
+    row.  An f32 sum of d products rounds at most d times: 2^-24 d of
+    sum |x||w|, the outlier adding nothing.  Rows with and without an outlier
+    share row tiles; each row alone gives the same bits."""
+    rng = np.random.default_rng(vocab * 3 + d + nrows + dtype)
+    at = d // 3
+    v = rng.uniform(-1, 1, (vocab, d)).astype(np.float32)
+    v[::2, at] = 0.0
+    if dtype == g.F16:
+        t = g.QTensor("embed", g.F16, (vocab, d), v.astype(np.float16).view(np.uint8).ravel().copy(),
+                      np.zeros(0, np.uint8))
+    else:
+        t = g.QTensor("embed", dtype, (vocab, d), *oracle.quantize(dtype, v))
+    e = t.to_f32().astype(np.float64)
+    assert (e[::2, at] == 0.0).all()
+    rows = rng.standard_normal((nrows, d)).astype(np.float32)
+    wide = [r for r in range(nrows) if r % 3]
+    for i, r in enumerate(wide):
+        rows[r, at] = (-1.0) ** i * 2.0 ** (12 + 90 * i / len(wide))
+    labels = rng.choice(np.arange(0, vocab, 2), nlabels, replace=False).astype(np.uint32)
+    w = g.DeviceWeight(t)
+    lab = dev(labels.view(np.int32))
+
+    def run(f, x):
+        xd = dev(x)
+        out = torch.full((len(x), nlabels + 1), float("nan"), dtype=torch.float32, device="cuda")
+        f(xd.data_ptr(), len(x), lab.data_ptr(), nlabels, 0.0, out.data_ptr())
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    got = run(w.label_readout, rows)
+    z = rows.astype(np.float64) @ e.T
+    bound = 2.0 ** -24 * d * (np.abs(rows).astype(np.float64) @ np.abs(e).T)
+    assert (np.abs(got[:, :-1] - z[:, labels]) <= bound[:, labels]).all()
+    for r in (0, 1, nrows // 2, nrows - 1):
+        assert np.array_equal(run(w.label_readout, rows[r:r + 1])[0], got[r])
+    few = rows[:min(nrows, 4_000_000 // (vocab + 100))]
+    assert np.array_equal(run(w.label_readout_noalloc, few), got[:len(few)])
+
+
+def test_readout_of_an_infinite_weight():
+    """An infinite f16 weight gives its column infinities of the row
+    element's sign (NaN where that element is zero), as an f32 product does,
+    and leaves every other column alone."""
+    rng = np.random.default_rng(4)
+    v = rng.uniform(-1, 1, (200, 96)).astype(np.float16)
+    rows = (rng.integers(1, 64, (35, 96)) * rng.choice([-1, 1], (35, 96))).astype(np.float32)
+    rows[5, 40] = 0.0
+    lab = dev(np.arange(200, dtype=np.int32))
+    rd = dev(rows)
+
+    def run():
+        w = g.DeviceWeight(g.QTensor("embed", g.F16, v.shape, v.view(np.uint8).ravel().copy(), np.zeros(0, np.uint8)))
+        out = torch.zeros((35, 201), dtype=torch.float32, device="cuda")
+        w.label_readout(rd.data_ptr(), 35, lab.data_ptr(), 200, 0.0, out.data_ptr())
+        torch.cuda.synchronize()
+        return out.cpu().numpy()[:, :200]
+
+    ref = run()
+    v[17, 40] = np.inf
+    got = run()
+    others = np.arange(200) != 17
+    assert np.array_equal(got[:, others], ref[:, others])
+    live = np.arange(35) != 5
+    assert np.array_equal(got[live, 17], np.sign(rows[live, 40]) * np.inf) and np.isnan(got[5, 17])
 
 
 def test_readout_of_non_finite_rows_and_streams():
