@@ -21,36 +21,44 @@ struct omg_engine {
     std::unique_ptr<omg::Engine> e;
 };
 // Scratch of stream-ordered calls on one object, kept from call to call: an
-// allocation and its release cost the host about 14 us a call, more than a
-// small readout's kernels take.  It serves the first stream it is asked for
-// (calls there run in order, so they share it); any other stream, the
-// per-thread stream (one handle, many streams), calls being captured and
-// requests above LIMIT allocate in stream order.
+// allocation and its release cost 12 us a call back to back and 40 where the
+// caller waits for each, more than a small readout's kernels take; the event
+// that marks a call's end costs 4 and nothing.  A call takes the kept block when the
+// call that had it last is over, or is on the same stream: there it waits for
+// that call's event all the same, since a new stream can carry a destroyed
+// one's handle.  Calls that find it busy on another stream, calls being
+// captured and requests above LIMIT allocate in stream order.
 class StreamScratch {
    public:
     ~StreamScratch() {
+        if (done_) {
+            (void)hipEventSynchronize(done_);
+            (void)hipEventDestroy(done_);
+        }
         if (p_) (void)hipFree(p_);
     }
     // f(scratch) with at least `bytes`; queues its work on s.
     template <class F>
     void with(hipStream_t s, size_t bytes, F&& f) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (s != hipStreamPerThread) OMG_HIP(hipStreamIsCapturing(s, &cap));
-        if (s != hipStreamPerThread && cap == hipStreamCaptureStatusNone && bytes <= LIMIT) {
+        if (bytes <= LIMIT && !capturing(s)) {
             int dev = 0;  // the null stream is one per device
             OMG_HIP(hipGetDevice(&dev));
             std::lock_guard<std::mutex> lock(mu_);
-            if (!p_ || (s == owner_ && dev == dev_)) {
+            if (take(s, dev)) {
                 if (bytes > bytes_) {
                     if (p_) OMG_HIP(hipFreeAsync(p_, s));
                     p_ = nullptr;
                     bytes_ = 0;
                     OMG_HIP(hipMallocAsync(&p_, bytes, s));
                     bytes_ = bytes;
-                    owner_ = s;
-                    dev_ = dev;
                 }
-                f(p_);
+                try {
+                    f(p_);
+                } catch (...) {
+                    (void)hipEventRecord(done_, s);
+                    throw;
+                }
+                OMG_HIP(hipEventRecord(done_, s));
                 return;
             }
         }
@@ -67,9 +75,47 @@ class StreamScratch {
 
    private:
     static constexpr size_t LIMIT = size_t(64) << 20;
+
+    // (a failed look leaves no error behind for the launches' own checks)
+    static bool capturing(hipStream_t s) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+        (void)hipGetLastError();
+        return true;
+    }
+    // Whether the block is the next call's on s; s then runs after the call
+    // that had it last.
+    bool take(hipStream_t s, int dev) {
+        if (!done_) {
+            OMG_HIP(hipEventCreateWithFlags(&done_, hipEventDisableTiming));
+            dev_ = dev;
+        } else {
+            if (dev != dev_) return false;
+            // (the per-thread stream is one handle for many streams)
+            if (s == owner_ && s != hipStreamPerThread) {
+                OMG_HIP(hipStreamWaitEvent(s, done_, 0));
+            } else if (!over()) {
+                return false;
+            }
+        }
+        owner_ = s;
+        return true;
+    }
+    // Another thread may be capturing, which a query of an event outside its
+    // graph must not disturb.
+    bool over() {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        const hipError_t e = hipEventQuery(done_);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e == hipSuccess;
+    }
+
     std::mutex mu_;
     void* p_ = nullptr;
     size_t bytes_ = 0;
+    hipEvent_t done_ = nullptr;  // after the last call that had the block
     hipStream_t owner_ = nullptr;
     int dev_ = 0;
 };

@@ -647,9 +647,9 @@ void launch_gather_out(hipStream_t s, const half_t* a, int64_t wa, const float* 
 // in 20,000.  Two parts in one range held 23 bits, and of an element
 // 2^-24 of the row's largest 15.
 //
-// Measured (MI355X, 25,000 columns, Q4, whole calls): 208 rows of 2,560
-// (26.6 GFLOP) on the f32 MFMA 647 us, on two parts 77, on three 96; 12 rows
-// of 640: 26, 16, 18.  Distance to float64 (of the rows' 2-norm): 3.8e-7,
+// Measured (MI355X, 25,000 columns, Q4, the three launches back to back):
+// 208 rows of 2,560 (26.6 GFLOP) on the f32 MFMA 647 us, on two parts 77, on
+// three 96; 12 rows of 640: 26, 16, 18.  Distance to float64 (of the rows' 2-norm): 3.8e-7,
 // 0.87e-7, 0.84e-7 and 2.0e-7, 0.63e-7, 0.61e-7; f16 weights at 2,560 wide
 // 2.0e-7 on two parts, 1.5e-7 on three.  What bounds it is the MFMAs and,
 // beside them, VALU issue (decode, the scale fmas).

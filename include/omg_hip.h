@@ -271,10 +271,11 @@ int omg_dev_gemm_geglu(const omg_weight *wg, const omg_weight *wu, const void *x
  * the full vocabulary row: out f32 [nrows][nlabels + 1].  `rows` must be
  * 16-byte aligned.  Label ids must be below vocab; the device-resident ids
  * are not checked before the launch, and an id past the vocabulary gives
- * NaN in its column.  The full logits and per-workgroup partials live in
- * scratch device memory: up to 64 MiB kept with the weight for the first
- * stream it is read out on, otherwise (another stream, under capture, more)
- * allocated and freed by the call in stream order. */
+ * NaN in its column.  The split rows, the partials and (above 512 labels)
+ * the full logits live in scratch device memory: up to 64 MiB kept with the
+ * weight from call to call, whatever their streams; a call that finds it in
+ * use on another stream, is being captured or needs more allocates and frees
+ * its own in stream order. */
 int omg_dev_label_readout(const omg_weight *embed, const float *rows, int64_t nrows, const uint32_t *labels,
                           int64_t nlabels, float softcap, float *out, void *stream);
 /* No counterpart in the reference.  omg_dev_label_readout for callers that

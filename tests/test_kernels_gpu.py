@@ -318,7 +318,7 @@ def test_readout_of_an_infinite_weight():
 
 def test_readout_of_non_finite_rows_and_streams():
     """An infinity or a NaN in a row stays in that row; calls on two streams
-    with one weight keep apart."""
+    in turn, one at a time, give the same rows."""
     rng = np.random.default_rng(9)
     vocab, d, nrows = 500, 128, 40
     t, _ = weight(rng, vocab, d, g.Q8, "embed")
@@ -347,6 +347,94 @@ def test_readout_of_non_finite_rows_and_streams():
     live = [r for r in range(nrows) if r not in (3, 17)]
     assert np.array_equal(got[live], ref.cpu().numpy()[live])
     assert not np.isfinite(got[3, :26]).any() and np.isnan(got[17]).all()
+
+
+class _Readouts:
+    """Label readouts of one weight on inputs that are uploaded and outputs
+    that are allocated before the first of them is queued."""
+
+    def __init__(self, sizes, vocab=6000, d=512, nlabels=26):
+        rng = np.random.default_rng(sum(sizes))
+        self.t, _ = weight(rng, vocab, d, g.Q8, "embed")
+        self.nlabels = nlabels
+        self.labels = dev(np.arange(nlabels, dtype=np.int32))
+        self.rows = [dev(rng.standard_normal((n, d)).astype(np.float32)) for n in sizes]
+        self.out = [torch.zeros((n, nlabels + 1), dtype=torch.float32, device="cuda") for n in sizes]
+        alone = g.DeviceWeight(self.t)
+        self.want = []
+        for i in range(len(sizes)):
+            self.call(alone, i, None)
+            torch.cuda.synchronize()
+            self.want.append(self.out[i].clone())
+            self.out[i].zero_()
+        torch.cuda.synchronize()
+
+    def call(self, w, i, stream):
+        w.label_readout(self.rows[i].data_ptr(), len(self.rows[i]), self.labels.data_ptr(), self.nlabels, 0.0,
+                        self.out[i].data_ptr(), stream)
+
+    def check(self):
+        torch.cuda.synchronize()
+        for i, (got, want) in enumerate(zip(self.out, self.want)):
+            assert torch.equal(got, want), f"call {i}"
+
+
+def test_readout_scratch_of_overlapping_streams():
+    """Calls with one weight queued in turn on three streams (the null stream
+    among them) with nothing waited for in between, small and large ones so
+    that the kept scratch is too small, in use elsewhere and handed on: each
+    gives the rows it gives alone."""
+    r = _Readouts([180, 3, 70, 200, 40, 1] * 6)
+    w = g.DeviceWeight(r.t)
+    streams = [None, torch.cuda.Stream().cuda_stream, torch.cuda.Stream().cuda_stream]
+    for i in range(len(r.rows)):
+        r.call(w, i, streams[i % 3])
+    r.check()
+
+
+def test_readout_scratch_grows_on_one_stream():
+    """Small, large, small, larger on one stream without a wait: the larger
+    block replaces the kept one behind the calls that still use it."""
+    r = _Readouts([2, 120, 5, 64, 200, 33, 1, 230])
+    w = g.DeviceWeight(r.t)
+    s = torch.cuda.Stream().cuda_stream
+    for i in range(len(r.rows)):
+        r.call(w, i, s)
+    r.check()
+
+
+def test_readout_scratch_outlives_its_streams():
+    """Streams made, used once and destroyed (a new one can have the handle
+    of an old one): every call gives the rows it gives alone."""
+    import ctypes
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    r = _Readouts([150, 2, 90, 40] * 4)
+    w = g.DeviceWeight(r.t)
+    for i in range(len(r.rows)):
+        s = ctypes.c_void_p()
+        assert hip.hipStreamCreate(ctypes.byref(s)) == 0
+        r.call(w, i, s.value)
+        assert hip.hipStreamDestroy(s) == 0
+    r.check()
+
+
+def test_readout_under_capture():
+    """A call that is being captured takes scratch of its own: the graph's
+    replays give the eager rows, with eager calls on the kept scratch in
+    between."""
+    r = _Readouts([60, 100])
+    w = g.DeviceWeight(r.t)
+    r.call(w, 0, None)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        r.call(w, 1, torch.cuda.current_stream().cuda_stream)
+    for _ in range(3):
+        r.out[0].zero_()
+        r.out[1].zero_()
+        graph.replay()
+        r.call(w, 0, None)
+        r.check()
 
 
 # Wide tiles: a 7,944-column product makes more than one round of tiles from
