@@ -581,8 +581,11 @@ int omg_dev_label_readout(const omg_weight* embed, const float* rows, int64_t nr
         if (nrows <= 0 || nlabels <= 0) omg::fail(omg::E_INVALID, "label readout: no rows or no labels");
         const hipStream_t s = static_cast<hipStream_t>(stream);
         const omg::DevWeight& E = embed->t.w;
-        embed->scratch.with(s, size_t(omg::label_readout_bytes(nrows, E.rows, nlabels, E.cols)), [&](void* p) {
-            omg::launch_label_readout(s, E, rows, nrows, labels, nlabels, softcap, out, p);
+        const int64_t own = omg::label_readout_bytes(nrows, E.rows, E.cols);
+        const int64_t full = omg::label_logits_bytes(nrows, E.rows, nlabels);
+        embed->scratch.with(s, size_t(own + full), [&](void* p) {
+            omg::launch_label_readout(s, E, rows, nrows, labels, nlabels, softcap, out, p,
+                                      reinterpret_cast<float*>(static_cast<uint8_t*>(p) + own));
         });
     });
 }

@@ -295,8 +295,8 @@ std::unique_ptr<Engine> Builder::finish(int64_t capacity, int64_t max_rows) {
     const int64_t width = std::max(c.vocab, d);
     E.logits_ = DevBuf(size_t(max_rows * width) * 4);
     E.label_lse_ = DevBuf(size_t(max_rows * (c.vocab + 1)) * 4);
-    // the readout's partials, full rows and split rows
-    E.readout_ = DevBuf(size_t(label_readout_bytes(max_rows, c.vocab, c.vocab, d)));
+    // the readout's partials and split rows (its full rows: logits_)
+    E.readout_ = DevBuf(size_t(label_readout_bytes(max_rows, c.vocab, d)));
     E.kv_stage_ = DevBuf(size_t(E.cap_pad_ * 2 * c.kv_heads * hd) * 2);
     if (c.per_layer_dim > 0) {
         const int64_t P = c.per_layer_dim;
@@ -1186,7 +1186,7 @@ void Engine::readout(const PassPlan& p) {
         // only k + 1 floats per row leave the device.
         step("label_readout", 0, [&] {
             launch_label_readout(stream_, embed_.w, rows_.as<float>(), p.nrows, d_labels_, p.nlabels, c.softcap,
-                                 label_lse_.as<float>(), readout_.p);
+                                 label_lse_.as<float>(), readout_.p, logits_.as<float>());
         });
     }
 }

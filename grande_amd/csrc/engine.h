@@ -227,7 +227,8 @@ class Engine {
     const int32_t* d_wanted_ = nullptr;
     const uint32_t* d_labels_ = nullptr;
     // Label logits + full-row log-sum-exp per wanted row (WANT_LABELS_LSE),
-    // and the logits kernel's per-workgroup (max, sum of exp) pairs.
+    // and the readout's scratch (launch_label_readout: the logits kernel's
+    // (max, sum of exp) pairs, the split rows).
     DevBuf label_lse_, readout_;
     DevBuf x16_, pli_, plg_, pl16_;  // per-layer inputs: f16(x), [t][layers x P] f32, gate f32, gated f16
     // attention chunk lengths in key tiles: [0] sliding layers, [1] global

@@ -126,18 +126,20 @@ struct LogitsOut {
     float* lab_out = nullptr;
 };
 // logits[r][j] = rows[r] . deq(E[cols ? cols[j] : j]) (softcap applied), at
-// f32 precision, from E's stage tiles.  `scratch` (split_rows_bytes, used
-// above 32 rows) may be null: then the workgroups split the rows themselves.
+// f32 precision, from E's stage tiles.  `scratch` (split_rows_bytes) may be
+// null: then the workgroups split the rows themselves.
 void launch_logits(hipStream_t s, const DevWeight& E, const float* rows, int64_t nrows, const uint32_t* cols,
                    int64_t ncols, float softcap, const LogitsOut& o, void* scratch);
 int64_t logits_blocks(int64_t ncols);
 int64_t split_rows_bytes(int64_t nrows, int64_t K);
 // The label readout (launch_logits, then launch_label_lse) into out
 // [nrows][nlabels + 1], its scratch (label_readout_bytes, 256-byte aligned)
+// and the full rows it needs for many labels (label_logits_bytes, 0: none)
 // the caller's.
 void launch_label_readout(hipStream_t s, const DevWeight& E, const float* rows, int64_t nrows, const uint32_t* labels,
-                          int64_t nlabels, float softcap, float* out, void* scratch);
-int64_t label_readout_bytes(int64_t nrows, int64_t vocab, int64_t nlabels, int64_t K);
+                          int64_t nlabels, float softcap, float* out, void* scratch, float* logits);
+int64_t label_readout_bytes(int64_t nrows, int64_t vocab, int64_t K);
+int64_t label_logits_bytes(int64_t nrows, int64_t vocab, int64_t nlabels);
 // The same with its scratch in a fixed device array instead of allocated
 // memory: nothing is allocated; nrows x vocab + 2 x nrows x ceil(vocab / 64)
 // floats must fit its 4,194,304.

@@ -1348,22 +1348,20 @@ static void label_readout(hipStream_t s, const DevWeight& E, const float* rows, 
     launch_label_lse(s, logits, nrows, E.rows, part, logits_blocks(E.rows), labels, nlabels, out);
 }
 
-// Scratch layout: partials, then (more labels than a scan takes) the full
-// rows, then the split rows.
+// Scratch layout: partials, then the split rows.
 static int64_t a256(int64_t n) { return (n + 255) / 256 * 256; }
-int64_t label_readout_bytes(int64_t nrows, int64_t vocab, int64_t nlabels, int64_t K) {
-    return a256(logits_blocks(vocab) * nrows * 8) + (nlabels > LABEL_SCAN ? a256(nrows * vocab * 4) : 0) +
-           split_rows_bytes(nrows, K);
+int64_t label_readout_bytes(int64_t nrows, int64_t vocab, int64_t K) {
+    return a256(logits_blocks(vocab) * nrows * 8) + a256(split_rows_bytes(nrows, K));
+}
+int64_t label_logits_bytes(int64_t nrows, int64_t vocab, int64_t nlabels) {
+    return nlabels > LABEL_SCAN ? nrows * vocab * 4 : 0;
 }
 void launch_label_readout(hipStream_t s, const DevWeight& E, const float* rows, int64_t nrows, const uint32_t* labels,
-                          int64_t nlabels, float softcap, float* out, void* scratch) {
+                          int64_t nlabels, float softcap, float* out, void* scratch, float* logits) {
     if (nrows <= 0 || nlabels <= 0) fail(E_INVALID, "label readout: no rows or no labels");
     uint8_t* p = static_cast<uint8_t*>(scratch);
-    float2* part = reinterpret_cast<float2*>(p);
-    p += a256(logits_blocks(E.rows) * nrows * 8);
-    float* logits = reinterpret_cast<float*>(p);
-    if (nlabels > LABEL_SCAN) p += a256(nrows * E.rows * 4);
-    label_readout(s, E, rows, nrows, labels, nlabels, softcap, out, logits, part, p);
+    label_readout(s, E, rows, nrows, labels, nlabels, softcap, out, logits, reinterpret_cast<float2*>(p),
+                  p + a256(logits_blocks(E.rows) * nrows * 8));
 }
 
 void launch_label_readout_noalloc(hipStream_t s, const DevWeight& E, const float* rows, int64_t nrows,

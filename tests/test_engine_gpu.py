@@ -430,10 +430,9 @@ def test_label_lse_readout():
 
 
 def test_logits_many_rows_and_wide_rows():
-    """The logits kernel's edges: more readout rows than one pass of the
-    kernel takes (44 rows: three passes of 16), a model width spanning two
-    staged K chunks (d 576 = 512 + 64) and a vocabulary that ends inside a
-    workgroup's 64 columns (300).  Every row against the oracle's logits
+    """The logits kernel's edges: more readout rows than a row tile (44: 32
+    and 12), an odd number of K stages (d 576 = 9 x 64) and a vocabulary that
+    ends inside a 32-column tile (300).  Every row against the oracle's logits
     of the engine's own hidden rows (reference.rs:564-598's 1e-3 of the
     scale); label columns and LABELS_LSE's columns bit-equal to the full
     row; the log-sum-exp within 1e-5 of the float64 one."""
@@ -459,6 +458,39 @@ def test_logits_many_rows_and_wide_rows():
             exp_lse = m + np.log(np.exp(r64 - m).sum())
             assert abs(ls[-1] - exp_lse) <= 1e-5 * max(1.0, abs(exp_lse))
     assert nrows == 44
+
+
+def test_readout_memory_and_many_labels():
+    """What a large vocabulary adds to an engine's device memory: the full
+    logits and the label columns, rows x vocabulary floats each, and no third
+    such buffer (the embedding and the partials take under a quarter of one).
+    More labels than a column tile scans (512) read their columns from the
+    full logits: the same bits as the LOGITS row, and its log-sum-exp."""
+    torch = pytest.importorskip("torch")
+    vocab, max_rows = 1 << 17, 512
+
+    def made(v):
+        w = g.Weights.synth(gguf_tiny(vocab=v), 3, g.Q4, g.Q4)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        eng = g.Engine.new(w, 64, max_rows)
+        return eng, free - torch.cuda.mem_get_info()[0]
+
+    first = made(1024)  # (it also loads what a process loads once)
+    small, base = made(1024)
+    eng, used = made(vocab)
+    rows = max_rows * (vocab - 1024) * 4
+    assert used - base < 2.25 * rows, f"{(used - base) / rows:.2f} full-logits buffers"
+    del first, small
+    labels = np.random.default_rng(1).integers(0, vocab, 700).tolist()
+    full = eng.evaluate(PREFIX, BRANCHES, Want.LOGITS)
+    got = eng.evaluate(PREFIX, BRANCHES, Want.LABELS_LSE, labels)
+    for fo, lo in zip(full, got):
+        for row, r in zip(fo.rows, lo.rows):
+            assert np.array_equal(r[:-1], row[labels])
+            z = row.astype(np.float64)
+            lse = z.max() + np.log(np.exp(z - z.max()).sum())
+            assert abs(r[-1] - lse) <= 1e-5 * max(1.0, abs(lse))
 
 
 def test_refused_request_leaves_resident_prefix_intact():
