@@ -17,10 +17,12 @@
 // (q - 8) * d (or q * d) to f16 once, the reference's f16 rounding point
 // (shaders/weight.wgsl:40-54).
 //
-// Two kernels with the same sums: gemm32_kernel (fragments of a whole stage
-// at a time; short products, where a tile's own latency counts) and
+// Three kernels with the same sums: gemm32_kernel (fragments of a whole stage
+// at a time; short products, where a tile's own latency counts),
 // gemm32w_kernel (fragments one k-step ahead, so twice the tile in the same
-// registers; products of more than one round of tiles).
+// registers; products of more than one round of tiles) and gemm32l_kernel
+// (f16 weights, which have nothing to decode: they go through LDS like X and
+// every wave of a tile reads them from there).
 //
 // X tiles are 128 B per row with the 16 B chunk c of row r stored at
 // c ^ ((r >> 1) & 7), so the rows of one fragment read hit distinct banks.
@@ -137,8 +139,7 @@ __device__ inline float gelu_tanh(float x) {
 
 // ------------------------------------------------------ 32x32x16 tiles
 
-// The decoder's products (f32 out and the gated GeGLU) on
-// v_mfma_f32_32x32x16_f16, which issues at full rate on gfx950 with one or
+// gemm32_kernel, on v_mfma_f32_32x32x16_f16, which issues at full rate on gfx950 with one or
 // two accumulation chains per wave (16x16x32 needs about sixteen).  Row-
 // owner scheme: each wave owns 32 * NJ weight rows across all BM = 32 * MI
 // activation rows, so its weights are private to it and go straight from
@@ -1118,6 +1119,184 @@ __global__ __launch_bounds__(NW_ * WAVE, 2) void gemm32w_kernel(GemmArgs g) {
     }
 }
 
+// f16 weights.  Nothing is decoded, so no wave has to own its weight rows:
+// both operands of a stage go by LDS DMA into a ring slot and 2 x 2 waves
+// each take 32 MI rows by 32 NJ weight rows of the tile.  With the weights in
+// registers (gemm32w_kernel) three row blocks were the most that fit and every
+// weight passed L2 once per 96 rows.  The same products, operand layouts and K
+// order as the other two, so the same sums.  Fragments are read one k-step
+// ahead, and a slot is refilled as soon as everyone holds its last fragments:
+// two workgroups share a CU and cover each other's waits.
+//
+// Isolated products (16x16x32 tiles with the weights through LDS / weights in
+// registers -> this): erf-gated, N 2 x 1,152, K 768: 49,152 rows 199 / 230 ->
+// 193 us, 8,192 41 / 49 -> 41, 500 10.8 / 11.4 -> 8.4; [q | k | v] heads, N
+// 2,304, K 768: 49,152 rows 343 / 265 -> 235, 300 11.0 / 12.5 -> 9.0; f32, N
+// 768, K 1,152, 49,152 rows 135 (128 x 128, weights in registers) / 137 ->
+// 115; tanh-gated, N 2 x 6,912, K 1,152, 2,384 rows 135 / 122 -> 86.
+//
+// A weight packet's lane runs (kernels.h: 64 bytes of lane l at 64 l) keep
+// their place, with the run's four 16-byte k-steps at ks ^ ((l >> 2) & 3): the
+// sixteen lanes of a read's quarter then hit distinct banks.
+template <int MI, int NJ, int EPI, int NS, int WM, int WN>
+struct CfgL {
+    static constexpr bool GATED = EPI == EPI_GELU_TANH || EPI == EPI_GELU_ERF;
+    static constexpr int NW = WM * WN, T = NW * WAVE;
+    static constexpr int BM = 32 * MI * WM;
+    static constexpr int WR = 32 * NJ;                // weight rows per wave
+    static constexpr int BNW = WN * WR;               // weight rows per tile
+    static constexpr int BN = GATED ? BNW / 2 : BNW;  // output columns per tile
+    static constexpr int PK = tile_packet_bytes(F16_DT);
+    static constexpr int X_CH = BM * 8, X_I = (X_CH + T - 1) / T, X_BYTES = X_I * T * 16;
+    static constexpr int W_BYTES = BNW / 32 * PK, W_I = W_BYTES / (T * 16);
+    static constexpr int C = X_I + W_I;               // memory instructions per wave and stage
+    static constexpr int STAGE = X_BYTES + W_BYTES, LDS = NS * STAGE;
+    static_assert(!GATED || NJ % 2 == 0, "gated tiles pair gate and up row blocks");
+    static_assert(W_BYTES % (T * 16) == 0, "whole DMA instructions per stage of weights");
+    static_assert(LDS <= 160 * 1024, "ring larger than the LDS");
+    static_assert(NS >= 2 && (NS - 1) * C <= 63, "vmcnt range");
+};
+
+template <int MI, int NJ, int EPI, int NS, int WM, int WN>
+__global__ __launch_bounds__(WM * WN * WAVE, 2) void gemm32l_kernel(GemmArgs g) {
+    using P = CfgL<MI, NJ, EPI, NS, WM, WN>;
+    constexpr bool GATED = P::GATED;
+    constexpr int NW = P::NW, BM = P::BM, BN = P::BN, WR = P::WR, PK = P::PK;
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = int(threadIdx.x), lane = tid % WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int wm = wave % WM, wn = wave / WM;
+    const int64_t N = g.w0.rows, K = g.w0.cols, M = g.m;
+    const int ntn = int((N + BN - 1) / BN);
+    const int ntiles = ntn * int((M + BM - 1) / BM);
+    const int per_xcd = int(gridDim.x) / 8;
+    const int tile = (int(blockIdx.x) % 8) * per_xcd + int(blockIdx.x) / 8;
+    if (tile >= ntiles) return;
+    const int64_t n0 = int64_t(tile % ntn) * BN, m0 = int64_t(tile / ntn) * BM;
+    const int kbeg = int(blockIdx.y) * int(K / g.ksplit);
+    const int nk = int((K / g.ksplit + G_BK - 1) / G_BK);
+    const int K32 = int(K), last = nk - 1;
+
+    uint32_t xoff[P::X_I];
+    int xcol[P::X_I];
+#pragma unroll
+    for (int i = 0; i < P::X_I; ++i) {
+        const int slot = (i * NW + wave) * WAVE + lane;
+        const int r = slot / 8, lc = (slot % 8) ^ swz(r);
+        xcol[i] = lc * 8;
+        xoff[i] = slot < P::X_CH && m0 + r < M ? uint32_t(((m0 + r) * g.ldx + lc * 8) * 2) : OOB;
+    }
+    // Weight blocks of the tile in LDS: wave column wn's NJ in order (gated:
+    // its gate blocks, then the same blocks of the up matrix).  A DMA
+    // instruction moves a quarter of one, 1 KB.
+    const int64_t stages = g.w0.stages, rblocks = (N + 31) / 32, rb0 = n0 / 32;
+    const int64_t live_blocks = rblocks - rb0;  // > 0: the tile starts inside N
+    uint32_t woff[P::W_I];
+    bool wup[P::W_I];
+#pragma unroll
+    for (int i = 0; i < P::W_I; ++i) {
+        const int q = i * NW + wave, b = q / 4, j = b % NJ;
+        wup[i] = GATED && j >= NJ / 2;
+        const int blk = GATED ? b / NJ * (NJ / 2) + j % (NJ / 2) : b;
+        woff[i] = blk < live_blocks ? uint32_t(blk * stages * PK + (q % 4) * 1024 + (lane / 4) * 64 +
+                                               ((lane % 4) ^ ((lane / 16) & 3)) * 16)
+                                    : OOB;
+    }
+    // Stages past the end repeat the last one (in range, never consumed), so
+    // every wave always issues P::C instructions per stage.
+    auto slot_base = [&](int s) { return smem + (unsigned(s) % unsigned(NS)) * P::STAGE; };
+    const int64_t xbytes = M * g.ldx * 2;
+    const bool ktail = (K32 & (G_BK - 1)) != 0;
+    const int st0 = kbeg / G_BK;
+    auto issue = [&](int s) {
+        uint8_t* base = slot_base(s);
+        const int sc = s < last ? s : last;
+        const int k0 = __builtin_amdgcn_readfirstlane(kbeg + sc * G_BK);
+        const bool tail = ktail && k0 + G_BK > K32;
+#pragma unroll
+        for (int i = 0; i < P::X_I; ++i) {
+            const uint32_t o = tail && xcol[i] >= K32 - k0 ? OOB : xoff[i];
+            const __amdgpu_buffer_rsrc_t r = rsrc(g.x, xbytes);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(base + (i * NW + wave) * WAVE * 16), 16, o,
+                                                     k0 * 2, 0, 0);
+        }
+        // (The offset is a named value: read from its array in the call, the
+        // host-side compile drops this kernel.)
+        const int st = __builtin_amdgcn_readfirstlane(st0 + sc);
+#pragma unroll
+        for (int i = 0; i < P::W_I; ++i) {
+            const uint32_t o = woff[i];
+            const DevWeight& wt = wup[i] ? g.w1 : g.w0;
+            const __amdgpu_buffer_rsrc_t r = rsrc(wt.tiles + rb0 * stages * PK, live_blocks * stages * PK);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                r, (lds_ptr_t)(base + P::X_BYTES + (i * NW + wave) * WAVE * 16), 16, o, st * PK, 0, 0);
+        }
+    };
+    auto fence = [] { asm volatile("" ::: "memory"); };
+
+    floatx16 acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = floatx16{};
+    const int lr = lane % 32, lh = lane / 32;
+    int foff[4], goff[4];  // the lane's X and weight fragment offsets per k-step
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        foff[ks] = (wm * MI * 32 + lr) * G_ROW + (((2 * ks + lh) ^ swz(lr)) * 16);
+        goff[ks] = P::X_BYTES + wn * NJ * PK + lane * 64 + (ks ^ ((lane / 4) & 3)) * 16;
+    }
+    struct Frag {
+        half8 x[MI], w[NJ];
+    };
+    auto read = [&](int s, int ks, Frag& f) {
+        const uint8_t* S = slot_base(s);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) f.w[j] = *reinterpret_cast<const half8*>(S + goff[ks] + j * PK);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) f.x[i] = *reinterpret_cast<const half8*>(S + foff[ks] + i * 32 * G_ROW);
+    };
+    // One k-step: the next one's fragment reads spread over this one's
+    // products; nothing moves across its ends.
+    auto kstep = [&](int s, int ks, const Frag& cur, Frag& nxt) {
+        read(s, ks, nxt);
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur.w[j], cur.x[i], acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < MI + NJ; ++u) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                     // LDS read
+            __builtin_amdgcn_sched_group_barrier(0x008, MI * NJ / (MI + NJ), 0);  // MFMA
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Frag fa, fb;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) issue(s);
+    fence();
+    wait_vm<(NS - 1) * P::C>();
+    lds_barrier();
+    read(0, 0, fa);
+    for (int kt = 0; kt < nk; ++kt) {
+        kstep(kt, 1, fa, fb);
+        kstep(kt, 2, fb, fa);
+        kstep(kt, 3, fa, fb);
+        // Stage kt + 1 landed (this wave's part; past the barrier
+        // everyone's, and everyone holds stage kt's last fragments).
+        fence();
+        wait_vm<(NS - 2) * P::C>();
+        lds_barrier();
+        issue(kt + NS);
+        fence();
+        __builtin_amdgcn_sched_barrier(0);
+        kstep(kt + 1, 0, fb, fa);
+    }
+    wait_vm<0>();  // no DMA into LDS outlives the workgroup
+    finish32<MI, NJ, EPI, true>(g, acc, m0 + wm * MI * 32, n0 + (GATED ? wn * (WR / 2) : wn * WR), lane);
+}
+
 // Resident X tiles up to this many bytes of LDS (one workgroup per CU
 // above half of it).
 constexpr int XR_MAX_LDS = 96 * 1024;
@@ -1175,6 +1354,24 @@ static void run32w(hipStream_t s, const GemmArgs& g) {
     OMG_HIP(hipGetLastError());
 }
 
+template <int MI, int NJ, int EPI, int NS, int WM = 2, int WN = 2>
+static void run32l(hipStream_t s, const GemmArgs& g) {
+    using P = CfgL<MI, NJ, EPI, NS, WM, WN>;
+    for (const DevWeight* w : {&g.w0, &g.w1})
+        if (!w->tiles || w->stages != (w->cols + G_BK - 1) / G_BK) fail(E_INVALID, "gemm: weight without stage tiles");
+    if (g.mshift != 0 || g.kfold != 0) fail(E_INVALID, "gemm: row shift or K pieces");
+    static bool lds_set = false;
+    if (!lds_set) {
+        OMG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm32l_kernel<MI, NJ, EPI, NS, WM, WN>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, P::LDS));
+        lds_set = true;
+    }
+    const int64_t tiles = ((g.w0.rows + P::BN - 1) / P::BN) * ((g.m + P::BM - 1) / P::BM);
+    const dim3 grid(unsigned((tiles + 7) / 8 * 8), unsigned(g.ksplit));
+    gemm32l_kernel<MI, NJ, EPI, NS, WM, WN><<<grid, dim3(P::T), P::LDS, s>>>(g);
+    OMG_HIP(hipGetLastError());
+}
+
 // Row blocks (of 32) of the wide tile, at least LO: a workgroup of MI blocks
 // takes about 1 + MI units of time whatever the product, and ROUND tiles run
 // at a time, so the MI with the least rounds x (1 + MI) is taken (the larger
@@ -1207,11 +1404,28 @@ static void run_wide(hipStream_t s, const GemmArgs& g, int64_t cols_per_tile) {
     return run32w<QUANT, 2, 2, EPI, 4, 4>(s, g);
 }
 
+// f16 weights through LDS: 64, 128 or 192 rows x 128 weight rows.  64 while
+// those tiles make one round of the 256 CUs; past it the two large tiles run
+// two to a CU, 512 at a time, and take about three and four units: the least
+// rounds x units (the larger tile of equals).  Over 34 products from 900 to
+// 49,152 rows (erf-gated, q/k/v heads, bias + ReLU, f32, tanh-gated) it picks
+// the faster of the two or one within 6% of it.
+template <int EPI, bool SHORT = true>
+static void run_lds(hipStream_t s, const GemmArgs& g, int64_t cols_per_tile) {
+    const int64_t ntn = (g.w0.rows + cols_per_tile - 1) / cols_per_tile * g.ksplit;
+    auto tiles = [&](int64_t rows) { return (g.m + rows - 1) / rows * ntn; };
+    if constexpr (SHORT)
+        if (tiles(64) <= 256) return run32l<1, 2, EPI, 3>(s, g);
+    if (4 * ((tiles(192) + 511) / 512) <= 3 * ((tiles(128) + 511) / 512)) return run32l<3, 2, EPI, 2>(s, g);
+    run32l<2, 2, EPI, 2>(s, g);
+}
+
 // Tile choice, measured on MI355X (tiles are activation rows x weight rows;
-// both kernels give every output element the same sums, so rows never
+// every kernel gives every output element the same sums, so rows never
 // depend on M).  gemm32_kernel, whose K loop has the shorter stages, while
-// its tiles make one round of the 256 CUs; above that the wide tiles.
-// Isolated products, 16x16x32 tiles / gemm32_kernel before -> now:
+// its tiles make one round of the 256 CUs; above that the wide tiles, or for
+// f16 weights the ones through LDS (figures there).  Isolated products,
+// 16x16x32 tiles / gemm32_kernel before -> now:
 //   [q | k | v] heads, N 2,304, K 768, Q8: 49,152 rows 303 -> 236 us, 6,000
 //   53 -> 33, 3,000 32 -> 21, 500 18.5 -> 9.8; erf-gated, N 2 x 1,152: 226
 //   -> 204, 53 -> 28, 33 -> 17, 12.1 -> 9.1; o, N 768: 84 -> 79, 20.8 ->
@@ -1224,14 +1438,27 @@ template <int QUANT, int EPI>
 static void dispatch(hipStream_t s, const GemmArgs& g) {
     const int64_t N = g.w0.rows, K = g.w0.cols, M = g.m;
     auto tiles = [&](int64_t rows, int64_t cols) { return (M + rows - 1) / rows * ((N + cols - 1) / cols) * g.ksplit; };
+    auto rounds = [&](int64_t rows, int64_t cols) { return (tiles(rows, cols) + 255) / 256; };
     if constexpr (EPI == EPI_QKV) {
         // a 64-wide head per wave
-        if (tiles(32, 256) <= 256) return run32<QUANT, 1, 2, EPI, 4, 4>(s, g);
-        if (tiles(64, 256) <= 256) return run32<QUANT, 2, 2, EPI, 4, 4>(s, g);
-        return run_wide<QUANT, EPI>(s, g, 256);
+        if constexpr (QUANT == F16_DT) return run_lds<EPI>(s, g, 128);
+        if constexpr (QUANT != F16_DT) {
+            if (tiles(32, 256) <= 256) return run32<QUANT, 1, 2, EPI, 4, 4>(s, g);
+            if (tiles(64, 256) <= 256) return run32<QUANT, 2, 2, EPI, 4, 4>(s, g);
+            return run_wide<QUANT, EPI>(s, g, 256);
+        }
     } else if constexpr (EPI == EPI_RELU_F16) {
-        if (tiles(32, 128) <= 256) return run32<QUANT, 1, 1, EPI, 4, 4>(s, g);
-        return run_wide<QUANT, EPI>(s, g, 256);
+        if constexpr (QUANT == F16_DT) {
+            // 64 x 64 up to a round of those (N 3,072, K 768, 32 x 128 with
+            // the weights in registers -> this: 150 rows 9.3 -> 7.5 us, 300
+            // 11.2 -> 8.0)
+            if (M <= 64) return run32<QUANT, 1, 1, EPI, 4, 4>(s, g);
+            if (tiles(64, 64) <= 256) return run32l<1, 1, EPI, 4>(s, g);
+            return run_lds<EPI>(s, g, 128);
+        } else {
+            if (tiles(32, 128) <= 256) return run32<QUANT, 1, 1, EPI, 4, 4>(s, g);
+            return run_wide<QUANT, EPI>(s, g, 256);
+        }
     } else if constexpr (EPI == EPI_QKPREP) {
         // One head on eight waves of one 32-row weight block each (half the
         // decode per wave and K stage of the four-wave tile): short passes,
@@ -1255,12 +1482,15 @@ static void dispatch(hipStream_t s, const GemmArgs& g) {
             return run32w<QUANT, 3, 1, EPI, 3, 4, true>(s, g);
         }
         if (M <= 512 && tiles(32, 128) <= 512) return run32<QUANT, 1, 1, EPI, 4, 4>(s, g);
-        if (g.ksplit > 1 && tiles(96, 128) <= 256) return run32<QUANT, 3, 1, EPI, 4, 4>(s, g);
+        if ((g.ksplit > 1 || (QUANT == F16_DT && tiles(64, 128) > 256)) && tiles(96, 128) <= 256)
+            return run32<QUANT, 3, 1, EPI, 4, 4>(s, g);
         if (g.ksplit == 1 && tiles(64, 128) <= 256) return run32<QUANT, 2, 1, EPI, 4, 4>(s, g);
-        // 128 x 256 (five units a round) against 96 x 128 (2.4)
-        if (QUANT == F16_DT || 50 * ((tiles(128, 256) + 255) / 256) > 24 * ((tiles(96, 128) + 255) / 256))
-            return run32w<QUANT, 3, 1, EPI, 3, 4>(s, g);
-        if constexpr (QUANT != F16_DT) return run32w<QUANT, 4, 2, EPI, 3, 4>(s, g);
+        if constexpr (QUANT == F16_DT) return run_lds<EPI, false>(s, g, 128);
+        if constexpr (QUANT != F16_DT) {
+            // 128 x 256 (five units a round) against 96 x 128 (2.4)
+            if (50 * rounds(128, 256) > 24 * rounds(96, 128)) return run32w<QUANT, 3, 1, EPI, 3, 4>(s, g);
+            return run32w<QUANT, 4, 2, EPI, 3, 4>(s, g);
+        }
     } else {
         // Branch-sized passes (M <= 64) pair the waves (a gate and an up
         // wave per 32 columns: half the decode per wave and stage; flushed
@@ -1274,8 +1504,11 @@ static void dispatch(hipStream_t s, const GemmArgs& g) {
             if (K <= 1024) return run32<QUANT, 1, 1, EPI, 9, 2, false, true>(s, g);
             return run32<QUANT, 2, 1, EPI, 4, 4, false, true>(s, g);
         }
-        if (tiles(32, 128) <= 256) return run32<QUANT, 1, 2, EPI, 4, 4>(s, g);
-        return run_wide<QUANT, EPI>(s, g, 128);
+        if constexpr (QUANT == F16_DT) return run_lds<EPI>(s, g, 64);
+        if constexpr (QUANT != F16_DT) {
+            if (tiles(32, 128) <= 256) return run32<QUANT, 1, 2, EPI, 4, 4>(s, g);
+            return run_wide<QUANT, EPI>(s, g, 128);
+        }
     }
 }
 

@@ -438,10 +438,10 @@ def test_readout_under_capture():
 
 
 # Wide tiles: a 7,944-column product makes more than one round of tiles from
-# a few dozen rows on, so the rows below pass through the short tiles, every
-# wide row-block count and its partial last tile (and columns past the last
-# whole tile); K 96 and 160 end in half a stage, 320 and 640 have an odd and
-# an even stage count.
+# a few dozen rows on, so the rows below pass through the short tiles and
+# wide ones of several row-block counts (and columns past the last whole
+# tile); K 96 and 160 end in half a stage, 320 and 640 have an odd and an even
+# stage count.
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("k", [96, 160, 320, 640])
 def test_wide_tiles_give_the_short_tiles_rows(k, dtype):
@@ -486,4 +486,67 @@ def test_wide_tiles_give_the_short_tiles_rows(k, dtype):
             from math import erf
             z = a[:40]
             z = (gelu(z) if kind == "tanh" else 0.5 * z * (1.0 + np.vectorize(erf)(z / np.sqrt(2.0)))) * u[:40]
+            assert np.max(np.abs(got[:40] - z) / np.maximum(np.abs(z), 1.0)) < 2e-3
+
+
+# 7,944 columns again, at the rows where the choice of a tile changes (and one
+# past them): f32 32 x 128, 64 x 128, 96 x 128, 128 x 256 and with f16 weights
+# 96 x 128, 128 x 128, 192 x 128; bias + ReLU on two and four waves, one to four
+# wide row blocks, f16 64 x 64 up to 192 x 128; the gated products' paired, short
+# and wide tiles, f16 64 to 192 rows.
+TILE_ROWS = (1, 33, 65, 100, 129, 200, 257, 300, 385, 450, 513, 700, 769, 801, 1000, 1025)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("k,ldx,ldy,shift", [(96, 96, 7944, 0), (320, 336, 7956, 0), (160, 168, 7944, 4)])
+def test_every_tile_gives_the_same_rows(k, ldx, ldy, shift, dtype):
+    """A row's outputs are the same bits whatever M selects, with X rows
+    further apart than K and with output rows or a base off the 16 bytes that
+    the eight-column f16 stores want (they fall back to four columns: ldy
+    7,956, or the base four columns in), and match float64: f32 sums of K
+    products within 2^-23 K of sum |x||w|, f16 outputs half an ulp more.
+    Columns past N stay as they were."""
+    from math import erf
+    rng = np.random.default_rng(7 * k + dtype)
+    n, rows = 7944, 1090
+    (tg, gd), (tu, ud) = weight(rng, n, k, dtype, "gate"), weight(rng, n, k, dtype, "up")
+    wg, wu = g.DeviceWeight(tg), g.DeviceWeight(tu)
+    bias = rng.uniform(-1, 1, n).astype(np.float16)
+    x = rng.uniform(-1, 1, (rows, ldx)).astype(np.float16)
+    bd, xd = dev(bias), dev(x)
+
+    def run(m, kind):
+        y = torch.full((m * ldy + 16,), 7.0, dtype=torch.float32 if kind == "f32" else torch.float16, device="cuda")
+        at = 0 if kind == "f32" else shift
+        p = y.data_ptr() + 2 * at
+        if kind == "f32":
+            wg.gemm(xd.data_ptr(), ldx, m, p, ldy)
+        elif kind == "relu":
+            wg.gemm_bias_relu(xd.data_ptr(), ldx, m, bd.data_ptr(), p, ldy)
+        else:
+            (wg.gemm_geglu if kind == "tanh" else wg.gemm_geglu_erf)(wu, xd.data_ptr(), ldx, m, p, ldy)
+        torch.cuda.synchronize()
+        y = y.cpu().numpy()
+        assert (y[:at] == 7.0).all() and (y[at + m * ldy:] == 7.0).all()
+        y = y[at:at + m * ldy].reshape(m, ldy)
+        assert (y[:, n:] == 7.0).all(), f"{kind} columns past N at M {m}"
+        return y[:, :n]
+
+    xf = x[:, :k].astype(np.float64)
+    a, mass = xf @ gd.T, np.abs(xf) @ np.abs(gd).T
+    u = xf[:40] @ ud.T
+    bound = 2.0 ** -23 * k * mass
+    for kind in ("f32", "relu", "tanh", "erf"):
+        full = run(rows, kind)
+        for m in TILE_ROWS:
+            assert np.array_equal(run(m, kind), full[:m]), f"{kind} rows at M {m}"
+        got = full.astype(np.float64)
+        if kind == "f32":
+            assert (np.abs(got - a) <= bound + 1e-30).all()
+        elif kind == "relu":
+            z = np.maximum(a + bias, 0.0)
+            assert (np.abs(got - z) <= bound + 2.0 ** -11 * np.abs(z) + 1e-7).all()
+        else:
+            z = a[:40]
+            z = (gelu(z) if kind == "tanh" else 0.5 * z * (1.0 + np.vectorize(erf)(z / np.sqrt(2.0)))) * u
             assert np.max(np.abs(got[:40] - z) / np.maximum(np.abs(z), 1.0)) < 2e-3

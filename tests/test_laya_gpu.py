@@ -110,6 +110,53 @@ def test_qkv_heads_epilogue(lengths, heads, rope, dtype):
         assert rel_diff(got, exp) < 2e-3, f"section {sec}"
 
 
+# Rows at which the tile changes (12 heads, N 2,304): f16 64, 128 and 192 rows,
+# quantized 32, 64 and wide tiles of two to four row blocks, each with a partial
+# last tile.
+@pytest.mark.parametrize("dtype", [g.F16, g.Q8, g.Q4])
+def test_qkv_heads_of_every_tile(dtype):
+    """q, k and V^T of a row are the same bits whatever M selects, the odd
+    last key of a launch among them, and the last rows match the f32 product
+    rotated and scaled."""
+    rng = np.random.default_rng(3 + dtype)
+    heads, rows = 12, 5461
+    d = 64 * heads
+    x = rng.uniform(-1, 1, (rows, d)).astype(np.float16)
+    wt, wd = qweight(rng, 3 * d, d, dtype, 0.15)
+    bias = (rng.uniform(-1, 1, 3 * d) * 0.2).astype(np.float16)
+    meta = pack_meta([257] * (rows // 257) + [rows % 257])
+    table = rope_table(10000.0, 512)
+    w = g.DeviceWeight(wt)
+    xd, bd, md, rd = dev(x), dev(bias), dev(meta), dev(table)
+
+    def run(t):
+        tpad = (t + 63) // 64 * 64
+        out = [torch.full((heads * tpad * 64,), 3.0, dtype=torch.float16, device="cuda") for _ in range(3)]
+        w.qkv_heads(xd.data_ptr(), d, t, bd.data_ptr(), rd.data_ptr(), md.data_ptr(), 0.125, tpad,
+                    *(o.data_ptr() for o in out))
+        torch.cuda.synchronize()
+        q, k, vt = (o.cpu().numpy() for o in out)
+        v = unpack_vt(vt, heads, tpad)
+        q, k = q.reshape(heads, tpad, 64), k.reshape(heads, tpad, 64)
+        assert (v[:, t:] == 3.0).all() and (q[:, t:] == 3.0).all() and (k[:, t:] == 3.0).all()
+        return [a[:, :t] for a in (q, k, v)]
+
+    full = run(rows)
+    for t in (1, 63, 500, 897, 1801, 2701, 3601, 5377):
+        for got, want in zip(run(t), full):
+            assert np.array_equal(got, want[:, :t]), f"{t} rows"
+    tail = slice(rows - 70, rows)
+    y = (x[tail].astype(np.float32) @ wd.T + bias.astype(np.float32)).reshape(70, 3, heads, 64)
+    cs = table[meta[tail, 0]]
+    c, sn = cs[:, None, :, 0], cs[:, None, :, 1]
+    for s in (0, 1):
+        a, b = y[:, s, :, :32].copy(), y[:, s, :, 32:].copy()
+        y[:, s, :, :32], y[:, s, :, 32:] = a * c - b * sn, b * c + a * sn
+    y[:, 0] *= 0.125
+    for s in range(3):
+        assert rel_diff(full[s][:, tail].astype(np.float32), y[:, s].transpose(1, 0, 2)) < 2e-3, f"section {s}"
+
+
 def attention_ref(q, k, v, meta, window):
     """float64 softmax(q . k) v over the visible keys of each row."""
     heads, t = q.shape[0], meta.shape[0]
