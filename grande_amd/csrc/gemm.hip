@@ -38,6 +38,7 @@
 // past M or N read as zero in hardware; in the K tail (K % 64 == 32) the X
 // lanes past K are sent out of range by their lane offset (a zero activation
 // times the packet's zero padding).
+#include <algorithm>
 #include <climits>
 #include <string>
 #include <utility>
@@ -1464,22 +1465,36 @@ static void dispatch(hipStream_t s, const GemmArgs& g) {
         // decode per wave and K stage of the four-wave tile): short passes,
         // and long ones whose 64-row X tile stays resident (K <= 768; the
         // 270M model's cold q/k/v 15.9 -> 13.3 us, its cold pass -3.2%).
-        // Longer K: wide tiles against 64 rows on four waves of the short
-        // stages, 4B model (K 2,560), 16,320 rows 388 -> 337 us, 8,800 217
-        // -> 198, 4,100 118 -> 105, 1,980 55.0 -> 55.8; 1B (K 1,152), 2,352
-        // rows 23.7 -> 24.1, 992 21.5 -> 19.6.
+        // Longer K: 64 rows on four waves of the short stages while the wide
+        // rule would take no more and two workgroups per CU hold them all
+        // (1B, K 1,152, Q4: 992 rows 17.0 us against 15.7, 2,352 18.1 against
+        // 16.8, f16 23.2 against 19.5; 4B, K 2,560, Q4, 1,980 rows 49.9
+        // against 49.3), past that wide tiles (16,320 rows 355 -> 324, 4,100
+        // 109 -> 96).
         if (M <= 512) return run32<QUANT, 1, 1, EPI, 4, 8>(s, g);
         if (K <= 768) return run32<QUANT, 2, 1, EPI, 4, 8>(s, g);
+        if (tiles(64, 256) <= 512 && wide_blocks<QUANT, 2, 512>(M, (N + 255) / 256) == 2)
+            return run32<QUANT, 2, 2, EPI, 4, 4>(s, g);
         return run_wide<QUANT, EPI, 2, 512>(s, g, 256);
     } else if constexpr (EPI == EPI_F32) {
         if (g.kfold > 0) {
-            // K pieces added in registers (up to 96-row tiles: the totals
-            // fit).  96 rows of the wide kernel against the short stages, 4B
-            // down (N 2,560, K 10,240): 16,320 rows 935 -> 896 us, 8,800 531
-            // -> 512, 3,000 214 -> 192, 1,980 133 -> 137; 128 rows were 884,
-            // 515, 180 and 153.
+            // K pieces added in registers (the totals take what a second
+            // weight block would).  A round of 64, 96 or 128 rows x 128 takes
+            // about 50, 62 or 84 units, one alone 65, 80 or 95, and the least
+            // sum is taken.  N 2,560, K 10,240, Q4 (96 rows of the short
+            // stages / of the wide kernel -> this): 560 rows 76 / 77 -> 63 us,
+            // 1,600 120 / 122 -> 107, 1,980 122 / 126 -> 122, 2,663 194 / 171
+            // -> 158, 16,320 904 / 871 -> 859; f16, 930 rows 74 / 109 -> 74.
+            // The wide kernel's 96 rows only past four rounds, where it is 4%
+            // the faster, and not on Q8, where it is 3% the slower.
             if (M <= 512) return run32<QUANT, 1, 1, EPI, 4, 4, true>(s, g);
-            return run32w<QUANT, 3, 1, EPI, 3, 4, true>(s, g);
+            const int64_t r96 = rounds(96, 128);
+            const int64_t c64 = std::max<int64_t>(65, 50 * rounds(64, 128)), c96 = std::max<int64_t>(80, 62 * r96),
+                          c128 = std::max<int64_t>(95, 84 * rounds(128, 128));
+            if (c64 < c96 && c64 < c128) return run32<QUANT, 2, 1, EPI, 4, 4, true>(s, g);
+            if (c128 <= c96) return run32w<QUANT, 4, 1, EPI, 3, 4, true>(s, g);
+            if (QUANT == Q8_DT || r96 <= 4) return run32<QUANT, 3, 1, EPI, 4, 4, true>(s, g);
+            if constexpr (QUANT != Q8_DT) return run32w<QUANT, 3, 1, EPI, 3, 4, true>(s, g);
         }
         if (M <= 512 && tiles(32, 128) <= 512) return run32<QUANT, 1, 1, EPI, 4, 4>(s, g);
         if ((g.ksplit > 1 || (QUANT == F16_DT && tiles(64, 128) > 256)) && tiles(96, 128) <= 256)
@@ -1487,8 +1502,13 @@ static void dispatch(hipStream_t s, const GemmArgs& g) {
         if (g.ksplit == 1 && tiles(64, 128) <= 256) return run32<QUANT, 2, 1, EPI, 4, 4>(s, g);
         if constexpr (QUANT == F16_DT) return run_lds<EPI, false>(s, g, 128);
         if constexpr (QUANT != F16_DT) {
-            // 128 x 256 (five units a round) against 96 x 128 (2.4)
-            if (50 * rounds(128, 256) > 24 * rounds(96, 128)) return run32w<QUANT, 3, 1, EPI, 3, 4>(s, g);
+            // A round of 64 x 128 of the short stages takes 37 units, of 96 x
+            // 128 48, of 128 x 256 100.  N 2,560, K 2,048, Q4 (96 x 128 ->
+            // this): 1,350 rows 27.1 -> 21.8 us, 1,600 28.3 -> 24.7, 2,663
+            // 39.6 -> 37.1, 16,320 183 -> 169.
+            const int64_t c64 = 37 * rounds(64, 128), c96 = 48 * rounds(96, 128), c256 = 100 * rounds(128, 256);
+            if (c64 < c96 && c64 < c256) return run32<QUANT, 2, 1, EPI, 4, 4>(s, g);
+            if (c96 < c256) return run32w<QUANT, 3, 1, EPI, 3, 4>(s, g);
             return run32w<QUANT, 4, 2, EPI, 3, 4>(s, g);
         }
     } else {

@@ -518,6 +518,27 @@ def test_refused_request_leaves_resident_prefix_intact():
     assert np.array_equal(first[0].rows[0], third[0].rows[0])
 
 
+@pytest.mark.parametrize("linear", ["Q4", "Q8", "F16"])
+def test_deep_k_pieces_of_every_tile(linear):
+    """A K 4,096 down projection in four pieces, 2,304 wide (18 column tiles),
+    in cold passes (profiled: one row range) whose rows pick 64, 96 and 128
+    rows per tile and, past four rounds, 96 rows of the wide kernel: the same
+    rows as the short warm pass, a workgroup per piece."""
+    cfg = gemma3_tiny(d=2304, ff=4096, layers=1, sliding=[True], window=40)
+    eng, _, _, _ = build(cfg, 23, getattr(g, linear), g.Q8, capacity=5632, oracle_models=False)
+    rng = np.random.default_rng(23)
+    eng.profile(True)
+    for rows in (541, 901, 1301, 1601, 5521):
+        prefix = rng.integers(0, 40, rows - 33).tolist()
+        branches = [BranchTokens(rng.integers(0, 40, 33).tolist(), [0, 5, 32])]
+        eng.evict_resident()
+        cold = eng.evaluate(prefix, branches, Want.HIDDEN)
+        warm = eng.evaluate(prefix, branches, Want.HIDDEN)
+        assert eng.prefix_source() == PrefixSource.RESIDENT
+        assert all(np.array_equal(a, b) for a, b in zip(cold[0].rows, warm[0].rows)), f"{rows} rows"
+    eng.profile(False)
+
+
 @pytest.mark.parametrize("heads,kv", [(4, 1), (8, 2), (2, 2)])
 def test_long_groups_bit_equal_to_separate_passes(heads, kv):
     """Groups long enough that their key ranges are cut into chunks (256
@@ -544,16 +565,17 @@ def test_long_groups_bit_equal_to_separate_passes(heads, kv):
 
 
 @pytest.mark.parametrize("rows,d,linear", [(1190, 800, "Q4"), (2390, 832, "Q8"), (2390, 800, "F16"), (2890, 832, "Q4"),
-                                           (2890, 800, "Q8")])
+                                           (2890, 800, "Q8"), (3230, 800, "Q4"), (1190, 832, "F16")])
 def test_wide_qkv_tiles_bit_equal_to_short_passes(rows, d, linear):
-    """The q/k/v product with K > 768 in passes of 64-, 96- and 128-row
-    wide tiles (20 head slots: 1,190, 2,390 and 2,890 rows; K 800 ends in
-    half a stage), behind a resident prefix of odd length, so that the tiles
-    start before the pass: every group's rows are bit-equal to its rows
-    alone, in passes of at most 512 rows on the eight-wave tile."""
+    """The q/k/v product with K > 768 in passes (profiled: one row range) of
+    64 rows of the short stages and 96-, 128- and 64-row wide tiles (20 head
+    slots: 1,190, 2,390, 2,890 and 3,230 rows; K 800 ends in half a stage),
+    behind a resident prefix of odd length, so that the tiles start before the
+    pass: every group's rows are bit-equal to its rows alone, in passes of at
+    most 512 rows on the eight-wave tile."""
     rng = np.random.default_rng(rows + d)
     cfg = gguf_tiny(16, 2, window=90, d=d)
-    eng, _, _, _ = build(cfg, 43, getattr(g, linear), g.Q8, capacity=3072, oracle_models=False)
+    eng, _, _, _ = build(cfg, 43, getattr(g, linear), g.Q8, capacity=3584, oracle_models=False)
     sizes = [500] * (rows // 500) + [rows % 500]
     groups = [Group([2, 5, 9], [BranchTokens([7, 8], [1])])]
     groups += [Group(rng.integers(0, 64, n - 31).tolist(), [BranchTokens(rng.integers(0, 64, 31).tolist(), [0, 30])])
@@ -564,7 +586,9 @@ def test_wide_qkv_tiles_bit_equal_to_short_passes(rows, d, linear):
         alone.append(eng.evaluate(gr.prefix, gr.branches, Want.HIDDEN))
     eng.evict_resident()
     eng.evaluate(groups[0].prefix, groups[0].branches, Want.HIDDEN)  # resident: base 3
+    eng.profile(True)
     together = eng.evaluate_groups(groups, Want.HIDDEN)
+    eng.profile(False)
     assert together[0].prefix_source == PrefixSource.RESIDENT
     for i, (a, t) in enumerate(zip(alone, together)):
         for x, y in zip(a, t.branches):

@@ -550,3 +550,29 @@ def test_every_tile_gives_the_same_rows(k, ldx, ldy, shift, dtype):
             z = a[:40]
             z = (gelu(z) if kind == "tanh" else 0.5 * z * (1.0 + np.vectorize(erf)(z / np.sqrt(2.0)))) * u
             assert np.max(np.abs(got[:40] - z) / np.maximum(np.abs(z), 1.0)) < 2e-3
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_every_f32_tile_of_a_narrow_product(dtype):
+    """2,560 columns, K 640: the rows where 64 x 128 of the short stages takes
+    over again past its first round, the 96- and 128-row tiles and, f16, 192
+    rows: the same bits as the longest launch's rows, and float64's within the
+    bound of f32 sums."""
+    rng = np.random.default_rng(50 + dtype)
+    n, k, rows = 2560, 640, 3700
+    t, wd = weight(rng, n, k, dtype)
+    w = g.DeviceWeight(t)
+    x = rng.uniform(-1, 1, (rows, k)).astype(np.float16)
+    xd = dev(x)
+
+    def run(m):
+        y = torch.zeros((m, n), dtype=torch.float32, device="cuda")
+        w.gemm(xd.data_ptr(), k, m, y.data_ptr(), n)
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    full = run(rows)
+    for m in (500, 513, 769, 1153, 1601, 2401, 3201, 3649):
+        assert np.array_equal(run(m), full[:m]), f"rows at M {m}"
+    xf = x.astype(np.float64)
+    assert (np.abs(full - xf @ wd.T) <= 2.0 ** -23 * k * (np.abs(xf) @ np.abs(wd).T)).all()
