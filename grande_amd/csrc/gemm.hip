@@ -1449,14 +1449,16 @@ static void dispatch(hipStream_t s, const GemmArgs& g) {
             return run_wide<QUANT, EPI>(s, g, 256);
         }
     } else if constexpr (EPI == EPI_RELU_F16) {
+        // 32 x 64 on two waves for the fewest rows (N 3,072, K 768, 32 x 128
+        // on four waves -> this: 12 rows f16 7.8 -> 6.0 us, Q4 7.0 -> 6.4, Q8
+        // 7.1 -> 6.6); f16 64 x 64 through LDS up to a round of those (150
+        // rows 9.3 -> 7.5, 300 11.2 -> 8.0).
         if constexpr (QUANT == F16_DT) {
-            // 64 x 64 up to a round of those (N 3,072, K 768, 32 x 128 with
-            // the weights in registers -> this: 150 rows 9.3 -> 7.5 us, 300
-            // 11.2 -> 8.0)
-            if (M <= 64) return run32<QUANT, 1, 1, EPI, 4, 4>(s, g);
+            if (M <= 64) return run32<QUANT, 1, 1, EPI, 4, 2>(s, g);
             if (tiles(64, 64) <= 256) return run32l<1, 1, EPI, 4>(s, g);
             return run_lds<EPI>(s, g, 128);
         } else {
+            if (tiles(32, 64) <= 256) return run32<QUANT, 1, 1, EPI, 4, 2>(s, g);
             if (tiles(32, 128) <= 256) return run32<QUANT, 1, 1, EPI, 4, 4>(s, g);
             return run_wide<QUANT, EPI>(s, g, 256);
         }
@@ -1526,6 +1528,11 @@ static void dispatch(hipStream_t s, const GemmArgs& g) {
         }
         if constexpr (QUANT == F16_DT) return run_lds<EPI>(s, g, 64);
         if constexpr (QUANT != F16_DT) {
+            // (the encoder's short gated product on two waves while those
+            // tiles make one round: N 1,152, K 768, 100 rows, Q4 9.2 -> 8.2
+            // us, Q8 9.8 -> 8.5)
+            if constexpr (EPI == EPI_GELU_ERF)
+                if (tiles(32, 64) <= 256) return run32<QUANT, 1, 2, EPI, 4, 2>(s, g);
             if (tiles(32, 128) <= 256) return run32<QUANT, 1, 2, EPI, 4, 4>(s, g);
             return run_wide<QUANT, EPI>(s, g, 128);
         }
