@@ -557,6 +557,7 @@ int64_t LayaEngine::pack(const LayaSeq* seqs, int64_t n) {
     d_first_ = reinterpret_cast<const int32_t*>(dv + o_first);
     t_ = at;
     nrows_ = nw;
+    nseqs_ = n;
     return total;
 }
 
@@ -674,6 +675,7 @@ void LayaEngine::set_full_last_layer(bool on) {
 void LayaEngine::launch_prepared() {
     if (t_ == 0) fail(E_INVALID, "nothing prepared");
     forward();
+    score();
 }
 
 void LayaEngine::hidden(const LayaSeq* seqs, int64_t n, float* out, int64_t out_floats) {
@@ -687,11 +689,11 @@ void LayaEngine::hidden(const LayaSeq* seqs, int64_t n, float* out, int64_t out_
     std::memcpy(out, h_out_, size_t(nrows_ * cfg_.d) * 4);
 }
 
-// The scorer on the read-out rows of the pass just queued: n sequences'
-// act probabilities after their nrows_ - n marker logits in scores_.
-void LayaEngine::score(int64_t n) {
+// The scorer on the read-out rows of the pass just queued: its sequences'
+// act probabilities after their nrows_ - nseqs_ marker logits in scores_.
+void LayaEngine::score() {
     const LayaConfig& c = cfg_;
-    const int64_t d = c.d, nm = nrows_ - n;
+    const int64_t d = c.d, n = nseqs_, nm = nrows_ - n;
     const Scorer& S = scorer_;
     if (nm > 0) {
         step("score_norm", [&] {
@@ -729,7 +731,7 @@ void LayaEngine::evaluate(const LayaSeq* seqs, int64_t n, float* logits, int64_t
     if (nlogits < want || nact < n) fail(E_INVALID, "output buffer too small");
     pack(seqs, n);
     forward();
-    score(n);
+    score();
     const int64_t got = want + (cfg_.act_out > 0 ? n : 0);
     OMG_HIP(hipMemcpyAsync(h_out_, scores_.p, size_t(got) * 4, hipMemcpyDeviceToHost, stream_));
     sync();

@@ -128,13 +128,13 @@ class LayaEngine {
     LayaEngine() = default;
     int64_t pack(const LayaSeq* seqs, int64_t n);  // returns the token count; fills wanted
     void forward();
-    void score(int64_t n);
+    void score();
     template <class F>
     void step(const char* name, F&& f);
 
     LayaConfig cfg_;
     int64_t capacity_ = 0, max_rows_ = 0, rows_cap_ = 0, tpad_ = 0;
-    int64_t t_ = 0, nrows_ = 0;
+    int64_t t_ = 0, nrows_ = 0, nseqs_ = 0;
     hipStream_t stream_ = nullptr;
     DevTensor embed_;
     DevBuf embed_norm_, final_norm_, type_emb_;

@@ -315,8 +315,8 @@ int omg_dev_attention_bi(const void *q16, const void *k16, const void *vt, const
 /* ---- the bidirectional encoder path (crates/omg-wgpu/src/laya.rs) ----
  * An mmBERT / ModernBERT encoder with Laya's decision head: every question
  * is one sequence; a request's sequences run as one packed pass isolated by
- * the attention mask; the scorer reads the [CLS] and [MASK] rows on the
- * host. */
+ * the attention mask; the scorer and the act head read the [CLS] and [MASK]
+ * rows on the device. */
 typedef struct omg_laya omg_laya;
 typedef struct omg_laya_builder omg_laya_builder;
 
@@ -380,7 +380,9 @@ int omg_laya_evaluate(omg_laya *e, const omg_laya_seq *seqs, size_t n, float *lo
                       size_t nact);
 /* LayaConfig::temperature_for (laya.rs:234-248). */
 int omg_laya_temperature(const omg_laya *e, int qtype, size_t k, float *out);
-/* Measurement, as omg_pass_prepare / omg_pass_launch / omg_sync / omg_profile. */
+/* Measurement, as omg_pass_prepare / omg_pass_launch / omg_sync / omg_profile:
+ * a launch is the device work of one omg_laya_evaluate, the forward pass, the
+ * scorer and the act head. */
 int omg_laya_prepare(omg_laya *e, const omg_laya_seq *seqs, size_t n);
 int omg_laya_launch(omg_laya *e);
 int omg_laya_sync(omg_laya *e);

@@ -463,3 +463,19 @@ def test_scorer_on_device_matches_float64(counts, act, dtype):
         a = T["act.l2"] @ a + T["act.l2_b"]
         a = np.exp(a - a.max())
         assert abs(o.act_probability - a[0] / a.sum()) < 1e-5
+
+
+@pytest.mark.parametrize("act", [{"ask": 1.0}, None])
+def test_a_prepared_launch_runs_the_scorer(act):
+    """A prepared launch is an evaluate's device work: the same kernels, as
+    often, the scorer's and the act head's among them."""
+    cfg = tiny(act_costs=act)
+    eng = ly.LayaEngine.new(ly.synth_weights(cfg, 8, g.Q8, g.Q8), 400, 40)
+    seqs = random_seqs(np.random.default_rng(8), 300, 3, 20, 60)
+    counts = []
+    for run in (lambda: eng.evaluate(seqs), lambda: (eng.prepare(seqs), eng.launch(), eng.sync())):
+        eng.profile(True)
+        run()
+        counts.append({name: n for name, (n, _) in eng.profile_report().items()})
+        eng.profile(False)
+    assert counts[0] == counts[1] and {"score_norm", "score_l1", "score"} <= set(counts[1])
