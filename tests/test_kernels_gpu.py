@@ -576,3 +576,32 @@ def test_every_f32_tile_of_a_narrow_product(dtype):
         assert np.array_equal(run(m), full[:m]), f"rows at M {m}"
     xf = x.astype(np.float64)
     assert (np.abs(full - xf @ wd.T) <= 2.0 ** -23 * k * (np.abs(xf) @ np.abs(wd).T)).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("vocab,d,nrows,nlabels", [(200, 4096, 800, 5), (1000, 64, 40, 600), (900, 192, 33, 513)])
+def test_readout_split_in_the_workgroups(vocab, d, nrows, nlabels, dtype):
+    """Without scratch for the split rows (they do not fit the fixed array, or
+    the full rows take it) the workgroups split the rows themselves, also with
+    fewer K stages than they convert at once: the same bits as with scratch,
+    and the logits the float64 ones within 2^-24 (2 + d / 8) of sum |x||w|."""
+    rng = np.random.default_rng(vocab + d + nrows + dtype)
+    t, _ = weight(rng, vocab, d, dtype, "embed")
+    e = t.to_f32().astype(np.float64)
+    rows = rng.standard_normal((nrows, d)).astype(np.float32)
+    rows[nrows // 3, d // 2] = 2.0 ** 60  # a row of the f32 product
+    labels = rng.choice(vocab, nlabels, replace=False).astype(np.uint32)
+    w = g.DeviceWeight(t)
+    rd, lab = dev(rows), dev(labels.view(np.int32))
+    outs = []
+    for f in (w.label_readout, w.label_readout_noalloc):
+        out = torch.full((nrows, nlabels + 1), float("nan"), dtype=torch.float32, device="cuda")
+        f(rd.data_ptr(), nrows, lab.data_ptr(), nlabels, 0.0, out.data_ptr())
+        torch.cuda.synchronize()
+        outs.append(out.cpu().numpy())
+    assert np.array_equal(outs[0], outs[1])
+    rows64 = rows.astype(np.float64)
+    z = rows64 @ e.T
+    bound = 2.0 ** -24 * (2 + d / 8) * (np.abs(rows64) @ np.abs(e).T)
+    bound[nrows // 3] *= 8  # (its sums round once per product)
+    assert (np.abs(outs[0][:, :-1] - z[:, labels]) <= bound[:, labels]).all()
