@@ -406,7 +406,10 @@ __device__ inline void finish32(const GemmArgs& g, const floatx16 (&acc)[MI][NJ]
                 for (int e = 0; e < 16; ++e) v[j][e] = acc[i][j][e] + bias[j][e];
             if (sec < 2) {
                 if (o.rope) {
-                    // rope_bi.wgsl:30-49: a' = a cos - b sin, b' = b cos + a sin.
+                    // rope_bi.wgsl:30-49: a' = a cos - b sin, b' = b cos + a sin,
+                    // each with a's product inside the fmaf (the other order
+                    // moves one q or k in 20,000 by an f16 ulp, which the
+                    // encoder's 22 layers turn into 1e-3 of its logits).
                     const float2* rp = o.rope + int64_t(live ? o.meta[4 * m] : 0) * 32 + 4 * lh;
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
@@ -417,7 +420,7 @@ __device__ inline void finish32(const GemmArgs& g, const floatx16 (&acc)[MI][NJ]
                         for (int r = 0; r < 4; ++r) {
                             const float a = v[0][4 * q + r], b = v[1][4 * q + r];
                             v[0][4 * q + r] = fmaf(a, cs[r], -(b * sn[r]));
-                            v[1][4 * q + r] = fmaf(b, cs[r], a * sn[r]);
+                            v[1][4 * q + r] = fmaf(a, sn[r], b * cs[r]);
                         }
                     }
                 }

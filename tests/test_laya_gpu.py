@@ -157,6 +157,47 @@ def test_qkv_heads_of_every_tile(dtype):
         assert rel_diff(full[s][:, tail].astype(np.float32), y[:, s].transpose(1, 0, 2)) < 2e-3, f"section {s}"
 
 
+@pytest.mark.parametrize("dtype", [g.F16, g.Q8, g.Q4])
+@pytest.mark.parametrize("t", [100, 3000])
+def test_qkv_heads_rounding(t, dtype):
+    """q and k are the f32 product's sums (the plain product's bits) plus the
+    bias, rotated in f32 as fma(a, cos, -(b sin)) and fma(a, sin, b cos) (one
+    rounding of the second product, one of the sum) and scaled, each rounded
+    to f16 from f32: bit for bit.  A float64 sum of the exact first product
+    and the rounded second one, rounded to f32, is that fma but for ties of
+    its 53 bits, which the values here do not make."""
+    rng = np.random.default_rng(t + dtype)
+    heads, d = 3, 192
+    x = rng.standard_normal((t, d)).astype(np.float16)
+    wt, _ = qweight(rng, 3 * d, d, dtype, 0.1)
+    bias = rng.standard_normal(3 * d).astype(np.float16)
+    meta = pack_meta([181] * (t // 181) + [t % 181])
+    table = rope_table(10000.0, 256)
+    w = g.DeviceWeight(wt)
+    xd, bd, md, rd = dev(x), dev(bias), dev(meta), dev(table)
+    tpad = (t + 63) // 64 * 64
+    out = [torch.zeros(heads * tpad * 64, dtype=torch.float16, device="cuda") for _ in range(3)]
+    y = torch.zeros((t, 3 * d), dtype=torch.float32, device="cuda")
+    scale = np.float32(0.3)
+    w.gemm(xd.data_ptr(), d, t, y.data_ptr(), 3 * d)
+    w.qkv_heads(xd.data_ptr(), d, t, bd.data_ptr(), rd.data_ptr(), md.data_ptr(), float(scale), tpad,
+                *(o.data_ptr() for o in out))
+    torch.cuda.synchronize()
+    y = (y.cpu().numpy() + bias.astype(np.float32)).reshape(t, 3, heads, 64)
+    cs = np.asarray(table, np.float32)[meta[:, 0]]
+    c, s = cs[:, None, :, 0], cs[:, None, :, 1]
+
+    def fma(p, q, r):
+        return (p.astype(np.float64) * q.astype(np.float64) + r.astype(np.float64)).astype(np.float32)
+
+    for sec in range(3):
+        a, b = y[:, sec, :, :32], y[:, sec, :, 32:]
+        want = y[:, 2] if sec == 2 else np.concatenate([fma(a, c, -(b * s)), fma(a, s, b * c)], -1)
+        want = (want * scale if sec == 0 else want).astype(np.float16)
+        got = unpack_vt(out[2].cpu().numpy(), heads, tpad) if sec == 2 else out[sec].cpu().numpy().reshape(heads, tpad, 64)
+        assert np.array_equal(got[:, :t].transpose(1, 0, 2), want), f"section {sec}"
+
+
 def attention_ref(q, k, v, meta, window):
     """float64 softmax(q . k) v over the visible keys of each row."""
     heads, t = q.shape[0], meta.shape[0]
