@@ -1,6 +1,6 @@
 """Benchmark of the decision-path pass on one MI355X.
 
-Workload (the metric's configuration): a
+Workload (the headline metric's configuration, c2): a
 Gemma-3-270M-shaped decoder with seeded Q4_0 weights and a 25,000-row
 vocabulary, one 2,000-token state plus 12 question branches of 32 tokens
 in one block-causal pass, label readout at each branch's last position:
@@ -16,13 +16,13 @@ readback included: `api_ms` cold / warm are medians of the C ABI call on
 arguments marshalled once, `python_*` one call through the Python
 wrapper) are reported beside it.
 
-`--config c4` measures BASELINE.json configs[3] instead: the Laya encoder
-path over 192 sequences of 256 tokens (see bench_encoder).  `--config e2b`
+`--config c4` measures the Laya encoder
+path instead, over 192 sequences of 256 tokens (see bench_encoder).  `--config e2b`
 measures the reference's published Gemma 4 workload (E2B-shaped Q4_0, 12
 questions over a 2,000-token state; see bench_gemma4) as cold and warm
 latency against the published figures.
 
-Prints one JSON line (see the repository's driver contract).
+Prints one JSON line.
 """
 from __future__ import annotations
 
@@ -540,7 +540,7 @@ def main() -> int:
 
 
 def encoder_seqs(spec, rng):
-    """configs[3]'s requests: per question a 256-token sequence ([CLS] ...
+    """The encoder workload's requests: per question a 256-token sequence ([CLS] ...
     [SEP]) with one [MASK]; question types cycle choice / score / noul."""
     from grande_amd import laya as ly
 
@@ -704,7 +704,7 @@ def bench_gemma4(args) -> int:
 
 
 def bench_encoder(args) -> int:
-    """the Laya path (mmBERT-base-shaped encoder +
+    """The Laya path (mmBERT-base-shaped encoder +
     two decision-head layers, Q8_0) over 64 requests x 3 questions of 256
     tokens in one packed pass; a step is that pass with ids and metadata
     already in HBM."""

@@ -26,7 +26,7 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result", f"-I{INCL
 DEVICE = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 SOURCES = ["gemm.hip", "attention.hip", "norm.hip", "laya.hip", "model.cpp", "gguf.cpp", "state.cpp", "engine.cpp", "laya.cpp", "capi.cpp"]
-# Per-file device flags.  The GEMM and attention kernels keep their MFMA
+# Per-file device flags.  The kernels with MFMA products keep their
 # accumulators in ordinary VGPRs: with the AGPR form the register allocator
 # shuffles them between loop iterations (v_accvgpr moves in the main loop).
 EXTRA = {name: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for name in ("gemm.hip", "attention.hip", "norm.hip", "laya.hip")}

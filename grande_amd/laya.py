@@ -62,7 +62,7 @@ def laya_config_json(*, vocab: int, d: int, layers: int, heads: int, ff: int, lo
     return json.dumps(cfg)
 
 
-# mmBERT-base-shaped encoder, Q8_0, 56,000-token
+# The encoder benchmark: mmBERT-base-shaped encoder, Q8_0, 56,000-token
 # vocabulary; 64 requests x 3 questions of 256 tokens, one [MASK] each.
 MMBERT_BASE = dict(vocab=56_000, d=768, layers=22, heads=12, ff=1152, local_attention=128, global_every=3)
 C4 = dict(model=MMBERT_BASE, dtype=Q8, requests=64, questions=3, seq_len=256)

@@ -90,7 +90,7 @@ def gemma4_config_json(*, vocab: int, d: int, layers: int, heads: int, kv_heads:
     return json.dumps(cfg)
 
 
-# Gemma-3-shaped decoders with the vocabulary pruned
+# Benchmark configurations: Gemma-3-shaped decoders with the vocabulary pruned
 # to 25,000 rows.
 GEMMA3_270M = dict(vocab=25_000, d=640, layers=18, heads=4, kv_heads=1, head_dim=256, ff=2048, window=512)
 GEMMA3_1B = dict(vocab=25_000, d=1152, layers=26, heads=4, kv_heads=1, head_dim=256, ff=6912, window=512)

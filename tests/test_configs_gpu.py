@@ -1,4 +1,4 @@
-"""The BASELINE.json configurations on the GPU against the CPU oracle
+"""The benchmark configurations (c1 to c5) on the GPU against the CPU oracle
 (crates/omg-wgpu/tests/reference.rs restated), at their real shapes.
 
 C1 and C2 run the whole configuration through the oracle; C3 (1B) runs the
@@ -6,7 +6,7 @@ C1 and C2 run the whole configuration through the oracle; C3 (1B) runs the
 2,000-token state by the properties a pass must have (resident and restored
 states bit-equal to the full pass); C5 (4B) checks the full 8,000 + 208 x 40
 pass by those properties and isolation, and the oracle on the same shapes
-with two layers.  The readout bar is BASELINE.json's: after softmax within
+with two layers.  The readout bar: after softmax within
 2e-2 of the oracle, identical argmax per question."""
 from __future__ import annotations
 
@@ -46,7 +46,7 @@ def oracle_wanted_rows(model, prefix, branches):
 
 
 def assert_readout(got_logits, exp_logits, what):
-    """within 2e-2 after softmax, identical argmax."""
+    """Within 2e-2 after softmax, identical argmax."""
     worst = 0.0
     for i, (a, b) in enumerate(zip(got_logits, exp_logits)):
         pa, pb = oracle.softmax(a), oracle.softmax(b)
@@ -122,7 +122,7 @@ def test_c2_270m_q4_label_lse_route():
 
 
 def pointer_head(d: int, options: int = 52) -> np.ndarray:
-    """The seeded [d x 52] f32 pointer head of BASELINE.json configs[2]."""
+    """The seeded [d x 52] f32 pointer head of c3."""
     return (np.random.default_rng(52).standard_normal((d, options)) / np.sqrt(d)).astype(np.float32)
 
 

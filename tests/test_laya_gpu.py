@@ -9,8 +9,8 @@ layouts; the erf-GELU gated GEMM and the bias + ReLU GEMM.
 
 Engine level: hidden rows (rel 1e-2; the reference's own forward test
 allows 2e-2, crates/omg-wgpu/tests/reference.rs:380-431) and scorer
-outputs against the CPU oracle (oracle/laya.c) on tiny configs and on the mmBERT-base shapes of
-BASELINE.json configs[3] with two layers; the full configs[3] pass (64
+outputs against the CPU oracle (oracle/laya.c) on tiny configs and on the
+mmBERT-base shapes with two layers; the full encoder pass (64
 requests x 3 questions of 256 tokens) by the properties the pass must have:
 a sequence's rows do not depend on the other sequences of the batch
 (bit-equal), finite outputs, and the oracle on a sample of its sequences
@@ -415,7 +415,7 @@ def c4_config(**over) -> str:
 
 
 def test_c4_shapes_two_layers_match_oracle():
-    """configs[3]'s shapes (d 768, 12 heads of 64, ff 1152, window 64,
+    """The benchmark's encoder shapes (d 768, 12 heads of 64, ff 1152, window 64,
     56,000-token vocabulary, Q8) with two encoder layers (global, local)."""
     cfg = c4_config(layers=2)
     eng, orc = engine_and_oracle(cfg, 0x5EED, g.Q8, 4 * 256, 8)
@@ -429,7 +429,7 @@ def test_c4_shapes_two_layers_match_oracle():
 
 
 def test_c4_full_pass_properties():
-    """configs[3]: 64 requests x 3 questions of 256 tokens (49,152 tokens)
+    """64 requests x 3 questions of 256 tokens (49,152 tokens)
     through all 22 layers; a sample of sequences checked by the oracle and
     by isolation."""
     spec = ly.C4
